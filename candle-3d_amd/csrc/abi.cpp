@@ -1342,6 +1342,81 @@ int lux3d_sparse_conv3d_rulebook(const lux3d_tensor_t *x, const lux3d_tensor_t *
                     fn);
 }
 
+namespace {
+// table [passes, N, 27 / passes + 1] int32, passes 3 or 9; the passes or -1
+int order_table(const lux3d_tensor_t *table, int64_t n, const char *fn) {
+  const int64_t s = table->shape[0];
+  if ((s != 3 && s != 9) || table->shape[1] != n || table->shape[2] != 27 / s + 1) {
+    fail(LUX3D_ERR_SHAPE, "%s: table must be [3, %lld, 10] or [9, %lld, 4]", fn, (long long)n, (long long)n);
+    return -1;
+  }
+  return (int)s;
+}
+}  // namespace
+
+int lux3d_sparse_order(const lux3d_tensor_t *nbr, const lux3d_tensor_t *table, const lux3d_tensor_t *workspace,
+                       lux3d_stream_t stream) {
+  const char *fn = "lux3d_sparse_order";
+  int r;
+  if ((r = contiguous_of(nbr, fn, "nbr", LUX3D_I32, 2)) || (r = contiguous_of(table, fn, "table", LUX3D_I32, 3)) ||
+      (r = contiguous_of(workspace, fn, "workspace", LUX3D_I32, -1)))
+    return r;
+  const int64_t n = nbr->shape[0];
+  if (nbr->shape[1] != 27) return fail(LUX3D_ERR_SHAPE, "%s: nbr must be [N, 27]", fn);
+  const int passes = order_table(table, n, fn);
+  if (passes < 0) return LUX3D_ERR_SHAPE;
+  if (numel(workspace) < kOrderWs)
+    return fail(LUX3D_ERR_SHAPE, "%s: workspace must hold %lld int32", fn, (long long)kOrderWs);
+  if (n > INT32_MAX / 27) return fail(LUX3D_ERR_SHAPE, "%s: too many voxels", fn);
+  return hip_status(launch_sparse_order(static_cast<const int32_t *>(nbr->data), n, passes,
+                                        static_cast<int32_t *>(table->data), static_cast<int32_t *>(workspace->data),
+                                        stream_of(stream)),
+                    fn);
+}
+
+int lux3d_sparse_conv3d_ordered(const lux3d_tensor_t *x, const lux3d_tensor_t *table, const lux3d_tensor_t *weight,
+                                const lux3d_tensor_t *planes, const lux3d_tensor_t *bias, const lux3d_tensor_t *out,
+                                lux3d_stream_t stream) {
+  const char *fn = "lux3d_sparse_conv3d_ordered";
+  int r;
+  if ((r = contiguous_of(x, fn, "x", LUX3D_F32, 2)) || (r = contiguous_of(table, fn, "table", LUX3D_I32, 3)) ||
+      (r = contiguous_of(weight, fn, "weight", LUX3D_F32, 3)) ||
+      (r = contiguous_of(planes, fn, "planes", LUX3D_BF16, -1)) || (r = contiguous_of(out, fn, "out", LUX3D_F32, 2)))
+    return r;
+  const int64_t n = x->shape[0], cin = x->shape[1], cout = weight->shape[1];
+  const int passes = order_table(table, n, fn);
+  if (passes < 0) return LUX3D_ERR_SHAPE;
+  if (weight->shape[0] != 27 || weight->shape[2] != cin)
+    return fail(LUX3D_ERR_SHAPE, "SparseConv3d expects [N, %lld] with weight [27, Cout, %lld]", (long long)cin,
+                (long long)weight->shape[2]);
+  if (out->shape[0] != n || out->shape[1] != cout) return fail(LUX3D_ERR_SHAPE, "%s: out must be [%lld, %lld]", fn,
+                                                                (long long)n, (long long)cout);
+  if (cin % 16 || cin == 0)
+    return fail(LUX3D_ERR_SHAPE, "%s: Cin must be a positive multiple of 16 (use lux3d_sparse_conv3d)", fn);
+  if (cout > 0 && !sparse_ordered_fits(n, cin, cout))
+    return fail(LUX3D_ERR_SHAPE, "%s: x and the weight planes must stay below 2^31 bytes (use lux3d_sparse_conv3d)", fn);
+  if (numel(planes) * 2 < sparse_weight_planes_bytes(cin, cout))
+    return fail(LUX3D_ERR_SHAPE, "%s: planes must hold 27 x ceil(Cout / 32) x 32 x Cin x 3 bf16", fn);
+  if (!aligned16(x->data) || !aligned16(weight->data) || !aligned16(planes->data))
+    return fail(LUX3D_ERR_LAYOUT, "%s: x, weight and planes must be 16-byte aligned", fn);
+  const float *bp = nullptr;
+  if (bias) {
+    if ((r = contiguous_of(bias, fn, "bias", LUX3D_F32, -1))) return r;
+    if (numel(bias) != cout) return fail(LUX3D_ERR_SHAPE, "%s: bias must have %lld elements", fn, (long long)cout);
+    bp = static_cast<const float *>(bias->data);
+  }
+  SparseConvParams p;
+  p.x = static_cast<const float *>(x->data);
+  p.w = static_cast<const float *>(weight->data);
+  p.bias = bp;
+  p.out = static_cast<float *>(out->data);
+  p.n = n; p.cin = cin; p.cout = cout;
+  p.mfma = true;
+  return hip_status(launch_sparse_conv_ordered(p, static_cast<const int32_t *>(table->data), passes, planes->data,
+                                               stream_of(stream)),
+                    fn);
+}
+
 int lux3d_index_select_rows(const lux3d_tensor_t *src, const lux3d_tensor_t *ids, const lux3d_tensor_t *out,
                             const lux3d_tensor_t *bad_ids, lux3d_stream_t stream) {
   const char *fn = "lux3d_index_select_rows";

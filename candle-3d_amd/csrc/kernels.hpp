@@ -206,6 +206,16 @@ hipError_t launch_sparse_conv(const SparseConvParams &p, hipStream_t s);
 hipError_t launch_sparse_rulebook(const int32_t *nbr, int64_t n, int32_t *pairs, int32_t *counts, hipStream_t s);
 hipError_t launch_sparse_conv_rulebook(const SparseConvParams &p, const int32_t *pairs, const int32_t *counts,
                                        hipStream_t s);
+// Ordered path: table [passes, n, 27 / passes + 1] (passes 3 or 9), each pass's
+// rows (row id, neighbours of its taps) sorted by their mask of present taps
+// (ws: kOrderWs int32); then the conv, with the weights' bf16 terms in
+// `planes` (sparse_weight_planes_bytes).
+constexpr int64_t kOrderWs = 3 << 9;
+hipError_t launch_sparse_order(const int32_t *nbr, int64_t n, int passes, int32_t *table, int32_t *ws, hipStream_t s);
+inline int64_t sparse_weight_planes_bytes(int64_t cin, int64_t cout) { return 27 * ((cout + 31) / 32 * 32) * cin * 6; }
+bool sparse_ordered_fits(int64_t n, int64_t cin, int64_t cout);
+hipError_t launch_sparse_conv_ordered(const SparseConvParams &p, const int32_t *table, int passes, void *planes,
+                                      hipStream_t s);
 // out[m] = src[ids[m]] for m < rows (and m < *count when count is given);
 // rows of row_bytes bytes; ids out of range give zero rows.
 hipError_t launch_gather_rows(const void *src, int64_t nsrc, const void *ids, bool ids64, int64_t rows,

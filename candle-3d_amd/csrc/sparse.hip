@@ -26,6 +26,7 @@
 // the reference order (parent order, ascending subidx), and a row gather
 // copies the child features. The child count is written to device memory.
 #include <mutex>
+#include <type_traits>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -528,6 +529,421 @@ __global__ __launch_bounds__(256) void sparse_tap_x3_kernel(SparseConvParams p, 
   tap_epilogue<BM, BN, TM, TN>(p.out, Cout, n0, wm, wn, lane, dst, acc);
 }
 
+// ---- ordered path: rows grouped by the taps they use ---------------------------
+//
+// The 27 taps are handled in passes of T consecutive taps (T = 9 or 3). For
+// each pass the rows are sorted by their T-bit mask of present neighbours
+// (most taps first), so a tile of BM consecutive rows of the order shares one
+// mask or a few: the tile computes the taps of the union of its rows' masks
+// only, keeps its sums in registers over those taps and touches each output
+// row once per pass. Against one pass per tap that is 27 / T instead of 27
+// read-modify-write sweeps over the output, and against output-stationary
+// tiles in row order, whose union holds nearly every tap, 1.0-1.2 instead of
+// 1.3-4 times the products that exist (24k-150k voxel shells; T = 9).
+//
+// table [27 / T, n, T + 1]: per pass the rows in that order, each with its row
+// id and its T neighbour rows (-1: missing), from three launches: a histogram
+// of the masks, their starts (most taps first, then by value), and the
+// scatter. A workgroup reserves each mask's slots with one atomic, so the rows
+// of one mask are in no fixed order; no result depends on it, as a row's sums
+// do not depend on the other rows of its tile.
+
+// mask of taps s * T .. s * T + T - 1 of LDS row r of the neighbour table
+template <int T> __device__ __forceinline__ uint32_t tap_mask_of(const int32_t *r, int s, int64_t n) {
+  uint32_t m = 0;
+#pragma unroll
+  for (int k = 0; k < T; ++k) {
+    const int32_t v = r[s * T + k];
+    m |= (uint32_t)(v >= 0 && v < n) << k;
+  }
+  return m;
+}
+
+__global__ __launch_bounds__(256) void order_clear_kernel(int32_t *hist, int count) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < count) hist[i] = 0;
+}
+
+// SCATTER false: hist[s][mask] += rows of the workgroup; true: hist holds each
+// mask's next free slot, and the workgroup's rows are written to the table.
+template <int T, bool SCATTER>
+__global__ __launch_bounds__(256) void order_rows_kernel(const int32_t *nbr, int64_t n, int32_t *hist,
+                                                         int32_t *table) {
+  constexpr int S = 27 / T, NB = S << T;
+  __shared__ int32_t rows[256 * 27];
+  __shared__ int32_t cnt[NB];
+  const int t = threadIdx.x;
+  const int64_t i0 = (int64_t)blockIdx.x * 256, i = i0 + t;
+  const int64_t nrow = n - i0 < 256 ? n - i0 : 256;
+  for (int e = t; e < NB; e += 256) cnt[e] = 0;
+  for (int e = t; e < nrow * 27; e += 256) rows[e] = nbr[i0 * 27 + e];
+  __syncthreads();
+  int32_t bin[S], rank[S];
+  if (i < n) {
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      bin[s] = (s << T) + (int32_t)tap_mask_of<T>(rows + t * 27, s, n);
+      rank[s] = atomicAdd(&cnt[bin[s]], 1);
+    }
+  }
+  __syncthreads();
+  for (int e = t; e < NB; e += 256) {
+    const int32_t c = cnt[e];
+    if (c) cnt[e] = atomicAdd(&hist[e], c);
+  }
+  if constexpr (SCATTER) {
+    __syncthreads();
+    if (i < n) {
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        int32_t *dst = table + (s * n + cnt[bin[s]] + rank[s]) * (T + 1);
+        dst[0] = (int32_t)i;
+#pragma unroll
+        for (int k = 0; k < T; ++k) {
+          const int32_t v = rows[t * 27 + s * T + k];
+          dst[1 + k] = v >= 0 && v < n ? v : -1;
+        }
+      }
+    }
+  }
+}
+
+// The 2^T masks, most taps first, then by value.
+template <int T> struct MaskRanks {
+  uint16_t at[1 << T];
+  constexpr MaskRanks() : at() {
+    int k = 0;
+    for (int pc = T; pc >= 0; --pc)
+      for (int m = 0; m < (1 << T); ++m) {
+        int c = 0;
+        for (int v = m; v; v >>= 1) c += v & 1;
+        if (c == pc) at[k++] = (uint16_t)m;
+      }
+  }
+};
+__constant__ constexpr MaskRanks<9> kRanks9{};
+__constant__ constexpr MaskRanks<3> kRanks3{};
+
+// hist[s][mask] -> the first slot of the mask's rows. One workgroup per pass.
+template <int T> __global__ __launch_bounds__(512) void order_starts_kernel(int32_t *hist) {
+  constexpr int NB = 1 << T;
+  __shared__ int32_t wsum[8];
+  int32_t *hs = hist + (int64_t)blockIdx.x * NB;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int m = T == 9 ? kRanks9.at[t] : kRanks3.at[t < NB ? t : 0];
+  const int32_t c = t < NB ? hs[m] : 0;
+  int32_t incl = c;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int32_t v = __shfl_up(incl, d, 64);
+    if (lane >= d) incl += v;
+  }
+  if (lane == 63) wsum[wave] = incl;
+  __syncthreads();
+  int32_t base = 0;
+  for (int w = 0; w < wave; ++w) base += wsum[w];
+  if (t < NB) hs[m] = base + incl - c;
+}
+
+// W [27, Cout, Cin] f32 -> its exact three bf16 terms as 1 KB blocks
+// [27][ceil(Cout / 32)][Cin / 16][3]: 32 output channels x 16 input channels
+// of one term, lane l of a wavefront's fragment (channel l % 32, inputs 8 (l /
+// 32) .. + 7) at l * 16 bytes, so that the convolution copies blocks to LDS
+// as they are and reads fragments without bank conflicts. Channels past Cout
+// are zero. Done once per call (C 1024: 113 MB read, 170 MB written, about 60
+// us of 5 ms) instead of once per row tile.
+__global__ __launch_bounds__(256) void split_weights_kernel(const float *w, int64_t cin, int64_t cout, int64_t ncb,
+                                                            int64_t blocks, uint4 *planes) {
+  const int64_t g = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);  // one wavefront per 32 x 16 block
+  if (g >= blocks) return;
+  const int lane = threadIdx.x & 63;
+  const int64_t nk = cin / 16, k16 = g % nk, cb = g / nk % ncb, tap = g / nk / ncb;
+  const int64_t o = cb * 32 + (lane & 31);
+  float v[8] = {};
+  if (o < cout) Chunk<F32>::load<false>(w + (tap * cout + o) * cin + k16 * 16 + 8 * (lane >> 5), v);
+  uint32_t t1[4], t2[4], t3[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const Split3 r = split3_bf16(v[2 * e], v[2 * e + 1]);
+    t1[e] = r.t1;
+    t2[e] = r.t2;
+    t3[e] = r.t3;
+  }
+  uint4 *dst = planes + g * 3 * 64 + lane;
+  dst[0] = make_uint4(t1[0], t1[1], t1[2], t1[3]);
+  dst[64] = make_uint4(t2[0], t2[1], t2[2], t2[3]);
+  dst[128] = make_uint4(t3[0], t3[1], t3[2], t3[3]);
+}
+
+// One pass: out[row, :] = (first ? 0 : out[row, :]) + sum over the pass's taps k
+// of row of x[neighbour k, :] W_k^T (+ bias in the last pass), f32 on the bf16 matrix cores (six
+// bf16 MFMAs per product step, the terms and their order as in
+// sparse_tap_x3_kernel). Each tap is summed on its own from zero and then
+// added, as the per-tap path does: the matrix cores' running sums lose
+// accuracy with their length (24k voxels, C 1024, 20 taps: relative error
+// 1.6e-6 in one chain over all taps). A row without the tap adds nothing,
+// whatever the weights hold.
+//
+// BM x BN tile, four wavefronts as WM x WN, each TM x TN MFMA tiles of 32 x
+// 32. A 16-deep step of the pipeline is a stage of an LDS ring filled by
+// direct global -> LDS loads only: the f32 rows of x (64 bytes each, 16-byte
+// chunk c of row r in slot c ^ ((r >> 2) & 3); a missing row's offset lies
+// past the descriptor and reads as zeros) and the weight blocks as they are.
+// The three terms of x are formed in registers when its fragments are read
+// (WN wavefronts repeat them), so no pass over LDS and no second barrier are
+// needed: the ring's one barrier per step orders everything. Two workgroups
+// per CU (LDS and registers) overlap one's split with the other's MFMAs.
+template <int WM, int WN, int TM, int TN, int NS, int T>
+__global__ __launch_bounds__(64 * WM * WN, 2) void sparse_ordered_x3_kernel(SparseConvParams p, const int32_t *table,
+                                                                   const char *planes, int64_t planes_bytes, int tap0,
+                                                                   bool first, bool last, int tiles_n) {
+  typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+  constexpr int NW = WM * WN, NT = 64 * NW, BM = WM * TM * 32, BN = WN * TN * 32;
+  constexpr int ASEG = BM / 16, BSEG = BN / 32 * 3;           // 1 KB segments per stage
+  constexpr int AW = ASEG / NW, BW = (BSEG + NW - 1) / NW;    // per wavefront (spare ones repeat the last segment)
+  static_assert(ASEG % NW == 0, "whole x segments per wavefront");
+  constexpr int STAGE = (ASEG + BSEG) * 1024, OPS = AW + BW;
+  __shared__ __align__(16) char ring[NS * STAGE];
+  __shared__ int32_t nb[BM * T];
+  __shared__ int32_t rowid[BM];
+  __shared__ __align__(16) uint32_t rmask[BM];
+  __shared__ uint32_t wmask[NW];
+
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int wm = wave / WN, wn = wave % WN, l32 = lane & 31, hh = lane >> 5;
+  const int64_t n = p.n, Cin = p.cin, Cout = p.cout;
+  // workgroup i runs on XCD i % 8: the column tiles of a row tile follow each
+  // other on one XCD and share its L2 copy of the gathered rows
+  const int idx = (int)blockIdx.x / 8;
+  const int64_t m0 = ((int64_t)(idx / tiles_n) * 8 + blockIdx.x % 8) * BM, n0 = (int64_t)(idx % tiles_n) * BN;
+  if (m0 >= n) return;  // uniform: the grid covers whole groups of 8 row tiles
+
+  for (int e = t; e < BM * (T + 1); e += NT) {
+    const int r = e / (T + 1), k = e % (T + 1);
+    const int32_t v = m0 + r < n ? table[(m0 + r) * (T + 1) + k] : -1;
+    const int32_t s = v < n ? v : -1;  // nothing past the rows is read or written, whatever the table holds
+    if (k == 0) rowid[r] = s;
+    else nb[r * T + k - 1] = s;
+  }
+  __syncthreads();
+  uint32_t mine = 0;
+  for (int r = t; r < BM; r += NT) {
+    uint32_t m = 0;
+#pragma unroll
+    for (int k = 0; k < T; ++k) m |= (uint32_t)(nb[r * T + k] >= 0) << k;
+    rmask[r] = m;
+    mine |= m;
+  }
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) mine |= (uint32_t)__shfl_xor((int)mine, d, 64);
+  if (lane == 0) wmask[wave] = mine;
+  __syncthreads();
+  mine = 0;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) mine |= wmask[w];
+  const uint32_t taps = (uint32_t)__builtin_amdgcn_readfirstlane((int)mine);
+  const bool all = first || (last && p.bias);  // rows without a tap are written too
+  if (!taps && !all) return;  // uniform
+
+  const int nk = (int)(Cin / 16), ncb = (int)((Cout + 31) / 32);
+  const int nsteps = __builtin_popcount(taps) * nk;
+  const i32x4_t xr = buffer_rsrc(p.x, n * Cin * 4);
+  const i32x4_t wr = buffer_rsrc(planes, planes_bytes);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)ring;
+  // the issue side of the pipeline: tap, 16-deep step, and the lane's x offsets of the tap
+  uint32_t left = taps;
+  int ik = 0, itap = 0;
+  uint32_t aoff[AW];
+  auto issue_tap = [&]() {
+    itap = __builtin_ctz(left);
+#pragma unroll
+    for (int i = 0; i < AW; ++i) {
+      const int r = (wave * AW + i) * 16 + (lane >> 2), c = (lane & 3) ^ ((r >> 2) & 3);
+      const int32_t s = nb[r * T + itap];
+      aoff[i] = s >= 0 ? (uint32_t)s * (uint32_t)(Cin * 4) + c * 16 : 0x80000000u;  // x is below 2^31 bytes
+    }
+  };
+  auto issue = [&](int slot) {
+    const uint32_t st = lds0 + slot * STAGE;
+#pragma unroll
+    for (int i = 0; i < AW; ++i)
+      lds_load16(xr, aoff[i], (uint32_t)ik * 64, __builtin_amdgcn_readfirstlane(st + (wave * AW + i) * 1024));
+#pragma unroll
+    for (int i = 0; i < BW; ++i) {
+      int g = wave * BW + i;
+      g = g < BSEG ? g : BSEG - 1;
+      int cb = (int)(n0 / 32) + g / 3;
+      cb = cb < ncb ? cb : ncb - 1;  // columns past Cout: computed, never stored
+      const uint32_t off = (uint32_t)((((tap0 + itap) * ncb + cb) * nk + ik) * 3 + g % 3) * 1024u;
+      lds_load16(wr, (uint32_t)lane * 16, __builtin_amdgcn_readfirstlane(off),
+                 __builtin_amdgcn_readfirstlane(st + (ASEG + g) * 1024));
+    }
+  };
+  // advances the issue side; past the last step it stays there (a reload of
+  // the last stage into a slot that is not read again keeps the wait counts)
+  auto advance = [&]() {
+    if (ik + 1 < nk) {
+      ++ik;
+    } else if (left & (left - 1)) {
+      left &= left - 1;
+      ik = 0;
+      issue_tap();
+    }
+  };
+
+  f32x16_t acc[TM][TN], sum[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = f32x16_t{}, sum[i][j] = f32x16_t{};
+  int afr[TM][2];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int r = (wm * TM + i) * 32 + l32;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) afr[i][c] = r * 64 + (((2 * hh + c) ^ ((r >> 2) & 3)) << 4);
+  }
+  const int bfr = ASEG * 1024 + wn * TN * 3072 + lane * 16;
+
+  if (nsteps > 0) {
+    issue_tap();
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      issue(s);
+      advance();
+    }
+    // The next step's fragments are read and split between the current step's
+    // MFMAs: one slot of at most six VALU instructions after each (a slot is
+    // the first or the second half of the split of two values), pinned and
+    // fenced, as the compiler would otherwise sink the whole split to its use,
+    // past the branches below, where no MFMA runs beside it.
+    u32x4_t a[2][3][TM];
+    bf16x8_t b[2][3][TN];
+    float raw[TM][8];
+    auto read_a = [&](int slot) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          const float4 v = *reinterpret_cast<const float4 *>(ring + slot * STAGE + afr[i][c]);
+          raw[i][4 * c] = v.x, raw[i][4 * c + 1] = v.y, raw[i][4 * c + 2] = v.z, raw[i][4 * c + 3] = v.w;
+        }
+    };
+    auto read_b = [&](int slot, bf16x8_t (&fb)[3][TN]) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+          fb[q][j] = *reinterpret_cast<const bf16x8_t *>(ring + slot * STAGE + bfr + (j * 3 + q) * 1024);
+    };
+    // slot h of the split of raw (split3_bf16 in two halves)
+    auto split_slot = [&](int h, u32x4_t (&fa)[3][TM]) {
+      const int i = h / 8, e = h % 8 / 2;
+      float &lo = raw[i][2 * e], &hi = raw[i][2 * e + 1];
+      uint32_t term = pack_bf16x2(lo, hi);
+      lo -= __uint_as_float(term << 16);
+      hi -= __uint_as_float(term & 0xffff0000u);
+      if (h % 2 == 0) {
+        asm volatile("" : "+v"(term), "+v"(lo), "+v"(hi));  // formed here, not where it is used
+        fa[0][i][e] = term;
+      } else {
+        uint32_t last = pack_bf16x2(lo, hi);
+        asm volatile("" : "+v"(term), "+v"(last));
+        fa[1][i][e] = term;
+        fa[2][i][e] = last;
+      }
+    };
+    uint32_t done = taps;
+    int ck = 0, slot = 0;
+    auto step = [&](const u32x4_t (&fa)[3][TM], const bf16x8_t (&fb)[3][TN], u32x4_t (&na)[3][TM],
+                    bf16x8_t (&nb2)[3][TN]) {
+      // the next stage landed, and every wavefront has read this one
+      __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0((NS - 2) * OPS));
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      issue(slot);
+      slot = slot + 1 < NS ? slot + 1 : 0;
+      read_a(slot);
+      read_b(slot, nb2);
+      __builtin_amdgcn_sched_barrier(0);
+      // smallest terms first: (x3 w1, x2 w2, x1 w3), (x2 w1, x1 w2), x1 w1
+      constexpr int ta[6] = {2, 1, 0, 1, 0, 0}, tb[6] = {0, 1, 2, 0, 1, 0};
+      constexpr int SLOTS = 8 * TM, NM = 6 * TM * TN, FREE = NM - SLOTS - 1;  // MFMAs before the first slot
+      static_assert(FREE >= 0, "a slot per MFMA");
+#pragma unroll
+      for (int u = 0; u < NM; ++u) {
+        const int v = u / (TM * TN), i = u / TN % TM, j = u % TN;
+        sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, fa[ta[v]][i]), fb[tb[v]][j],
+                                                            sum[i][j], 0, 0, 0);
+        if (u >= FREE && u < FREE + SLOTS) {
+          split_slot(u - FREE, na);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      advance();
+      if (++ck == nk) {  // the tap is complete: rows that have it add its sum
+        const int k = __builtin_ctz(done);
+        done &= done - 1;
+        ck = 0;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const uint4 m = *reinterpret_cast<const uint4 *>(&rmask[(wm * TM + i) * 32 + 8 * q + 4 * hh]);
+            const uint32_t mq[4] = {m.x, m.y, m.z, m.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const bool has = (mq[e] >> k) & 1u;
+#pragma unroll
+              for (int j = 0; j < TN; ++j) acc[i][j][4 * q + e] += has ? sum[i][j][4 * q + e] : 0.f;
+            }
+          }
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) sum[i][j] = f32x16_t{};
+      }
+    };
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm((NS - 1) * OPS));  // stage 0 landed
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    read_a(0);
+    read_b(0, b[0]);
+#pragma unroll
+    for (int h = 0; h < 8 * TM; ++h) split_slot(h, a[0]);
+    int st = 0;
+    for (; st + 1 < nsteps; st += 2) {
+      step(a[0], b[0], a[1], b[1]);
+      step(a[1], b[1], a[0], b[0]);
+    }
+    if (st < nsteps) step(a[0], b[0], a[1], b[1]);
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));  // the trailing reloads
+  }
+
+  // lane holds rows 8 (e / 4) + 4 hh + e % 4, column l32 of each 32 x 32 tile;
+  // the rows of a tile are distinct, so all reads go out before the writes
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int64_t col = n0 + (wn * TN + j) * 32 + l32;
+    if (col >= Cout) continue;
+    const float bias = last && p.bias ? p.bias[col] : 0.f;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      int32_t d[16];
+      float old[16];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int r = (wm * TM + i) * 32 + 8 * (e >> 2) + 4 * hh + (e & 3);
+        d[e] = all || rmask[r] ? rowid[r] : -1;
+        old[e] = first ? 0.f : p.out[(int64_t)(d[e] >= 0 ? d[e] : 0) * Cout + col];
+      }
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        if (d[e] >= 0) p.out[(int64_t)d[e] * Cout + col] = old[e] + acc[i][j][e] + bias;
+    }
+  }
+}
+
 
 // Any Cin / Cout: one thread per output element, f32 sums in tap, channel order.
 __global__ __launch_bounds__(256) void sparse_conv_generic_kernel(SparseConvParams p) {
@@ -878,6 +1294,77 @@ hipError_t launch_sparse_conv_rulebook(const SparseConvParams &p, const int32_t 
     hipLaunchKernelGGL(fill_rows_kernel, dim3(grid_of(p.n * p.cout)), dim3(256), 0, s, p.out, p.n, p.cout, p.bias,
                        true);
   return hipGetLastError();
+}
+
+template <int T> static hipError_t launch_order(const int32_t *nbr, int64_t n, int32_t *table, int32_t *ws, hipStream_t s) {
+  constexpr int NB = (27 / T) << T;
+  hipLaunchKernelGGL(order_clear_kernel, dim3((NB + 255) / 256), dim3(256), 0, s, ws, NB);
+  if (n == 0) return hipGetLastError();
+  hipLaunchKernelGGL((order_rows_kernel<T, false>), dim3(grid_of(n)), dim3(256), 0, s, nbr, n, ws, table);
+  hipLaunchKernelGGL((order_starts_kernel<T>), dim3(27 / T), dim3(512), 0, s, ws);
+  hipLaunchKernelGGL((order_rows_kernel<T, true>), dim3(grid_of(n)), dim3(256), 0, s, nbr, n, ws, table);
+  return hipGetLastError();
+}
+
+hipError_t launch_sparse_order(const int32_t *nbr, int64_t n, int passes, int32_t *table, int32_t *ws, hipStream_t s) {
+  if (n < 0 || n > INT32_MAX / 27) return hipErrorInvalidValue;
+  if (passes == 3) return launch_order<9>(nbr, n, table, ws, s);
+  if (passes == 9) return launch_order<3>(nbr, n, table, ws, s);
+  return hipErrorInvalidValue;
+}
+
+bool sparse_ordered_fits(int64_t n, int64_t cin, int64_t cout) {
+  // 32-bit offsets of the direct loads (below 2^31 for x: a missing row's
+  // offset is 2^31) and of the weight blocks
+  return cin > 0 && cin % 16 == 0 && cout > 0 && n <= INT32_MAX / 27 && n * cin < (int64_t(1) << 29) &&
+         sparse_weight_planes_bytes(cin, cout) < (int64_t(1) << 31) && ((n + 63) / 64 + 7) * ((cout + 63) / 64) <= INT32_MAX;
+}
+
+template <int V> using I = std::integral_constant<int, V>;
+
+template <int T>
+static hipError_t launch_ordered(const SparseConvParams &p, const int32_t *table, const char *planes, hipStream_t s) {
+  constexpr int S = 27 / T;
+  const int64_t bytes = sparse_weight_planes_bytes(p.cin, p.cout);
+  for (int i = 0; i < S; ++i) {
+    // the pass with the centre tap first: nearly every row has a tap there,
+    // and that pass writes every row
+    const int seg = i == 0 ? S / 2 : (i <= S / 2 ? i - 1 : i);
+    const int32_t *tab = table + (int64_t)seg * p.n * (T + 1);
+    auto run = [&](auto wm, auto wn, auto tm, auto tn, auto ns) {
+      constexpr int BM = wm.value * tm.value * 32, BN = wn.value * tn.value * 32;
+      const int64_t tiles_m = (p.n + BM - 1) / BM, tiles_n = (p.cout + BN - 1) / BN;
+      hipLaunchKernelGGL((sparse_ordered_x3_kernel<wm.value, wn.value, tm.value, tn.value, ns.value, T>),
+                         dim3((unsigned)((tiles_m + 7) / 8 * 8 * tiles_n)), dim3(64 * wm.value * wn.value), 0, s, p, tab, planes,
+                         bytes, seg * T, i == 0, i == S - 1, (int)tiles_n);
+    };
+    // Tiles, measured over 2k-150k voxels and 64-1024 channels (us): 128 x 128,
+    // two per CU, once they number four per CU (24k x 1024: 5395 against 5931
+    // for 64 x 128; 150k x 256: 990 / 1018); below, 64 x 128, which spread
+    // wider and wait less per step (20k x 256: 340 / 405; 2k x 1024: 672 /
+    // 1040). 128 x 64 for up to 64 channels (150k x 64: 202 / 361 for 64 x
+    // 128), and for up to 128 once they number four per CU (100k x 128: 376 /
+    // 393).
+    const int64_t rows = (p.n + 127) / 128;
+    if (p.cout <= 64 || (p.cout <= 128 && 2 * rows >= 1024))
+      run(I<4>{}, I<1>{}, I<1>{}, I<2>{}, I<3>{});
+    else if (rows * ((p.cout + 127) / 128) >= 1024)
+      run(I<2>{}, I<2>{}, I<2>{}, I<2>{}, I<3>{});
+    else
+      run(I<2>{}, I<2>{}, I<1>{}, I<2>{}, I<4>{});
+  }
+  return hipGetLastError();
+}
+
+hipError_t launch_sparse_conv_ordered(const SparseConvParams &p, const int32_t *table, int passes, void *planes,
+                                      hipStream_t s) {
+  if (p.n <= 0 || p.cout <= 0) return hipSuccess;
+  if (!p.mfma || !sparse_ordered_fits(p.n, p.cin, p.cout) || (passes != 3 && passes != 9)) return hipErrorInvalidValue;
+  const int64_t ncb = (p.cout + 31) / 32, blocks = 27 * ncb * (p.cin / 16);
+  hipLaunchKernelGGL(split_weights_kernel, dim3((unsigned)((blocks + 3) / 4)), dim3(256), 0, s, p.w, p.cin, p.cout, ncb,
+                     blocks, static_cast<uint4 *>(planes));
+  const char *pl = static_cast<const char *>(planes);
+  return passes == 3 ? launch_ordered<9>(p, table, pl, s) : launch_ordered<3>(p, table, pl, s);
 }
 
 hipError_t launch_gather_rows(const void *src, int64_t nsrc, const void *ids, bool ids64, int64_t rows,

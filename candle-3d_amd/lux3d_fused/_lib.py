@@ -80,6 +80,8 @@ SIGNATURES = {
     "lux3d_sparse_conv3d": [TP, TP, TP, TP, TP, S],
     "lux3d_sparse_rulebook": [TP, TP, TP, S],
     "lux3d_sparse_conv3d_rulebook": [TP, TP, TP, TP, TP, TP, S],
+    "lux3d_sparse_order": [TP, TP, TP, S],
+    "lux3d_sparse_conv3d_ordered": [TP, TP, TP, TP, TP, TP, S],
     "lux3d_index_select_rows": [TP, TP, TP, TP, S],
     "lux3d_channel_to_spatial": [TP, TP, TP, TP, TP, TP, TP, TP, TP, S],
 }

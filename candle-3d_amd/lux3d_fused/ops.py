@@ -542,6 +542,15 @@ def sparse_neighbors_noalloc(coords: torch.Tensor, nbr: torch.Tensor,
     return nbr
 
 
+def _sparse_order(nbr: torch.Tensor, passes: int) -> torch.Tensor:
+    """lux3d_sparse_order's table int32 [passes, N, 27 / passes + 1] of a neighbour table."""
+    n = nbr.shape[0]
+    table = torch.empty((passes, n, 27 // passes + 1), dtype=torch.int32, device=nbr.device)
+    ws = torch.empty(3 << 9, dtype=torch.int32, device=nbr.device)
+    _lib.call("lux3d_sparse_order", desc(nbr), desc(table), desc(ws), _stream(nbr))
+    return table
+
+
 class SparseConv3d:
     """Submanifold 3x3x3 sparse convolution (trellis2_sparse.rs:135-243).
     `weight` is the checkpoint's flex_gemm layout [Cout, 3, 3, 3, Cin] (or
@@ -559,18 +568,59 @@ class SparseConv3d:
         out = torch.empty((feats.shape[0], self.out_channels), dtype=torch.float32, device=feats.device)
         if isinstance(coords_or_nbr, SparseRulebook):
             rb = coords_or_nbr
-            _lib.call("lux3d_sparse_conv3d_rulebook", desc(feats), desc(rb.pairs), desc(rb.counts),
-                      desc(self.weight27), desc(self.bias), desc(out), _stream(feats))
+            if self._ordered(feats, rb.nbr.shape[0]):
+                self._forward_ordered(rb.tables[_order_passes(feats.shape[0], self.in_channels)], feats, out)
+            else:
+                _lib.call("lux3d_sparse_conv3d_rulebook", desc(feats), desc(rb.pairs), desc(rb.counts),
+                          desc(self.weight27), desc(self.bias), desc(out), _stream(feats))
             return out
         nbr = coords_or_nbr if coords_or_nbr.shape[-1] == 27 else sparse_neighbors(coords_or_nbr)
-        _lib.call("lux3d_sparse_conv3d", desc(feats), desc(nbr), desc(self.weight27), desc(self.bias), desc(out),
-                  _stream(feats))
+        n, cin = nbr.shape[0], self.in_channels
+        # the order of one call's rows costs 21-60 us: output-stationary tiles
+        # are faster where the convolution itself is short (us, with the order:
+        # 3k x 128 140 against 121, 20k x 64 110 / 74; 4k x 256 215 / 248, 20k
+        # x 128 154 / 175, 150k x 64 249 / 271)
+        long = cin >= 256 or (cin >= 128 and n >= 8192) or n >= 98304
+        if (long and nbr.dim() == 2 and nbr.dtype == torch.int32 and nbr.is_contiguous()
+                and self._ordered(feats, n)):
+            self._forward_ordered(_sparse_order(nbr, _order_passes(n, cin)), feats, out)
+        else:
+            _lib.call("lux3d_sparse_conv3d", desc(feats), desc(nbr), desc(self.weight27), desc(self.bias), desc(out),
+                      _stream(feats))
         return out
+
+    def _ordered(self, feats: torch.Tensor, n: int) -> bool:
+        """Whether lux3d_sparse_conv3d_ordered takes this call on n voxels (its layout and size limits). Any other
+        call, an invalid one too, goes to the entry of the pair lists or of the neighbour table."""
+        cin, cout = self.in_channels, self.out_channels
+        return (feats.dim() == 2 and feats.dtype == torch.float32 and tuple(feats.shape) == (n, cin) and n > 0
+                and feats.is_contiguous() and feats.data_ptr() % 16 == 0
+                and tuple(self.weight27.shape) == (27, cout, cin) and self.weight27.dtype == torch.float32
+                and self.weight27.is_contiguous() and self.weight27.data_ptr() % 16 == 0
+                and cin >= 64 and cin % 16 == 0 and cout > 0 and n * cin < 1 << 29
+                and 2 * self._planes_numel() < 1 << 31)
+
+    def _planes_numel(self) -> int:
+        return 27 * ((self.out_channels + 31) // 32 * 32) * self.in_channels * 3
+
+    def _forward_ordered(self, table: torch.Tensor, feats: torch.Tensor, out: torch.Tensor):
+        planes = torch.empty(self._planes_numel(), dtype=torch.bfloat16, device=feats.device)
+        _lib.call("lux3d_sparse_conv3d_ordered", desc(feats), desc(table), desc(self.weight27), desc(planes),
+                  desc(self.bias), desc(out), _stream(feats))
+
+
+def _order_passes(n: int, cin: int) -> int:
+    """Passes of the ordered convolution: 9 (of 3 taps) where a tile's rows would otherwise share too few masks of 9
+    taps and a pass over the output is cheap beside its products (5k x 1024: 1094 against 1272 us, 12k x 1024: 2239 /
+    2419); else 3 (2k x 1024: 672 against 735 us, 40k x 512: 1791 / 1913, 150k x 256: 990 / 1299)."""
+    return 9 if cin >= 768 and 4096 <= n < 24576 else 3
 
 
 class SparseRulebook:
-    """Per-tap (dst, src) pair lists of a coordinate set, built once and reused
-    by every convolution on it (lux3d_sparse_rulebook)."""
+    """Per-tap (dst, src) pair lists of a coordinate set (lux3d_sparse_rulebook)
+    and its rows ordered by the taps they have (lux3d_sparse_order; one table
+    per pass count that a convolution on it may take), built once and reused
+    by every convolution on it."""
 
     def __init__(self, nbr: torch.Tensor):
         n = nbr.shape[0]
@@ -578,6 +628,7 @@ class SparseRulebook:
         self.pairs = torch.empty((27, n, 2), dtype=torch.int32, device=nbr.device)
         self.counts = torch.empty(27, dtype=torch.int32, device=nbr.device)
         _lib.call("lux3d_sparse_rulebook", desc(nbr), desc(self.pairs), desc(self.counts), _stream(nbr))
+        self.tables = {p: _sparse_order(nbr, p) for p in {_order_passes(n, 64), _order_passes(n, 1024)}}
 
 
 def index_select_rows(feats: torch.Tensor, ids: torch.Tensor, bad_ids: Optional[torch.Tensor] = None) -> torch.Tensor:

@@ -455,6 +455,24 @@ int lux3d_sparse_conv3d_rulebook(const lux3d_tensor_t *x, const lux3d_tensor_t *
                                  const lux3d_tensor_t *counts, const lux3d_tensor_t *weight,
                                  const lux3d_tensor_t *bias, const lux3d_tensor_t *out,
                                  lux3d_stream_t stream);
+/* lux3d_sparse_order + lux3d_sparse_conv3d_ordered: the same convolution in
+ * `passes` (3 or 9) launches of 27 / passes consecutive taps each, the rows of
+ * a launch grouped by which of its taps they have, so that only products that
+ * exist (and few others) reach the matrix cores and each output row is touched
+ * once per launch. The order is built once per coordinate set from nbr: table
+ * int32 [passes, N, 27 / passes + 1], workspace int32 [1536]. planes (bf16,
+ * 27 * ceil(Cout / 32) * 32 * Cin * 3 elements) receives the weights' three
+ * bf16 terms on every call; it holds nothing between calls. out = bias + the
+ * taps' sums, each tap summed on its own in f32 (the taps of the middle
+ * launch first). Cin % 16 == 0, 16-byte aligned x, weight and planes, and x
+ * and planes below 2^31 bytes (else LUX3D_ERR_SHAPE / LUX3D_ERR_LAYOUT: use
+ * lux3d_sparse_conv3d).                                                      */
+int lux3d_sparse_order(const lux3d_tensor_t *nbr, const lux3d_tensor_t *table,
+                       const lux3d_tensor_t *workspace, lux3d_stream_t stream);
+int lux3d_sparse_conv3d_ordered(const lux3d_tensor_t *x, const lux3d_tensor_t *table,
+                                const lux3d_tensor_t *weight, const lux3d_tensor_t *planes,
+                                const lux3d_tensor_t *bias, const lux3d_tensor_t *out,
+                                lux3d_stream_t stream);
 int lux3d_index_select_rows(const lux3d_tensor_t *src, const lux3d_tensor_t *ids,
                             const lux3d_tensor_t *out, const lux3d_tensor_t *bad_ids,
                             lux3d_stream_t stream);
