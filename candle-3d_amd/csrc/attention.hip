@@ -101,6 +101,15 @@ __device__ __forceinline__ void split3_into(float a, float b, u32x4_t &x1, u32x4
   x3[e] = r.t3;
 }
 
+// Slots of the 16-byte chunks of K / V rows of D 2-byte elements in LDS
+// without padding: chunk c of row r in slot c ^ k_swz(r) (v_swz(r)). A K
+// fragment read takes one chunk of 16 consecutive rows at a time, a V^T read
+// four consecutive chunks of four rows; each such 256 bytes then cover all 64
+// banks once. (With one swizzle c ^ ((r & 7) * D / 64) for both, every read
+// conflicted two ways: half of the LDS cycles.)
+template <int D> __device__ __forceinline__ int k_swz(int r) { return D == 128 ? r & 15 : (r >> 1) & 7; }
+template <int D> __device__ __forceinline__ int v_swz(int r) { return D == 128 ? (r & 3) << 2 : (r & 2) << 1; }
+
 // The value the partner lane (lane ^ 32) holds, paired with this lane's own:
 // v_permlane32_swap exchanges the two 32-lane halves.
 __device__ __forceinline__ float half_swap_max(float v) {
@@ -119,79 +128,33 @@ __device__ __forceinline__ int64_t xcd_logical_id(int64_t pid, int64_t n) {
   return (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + idx;
 }
 
-// LAZY: the reference maximum m moves only when a block's maximum exceeds it
-// by more than 8 (log2 units), so probabilities exp2(s - m) stay <= 2^8 and
-// the O rescale (skipped by a wave-uniform test while every factor is 1) is
-// rare after the first blocks. The final O / l is the same function.
-// DOT: the row sum l adds the probabilities as rounded for the P v product
-// (v_dot2 of a packed pair with (1, 1)), one instruction per pair.
-// PHASED (QT == 2): P v of query tile 0 is issued before the softmax of
-// tile 1, so the matrix cores and the VALU overlap inside one wavefront.
-// Measured on MI355X (TFLOP/s, VGGT frame / global, D 64): LAZY + DOT +
-// PHASED 617 / 795 against 579 / 700 without; D 128 (TripoSG / TRELLIS.2
-// 16k) LAZY + DOT 718 / 877 against 679 / 827, PHASED by key tile no gain.
-// QP (QP_*): q arrives raw; its head norm and rotation (the head kernels'
-// arithmetic and lane mapping, bit for bit) are applied while the Q
-// fragments are loaded, so the normalised q never goes through HBM.
-// EXACTP: f32 probabilities as three bf16 terms (see the file header).
-template <typename T, int D, int QT, int BKV, int MINW, bool LAZY, bool DOT, bool PHASED, int QP = QP_NONE,
-          bool DMA = false, bool EXACTP = false, int KS = 1>
-__global__ __launch_bounds__(256, MINW) void attn_mfma_kernel(AttnParams p, int64_t nqb, int64_t nwg) {
-  static_assert(!EXACTP || (std::is_same<T, BF16>::value && !DOT), "exact probabilities: bf16, f32 sums");
-  static_assert(KS == 1 || (!PHASED && (BKV / 32) % KS == 0), "key groups: whole 32-key tiles per wavefront");
+// Q of queries q0 .. q0 + 32 QT - 1 of (batch bi, head hi) as the B operand:
+// lane holds Q[query l32][c * 16 + 8 * hh + e] of each 32-query tile (queries
+// past Lq read row Lq - 1). QP: p.q is raw, and its head norm and rotation are
+// applied here, through the wavefront's part qs of an LDS area of 4 QT 32 D
+// elements that no wavefront uses for anything else until the next barrier.
+template <typename T, int D, int QT, int QP>
+__device__ __forceinline__ void load_q(const AttnParams &p, const char *qbase, int64_t bi, int64_t hi, int64_t q0,
+                                       uint16_t *qs, typename Mma<T>::op_t (&qf)[QT][D / 16]) {
   using M = Mma<T>;
   using op_t = typename M::op_t;
-  constexpr int QG = 4 / KS;               // query groups per workgroup (KS wavefronts each)
-  constexpr int BQ = QG * 32 * QT;
-  // 2-byte elements per K / V row in LDS: padded by 16 bytes, or (DMA)
-  // unpadded with 16-byte chunk c of row r in slot c ^ ((r & 7) * D / 64)
-  constexpr int KROW = DMA ? D : D + 8;
-  constexpr int KCH = BKV * D / 8 / 256;   // 16-byte K (and V) chunks per thread per block
-  constexpr int NKT = BKV / 32 / KS;       // 32-key tiles of a block per wavefront
-  constexpr int NDT = D / 32;              // 32-dim output tiles
-  static_assert(KCH >= 1 && BKV % 32 == 0 && D % 32 == 0, "tile shape");
-  __shared__ __align__(16) uint16_t smem[4 * BKV * KROW];
-  uint16_t(*Ks)[BKV * KROW] = reinterpret_cast<uint16_t(*)[BKV * KROW]>(smem);
-  uint16_t(*Vs)[BKV * KROW] = reinterpret_cast<uint16_t(*)[BKV * KROW]>(smem + 2 * BKV * KROW);
-
-  const int64_t lid = xcd_logical_id(blockIdx.x, nwg);
-  const int64_t bh = lid / nqb, qb = lid % nqb;
-  const int64_t bi = bh / p.H, hi = bh % p.H;
-  const char *qbase = reinterpret_cast<const char *>(p.q) + (bi * p.q_sb + hi * p.q_sh) * 2;
-  const char *kbase = reinterpret_cast<const char *>(p.k) + (bi * p.k_sb + hi * p.k_sh) * 2;
-  const char *vbase = reinterpret_cast<const char *>(p.v) + (bi * p.v_sb + hi * p.v_sh) * 2;
-  const int ob = EXACTP && p.out_f32 ? 4 : 2;  // output element bytes
-  char *obase = reinterpret_cast<char *>(p.o) + (bi * p.o_sb + hi * p.o_sh) * ob;
-
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int l32 = lane & 31, hh = lane >> 5;
-  // KS > 1: the KS wavefronts of query group qg hold the same queries and
-  // take key tiles kt0 .. kt0 + NKT - 1 of every block (key group kg)
-  const int qg = wave / KS, kg = wave % KS, kt0 = kg * NKT;
-  const int64_t Lq = p.Lq, Lk = p.Lk;
-
-  // Q as the B operand: lane holds Q[query l32][c * 16 + 8 * hh + e].
-  op_t qf[QT][D / 16];
+  const int lane = threadIdx.x & 63, l32 = lane & 31, hh = lane >> 5;
+  if constexpr (QP == QP_NONE) {
 #pragma unroll
-  for (int qt = 0; qt < QT; ++qt) {
-    int64_t qr = qb * BQ + (qg * QT + qt) * 32 + l32;
-    qr = qr < Lq ? qr : Lq - 1;
-    if constexpr (QP == QP_NONE) {
+    for (int qt = 0; qt < QT; ++qt) {
+      int64_t qr = q0 + qt * 32 + l32;
+      qr = qr < p.Lq ? qr : p.Lq - 1;
 #pragma unroll
       for (int c = 0; c < D / 16; ++c)
         qf[qt][c] = *reinterpret_cast<const op_t *>(qbase + (qr * p.q_st + c * 16 + 8 * hh) * 2);
     }
-  }
-  if constexpr (QP != QP_NONE) {
+  } else {
     // Head norm + rotation of the wavefront's query rows with the head
     // kernels' mapping (D / 8 lanes per row, 8 elements per lane, the same
-    // DPP sums and partner exchange), written as bf16 / f16 into the K / V
-    // staging area, which is not in use yet; then each lane reads its
-    // fragments.
+    // DPP sums and partner exchange), written as bf16 / f16 into the
+    // wavefront's QT * 32 * D elements of qs; then each lane reads its fragments.
     static_assert(D == 64 || D == 128, "Q prologue head dims");
     constexpr int LPR = D / 8, RPP = 64 / LPR;  // lanes per row, rows per pass
-    static_assert(4 * QT * 32 * D <= 4 * BKV * KROW, "Q staging fits the K / V buffers");
-    uint16_t *qs = smem + wave * (QT * 32 * D);
     const int ch = lane % LPR;
     float w8[8], b8[8];
     if constexpr (QP == QP_LN_R1 || QP == QP_RMS) param8(p.qw, p.qw_dt, ch * 8, 1.f, w8);
@@ -208,8 +171,8 @@ __global__ __launch_bounds__(256, MINW) void attn_mfma_kernel(AttnParams p, int6
 #pragma unroll
     for (int it = 0; it < NP; ++it) {
       const int row = lane / LPR + it * RPP;
-      int64_t qr = qb * BQ + qg * QT * 32 + row;
-      qr = qr < Lq ? qr : Lq - 1;
+      int64_t qr = q0 + row;
+      qr = qr < p.Lq ? qr : p.Lq - 1;
       qrs[it] = qr;
       Chunk<T>::template load<false>(qbase + (qr * p.q_st + ch * 8) * 2, xs[it]);
       if constexpr (QP == QP_LN_R1) {
@@ -282,8 +245,65 @@ __global__ __launch_bounds__(256, MINW) void attn_mfma_kernel(AttnParams p, int6
 #pragma unroll
       for (int c = 0; c < D / 16; ++c)
         qf[qt][c] = *reinterpret_cast<const op_t *>(qs + (qt * 32 + l32) * D + c * 16 + 8 * hh);
-    lds_barrier();  // the staging area becomes the K / V buffers below
   }
+}
+
+// LAZY: the reference maximum m moves only when a block's maximum exceeds it
+// by more than 8 (log2 units), so probabilities exp2(s - m) stay <= 2^8 and
+// the O rescale (skipped by a wave-uniform test while every factor is 1) is
+// rare after the first blocks. The final O / l is the same function.
+// DOT: the row sum l adds the probabilities as rounded for the P v product
+// (v_dot2 of a packed pair with (1, 1)), one instruction per pair.
+// PHASED (QT == 2): P v of query tile 0 is issued before the softmax of
+// tile 1, so the matrix cores and the VALU overlap inside one wavefront.
+// Measured on MI355X (TFLOP/s, VGGT frame / global, D 64): LAZY + DOT +
+// PHASED 617 / 795 against 579 / 700 without; D 128 (TripoSG / TRELLIS.2
+// 16k) LAZY + DOT 718 / 877 against 679 / 827, PHASED by key tile no gain.
+// QP (QP_*): q arrives raw; its head norm and rotation (the head kernels'
+// arithmetic and lane mapping, bit for bit) are applied while the Q
+// fragments are loaded, so the normalised q never goes through HBM.
+// EXACTP: f32 probabilities as three bf16 terms (see the file header).
+template <typename T, int D, int QT, int BKV, int MINW, bool LAZY, bool DOT, bool PHASED, int QP = QP_NONE,
+          bool DMA = false, bool EXACTP = false, int KS = 1>
+__global__ __launch_bounds__(256, MINW) void attn_mfma_kernel(AttnParams p, int64_t nqb, int64_t nwg) {
+  static_assert(!EXACTP || (std::is_same<T, BF16>::value && !DOT), "exact probabilities: bf16, f32 sums");
+  static_assert(KS == 1 || (!PHASED && (BKV / 32) % KS == 0), "key groups: whole 32-key tiles per wavefront");
+  using M = Mma<T>;
+  using op_t = typename M::op_t;
+  constexpr int QG = 4 / KS;               // query groups per workgroup (KS wavefronts each)
+  constexpr int BQ = QG * 32 * QT;
+  // 2-byte elements per K / V row in LDS: padded by 16 bytes, or (DMA)
+  // unpadded and swizzled (k_swz, v_swz)
+  constexpr int KROW = DMA ? D : D + 8;
+  constexpr int KCH = BKV * D / 8 / 256;   // 16-byte K (and V) chunks per thread per block
+  constexpr int NKT = BKV / 32 / KS;       // 32-key tiles of a block per wavefront
+  constexpr int NDT = D / 32;              // 32-dim output tiles
+  static_assert(KCH >= 1 && BKV % 32 == 0 && D % 32 == 0, "tile shape");
+  __shared__ __align__(16) uint16_t smem[4 * BKV * KROW];
+  uint16_t(*Ks)[BKV * KROW] = reinterpret_cast<uint16_t(*)[BKV * KROW]>(smem);
+  uint16_t(*Vs)[BKV * KROW] = reinterpret_cast<uint16_t(*)[BKV * KROW]>(smem + 2 * BKV * KROW);
+
+  const int64_t lid = xcd_logical_id(blockIdx.x, nwg);
+  const int64_t bh = lid / nqb, qb = lid % nqb;
+  const int64_t bi = bh / p.H, hi = bh % p.H;
+  const char *qbase = reinterpret_cast<const char *>(p.q) + (bi * p.q_sb + hi * p.q_sh) * 2;
+  const char *kbase = reinterpret_cast<const char *>(p.k) + (bi * p.k_sb + hi * p.k_sh) * 2;
+  const char *vbase = reinterpret_cast<const char *>(p.v) + (bi * p.v_sb + hi * p.v_sh) * 2;
+  const int ob = EXACTP && p.out_f32 ? 4 : 2;  // output element bytes
+  char *obase = reinterpret_cast<char *>(p.o) + (bi * p.o_sb + hi * p.o_sh) * ob;
+
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int l32 = lane & 31, hh = lane >> 5;
+  // KS > 1: the KS wavefronts of query group qg hold the same queries and
+  // take key tiles kt0 .. kt0 + NKT - 1 of every block (key group kg)
+  const int qg = wave / KS, kg = wave % KS, kt0 = kg * NKT;
+  const int64_t Lq = p.Lq, Lk = p.Lk;
+
+  // Q in registers; with a prologue it passes through the K / V buffers
+  op_t qf[QT][D / 16];
+  static_assert(QP == QP_NONE || 4 * QT * 32 * D <= 4 * BKV * KROW, "Q staging fits the K / V buffers");
+  load_q<T, D, QT, QP>(p, qbase, bi, hi, qb * BQ + qg * QT * 32, smem + wave * (QT * 32 * D), qf);
+  if constexpr (QP != QP_NONE) lds_barrier();  // the staging area becomes the K / V buffers below
 
   // Staging: K and V rows as 16-byte chunks, both in their [key][dim]
   // layout. Keys past Lk are clamped to Lk - 1 (finite data; their scores
@@ -309,14 +329,12 @@ __global__ __launch_bounds__(256, MINW) void attn_mfma_kernel(AttnParams p, int6
   // part of the address the hardware range-checks; the scalar offset is not
   // checked) carries the whole in-block offset: keys past Lk fall outside
   // and read as zeros (finite; their scores are masked).
-  constexpr int SWZ = D / 64;
   uint32_t dk_off[KCH], dv_off[KCH];
 #pragma unroll
   for (int i = 0; i < KCH; ++i) {
     const int byte = (wave * KCH + i) * 1024 + lane * 16, r = byte / (2 * D), sl = (byte % (2 * D)) / 16;
-    const int c = sl ^ ((r & 7) * SWZ);
-    dk_off[i] = (uint32_t)(r * p.k_st * 2 + c * 16);
-    dv_off[i] = (uint32_t)(r * p.v_st * 2 + c * 16);
+    dk_off[i] = (uint32_t)(r * p.k_st * 2 + (sl ^ k_swz<D>(r)) * 16);
+    dv_off[i] = (uint32_t)(r * p.v_st * 2 + (sl ^ v_swz<D>(r)) * 16);
   }
   const int64_t kbytes = ((Lk - 1) * p.k_st + D) * 2, vbytes = ((Lk - 1) * p.v_st + D) * 2;
   const int64_t kstep = BKV * p.k_st * 2, vstep = BKV * p.v_st * 2;
@@ -408,7 +426,7 @@ __global__ __launch_bounds__(256, MINW) void attn_mfma_kernel(AttnParams p, int6
         for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
           for (int c = 0; c < D / 16; ++c) {
-            const int krow = (kt0 + kt) * 32 + l32, kch = DMA ? ((2 * c + hh) ^ ((krow & 7) * SWZ)) : 2 * c + hh;
+            const int krow = (kt0 + kt) * 32 + l32, kch = DMA ? (2 * c + hh) ^ k_swz<D>(krow) : 2 * c + hh;
             const op_t a = *reinterpret_cast<const op_t *>(&Ks[buf][krow * KROW + kch * 8]);
             s[qt][kt] = M::run(a, qf[qt][c], s[qt][kt]);
           }
@@ -417,7 +435,7 @@ __global__ __launch_bounds__(256, MINW) void attn_mfma_kernel(AttnParams p, int6
       for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
         for (int c = 0; c < D / 16; ++c) {
-          const int krow = (kt0 + kt) * 32 + l32, kch = DMA ? ((2 * c + hh) ^ ((krow & 7) * SWZ)) : 2 * c + hh;
+          const int krow = (kt0 + kt) * 32 + l32, kch = DMA ? (2 * c + hh) ^ k_swz<D>(krow) : 2 * c + hh;
           const op_t a = *reinterpret_cast<const op_t *>(&Ks[buf][krow * KROW + kch * 8]);
 #pragma unroll
           for (int qt = 0; qt < QT; ++qt) s[qt][kt] = M::run(a, qf[qt][c], s[qt][kt]);
@@ -526,7 +544,7 @@ __global__ __launch_bounds__(256, MINW) void attn_mfma_kernel(AttnParams p, int6
       const int g16 = lane & 15;
       const int vrow = (kt0 + kt) * 32 + 16 * jj + 4 * hh + (g16 >> 2);
       const int vcol = dt * 32 + 16 * ((lane >> 4) & 1) + 4 * (g16 & 3);  // rows vrow and vrow + 8 swizzle alike
-      const int vch = DMA ? ((vcol >> 3) ^ ((vrow & 7) * SWZ)) : vcol >> 3;
+      const int vch = DMA ? (vcol >> 3) ^ v_swz<D>(vrow) : vcol >> 3;
       const uint16_t *vr = &Vs[buf][vrow * KROW + vch * 8 + (vcol & 7)];
       const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t *)(vr));
       const s16x4_t hi2 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t *)(vr + 8 * KROW));
@@ -703,6 +721,286 @@ __global__ __launch_bounds__(256, MINW) void attn_mfma_kernel(AttnParams p, int6
                                    M::pack(o[qt][dt][4 * g + 2] * inv, o[qt][dt][4 * g + 3] * inv));
         *reinterpret_cast<uint2 *>(orow + (dt * 32 + 8 * g + 4 * hh) * 2) = w;
       }
+  }
+}
+
+// ---- pipelined form -------------------------------------------------------------
+//
+// The same arithmetic (LAZY, DOT) with the parts of a key block that depend on
+// each other taken from different blocks. Each of the 4 wavefronts keeps QT
+// tiles of 32 queries; the keys go by 32 per step, and step j is one straight
+// line of MFMAs with everything else in the gaps between them:
+//   scores of block j + 1 (its K fragments were read one step ahead), between
+//   them the exponentials of block j and the reads of V's fragments,
+//   O += P V of block j, between them the last exponentials, the maximum of
+//   block j + 1 and the reads of the K fragments after it.
+// An MFMA takes 32 cycles and up to about 24 cycles of VALU work issue beside
+// it for free (4 FMAs and an exponential per MFMA: 34.8 against 32.5 cycles,
+// one wavefront per SIMD). The order is fenced instruction by instruction:
+// left alone, the scheduler gathers the MFMAs. D 128 (QT 1, two workgroups per
+// CU) is then bound by the matrix cores, about 66% busy, at the clock that
+// this load leaves (about 1.8 GHz); D 64 by the VALU: 32 scores per lane and
+// tile pair are 0.7 us of FMAs, exponentials, packs and sums against 0.5 us of
+// MFMAs per 1000 steps. Before / after, us: TRELLIS.2 12 x 40000 x 128 9354 /
+// 8505, TripoSG 2 x 16 x 2048 x 128 74.5 / 68.1, VGGT 8 frames (D 64) 81.6 /
+// 76.0, 8 frames as one sequence 561 / 529.
+//
+// K and V arrive by direct global -> LDS loads in two stages of 64 keys; stage
+// g holds V's blocks 2 g, 2 g + 1 and K's blocks 2 g + 2, 2 g + 3, as steps 2
+// g and 2 g + 1 read them (what lies past Lk reads as zeros). One barrier per
+// stage; its successor's loads are issued behind it.
+template <typename T, int D, int QT, int MINW, int QP>
+__global__ __launch_bounds__(256, MINW) void attn_pipe_kernel(AttnParams p, int64_t nqb, int64_t nwg) {
+  using M = Mma<T>;
+  using op_t = typename M::op_t;
+  constexpr int BQ = 128 * QT, BK = 32, NS = 2, NC = D / 16, NDT = D / 32;
+  constexpr int KB = BK * D * 2, STAGE = 4 * KB;          // bytes of a block; a stage: V, V, K, K
+  constexpr int SEGW = 2 * KB / 1024 / 4;                 // direct loads per wavefront for two blocks
+  __shared__ __align__(16) char ring[NS * STAGE];
+
+  const int64_t lid = xcd_logical_id(blockIdx.x, nwg);
+  const int64_t bh = lid / nqb, qb = lid % nqb;
+  const int64_t bi = bh / p.H, hi = bh % p.H;
+  const char *qbase = reinterpret_cast<const char *>(p.q) + (bi * p.q_sb + hi * p.q_sh) * 2;
+  const char *kbase = reinterpret_cast<const char *>(p.k) + (bi * p.k_sb + hi * p.k_sh) * 2;
+  const char *vbase = reinterpret_cast<const char *>(p.v) + (bi * p.v_sb + hi * p.v_sh) * 2;
+  char *obase = reinterpret_cast<char *>(p.o) + (bi * p.o_sb + hi * p.o_sh) * 2;
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int l32 = lane & 31, hh = lane >> 5;
+  const int64_t Lq = p.Lq, Lk = p.Lk;
+
+  op_t qf[QT][NC];
+  static_assert(QP == QP_NONE || 4 * QT * 32 * D * 2 <= NS * STAGE, "Q staging fits the ring");
+  load_q<T, D, QT, QP>(p, qbase, bi, hi, qb * BQ + wave * (QT * 32),
+                       reinterpret_cast<uint16_t *>(ring) + wave * (QT * 32 * D), qf);
+  if constexpr (QP != QP_NONE) lds_barrier();
+
+  const int nkv = (int)((Lk + BK - 1) / BK);
+  uint32_t dk_off[SEGW], dv_off[SEGW];
+#pragma unroll
+  for (int i = 0; i < SEGW; ++i) {
+    const int byte = (wave * SEGW + i) * 1024 + lane * 16, r = byte / (2 * D), sl = (byte % (2 * D)) / 16;
+    dk_off[i] = (uint32_t)(r * p.k_st * 2 + (sl ^ k_swz<D>(r)) * 16);
+    dv_off[i] = (uint32_t)(r * p.v_st * 2 + (sl ^ v_swz<D>(r)) * 16);
+  }
+  // the next two blocks of K and of V: their first byte, and the bytes from there to the head's last (none: all
+  // loads read zeros)
+  const char *knext = kbase, *vnext = vbase;
+  int64_t kleft = ((Lk - 1) * p.k_st + D) * 2, vleft = ((Lk - 1) * p.v_st + D) * 2;
+  const int64_t kstep = 2 * BK * p.k_st * 2, vstep = 2 * BK * p.v_st * 2;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)ring;
+  auto dma = [&](const char *&base, int64_t &left, int64_t step, const uint32_t (&off)[SEGW], uint32_t lds) {
+    const i32x4_t rs = buffer_rsrc(base, left > 0 ? left : 0);
+#pragma unroll
+    for (int i = 0; i < SEGW; ++i)
+      lds_load16(rs, off[i], 0, __builtin_amdgcn_readfirstlane(lds + (wave * SEGW + i) * 1024));
+    base += step;
+    left -= step;
+  };
+  auto load_k = [&](int slot) { dma(knext, kleft, kstep, dk_off, lds0 + slot * STAGE + 2 * KB); };
+  auto load_stage = [&](int slot) {
+    dma(vnext, vleft, vstep, dv_off, lds0 + slot * STAGE);
+    load_k(slot);
+  };
+  // K fragment c of a block: rows l32, 16-byte chunk 2 c + hh
+  int kfo[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) kfo[c] = 2 * KB + l32 * 2 * D + (((2 * c + hh) ^ k_swz<D>(l32)) << 4);
+  // at: byte offset of the block in its stage's half, slot * STAGE + (block & 1) * KB
+  auto kfrag = [&](int at, int c) { return *reinterpret_cast<const op_t *>(ring + at + kfo[c]); };
+  // V^T fragment (dim tile dt, keys 16 jj ..), half h (keys + 8 h): see attn_mfma_kernel
+  typedef short s16x4_t __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s16x4_t lds_s16x4_t;
+  const int vr0 = 4 * hh + ((lane & 15) >> 2), vc0 = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+  int vfo[NDT];  // rows 16 jj + 8 h more keep the swizzle's row bits
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt) {
+    const int col = dt * 32 + vc0;
+    vfo[dt] = vr0 * 2 * D + (((col >> 3) ^ v_swz<D>(vr0)) << 4) + (col & 7) * 2;
+  }
+  auto vhalf = [&](int at, int dt, int jj, int h) {
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (lds_s16x4_t *)(ring + at + vfo[dt] + (16 * jj + 8 * h) * 2 * D));
+  };
+
+  f32x16_t o[QT][NDT], sa[QT], sb[QT];
+  float m[QT], l[QT], alpha[QT];
+  op_t kf[NC], pf[QT][2];
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) {
+    m[qt] = -INFINITY;
+    l[qt] = 0.f;
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt) o[qt][dt] = f32x16_t{};
+  }
+  const float c2 = p.scale * kLog2e;
+
+  // scores of block j past Lk become -inf
+  auto mask = [&](int j, f32x16_t (&s)[QT]) {
+    const int lim = (int)(Lk - (int64_t)j * BK) - 4 * hh;
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      if (8 * (i >> 2) + (i & 3) >= lim) {
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) s[qt][i] = -INFINITY;
+      }
+  };
+  // the maximum of tile qt in 8 steps, and the reference maximum it leads to
+  float mx[QT];
+  auto max_step = [&](const f32x16_t (&s)[QT], int qt, int i) {
+    mx[qt] = i == 0 ? fmaxf(s[qt][0], s[qt][1]) : fmaxf(fmaxf(mx[qt], s[qt][2 * i]), s[qt][2 * i + 1]);
+  };
+  auto max_done = [&](int qt) {
+    const float cand = half_swap_max(mx[qt]) * c2;
+    float mn = m[qt];
+    if (cand > mn + 8.f) mn = cand;
+    alpha[qt] = __builtin_amdgcn_exp2f(m[qt] - mn);
+    m[qt] = mn;
+  };
+
+  // prologue: K's blocks 0 and 1 into the slot of stage 1, stage 0, scores of block 0
+  load_k(1);
+  load_stage(0);
+  __builtin_amdgcn_s_waitcnt(waitcnt_vm(2 * SEGW));
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int c = 0; c < NC; ++c) kf[c] = kfrag(STAGE, c);
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) sa[qt] = M::run(kf[c], qf[qt][c], c == 0 ? f32x16_t{} : sa[qt]);
+#pragma unroll
+  for (int c = 0; c < NC; ++c) kf[c] = kfrag(STAGE + KB, c);
+  if (nkv == 1) mask(0, sa);
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) max_step(sa, qt, i);
+    max_done(qt);
+  }
+
+  // One step. NEXT: there is a block j + 1; MASKED: it is the last one.
+  auto step = [&](int j, f32x16_t (&s)[QT], f32x16_t (&sn)[QT], auto next_c, auto masked_c) {
+    constexpr bool NEXT = decltype(next_c)::value, MASKED = decltype(masked_c)::value;
+    constexpr int NA = NEXT ? QT * NC : 0, NB = QT * 2 * NDT, NM = NA + NB;  // MFMAs: scores, P v
+    const int at = (j >> 1 & 1) * STAGE + (j & 1) * KB;
+    if ((j & 1) == 0) {
+      // the stage landed, and every wavefront is done with the one before
+      __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      load_stage((j >> 1 & 1) ^ 1);
+    }
+    bool any = false;
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) any = any || alpha[qt] != 1.f;
+    if (__builtin_amdgcn_ballot_w64(any)) {
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) {
+        l[qt] *= alpha[qt];
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt) o[qt][dt] *= alpha[qt];
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    s16x4_t vh[NDT][2][2];
+    // exponentials, two pairs of scores at a time: 4 FMAs, 4 exponentials, 2 packs, 2 sums
+    auto exp_op = [&](int n) {
+      const int g = n / 12, r = n % 12, qt = g / 4, e0 = 4 * (g % 4);
+      if (r < 4) {
+        s[qt][e0 + r] = __builtin_fmaf(s[qt][e0 + r], c2, -m[qt]);
+      } else if (r < 8) {
+        s[qt][e0 + r - 4] = __builtin_amdgcn_exp2f(s[qt][e0 + r - 4]);
+      } else {
+        const int h = r & 1, pe = e0 / 2 + h;  // packed pair pe of the tile: element pe % 4 of fragment pe / 4
+        u32x4_t pk = __builtin_bit_cast(u32x4_t, pf[qt][pe / 4]);
+        if (r < 10) pk[pe % 4] = M::pack(s[qt][e0 + 2 * h], s[qt][e0 + 2 * h + 1]);
+        else l[qt] = M::sum2(pk[pe % 4], l[qt]);
+        pf[qt][pe / 4] = __builtin_bit_cast(op_t, pk);
+      }
+    };
+    constexpr int NEXP = 48 * QT, NMAX = NEXT ? 9 * QT : 0;  // VALU items per tile: 4 groups of 12; 8 steps and the end
+    // items are spread over the MFMAs: all exponentials by the first P v MFMA of tile 1, tile 0's by the first of
+    // tile 0; without scores of a next block they come first
+    constexpr int EXP_END = NEXT ? NA + NB / 2 : 0;
+    if constexpr (!NEXT) {
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+        for (int jj = 0; jj < 2; ++jj)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) vh[dt][jj][h] = vhalf(at, dt, jj, h);
+#pragma unroll
+      for (int n = 0; n < NEXP; ++n) exp_op(n);
+    }
+#pragma unroll
+    for (int u = 0; u < NM; ++u) {
+      if (u < NA) {
+        const int c = u / QT, qt = u % QT;
+        sn[qt] = M::run(kf[c], qf[qt][c], c == 0 ? f32x16_t{} : sn[qt]);
+        // V's 4 NDT fragment halves, spread over the score MFMAs
+        constexpr int PER = 4 * NDT / (NA ? NA : 1);
+#pragma unroll
+        for (int w = u * PER; w < (u + 1) * PER; ++w) vh[w / 4][w / 2 % 2][w % 2] = vhalf(at, w / 4, w / 2 % 2, w % 2);
+      } else {
+        const int b = u - NA, qt = b / (2 * NDT), jj = b / NDT % 2, dt = b % NDT;
+        const op_t a = __builtin_bit_cast(op_t, __builtin_shufflevector(vh[dt][jj][0], vh[dt][jj][1], 0, 1, 2, 3, 4, 5, 6, 7));
+        o[qt][dt] = M::run(a, pf[qt][jj], o[qt][dt]);
+        if (NEXT && b % QT == 0 && b / QT < NC) kf[b / QT] = kfrag(at, b / QT);
+      }
+      if constexpr (NEXT) {
+#pragma unroll
+        for (int n = 0; n < NEXP; ++n)
+          if (n >= u * NEXP / EXP_END && n < (u + 1) * NEXP / EXP_END) exp_op(n);
+        if (MASKED && u == EXP_END - 1) mask(j + 1, sn);
+#pragma unroll
+        for (int n = 0; n < NMAX; ++n)
+          if (u >= EXP_END && n >= (u - EXP_END) * NMAX / (NM - EXP_END) && n < (u - EXP_END + 1) * NMAX / (NM - EXP_END)) {
+            if (n % 9 < 8) max_step(sn, n / 9, n % 9);
+            else max_done(n / 9);
+          }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  constexpr std::true_type yes{};
+  constexpr std::false_type no{};
+  int j = 0;
+  for (; j + 5 < nkv; j += 4) {  // blocks up to j + 4 are not the last; the stages' offsets are constants
+    step(0, sa, sb, yes, no);
+    step(1, sb, sa, yes, no);
+    step(2, sa, sb, yes, no);
+    step(3, sb, sa, yes, no);
+  }
+  for (; j + 2 < nkv; ++j) {
+    step(j, sa, sb, yes, no);
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) sa[qt] = sb[qt];
+  }
+  if (j + 1 < nkv) {
+    step(j, sa, sb, yes, yes);
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) sa[qt] = sb[qt];
+    ++j;
+  }
+  step(j, sa, sb, no, no);
+  __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));  // the trailing reloads
+
+  // out[query][dim]: lane holds dims dt * 32 + 8 * g + 4 * hh + {0..3}, g = 0..3
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) {
+    const int64_t qr = qb * BQ + (wave * QT + qt) * 32 + l32;
+    const float inv = 1.f / half_swap_sum(l[qt]);
+    if (qr >= Lq) continue;
+    char *orow = obase + qr * p.o_st * 2;
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<uint2 *>(orow + (dt * 32 + 8 * g + 4 * hh) * 2) =
+            make_uint2(M::pack(o[qt][dt][4 * g] * inv, o[qt][dt][4 * g + 1] * inv),
+                       M::pack(o[qt][dt][4 * g + 2] * inv, o[qt][dt][4 * g + 3] * inv));
   }
 }
 
@@ -1083,6 +1381,22 @@ hipError_t launch_mfma(const AttnParams &p, hipStream_t s) {
   return hipGetLastError();
 }
 
+template <typename T, int D, int QT, int MINW>
+hipError_t launch_pipe(const AttnParams &p, hipStream_t s) {
+  const int64_t nqb = (p.Lq + 128 * QT - 1) / (128 * QT), nwg = p.B * p.H * nqb;
+  if (nwg > INT32_MAX || p.Lk > INT32_MAX - 256) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)nwg), block(256);
+#define LUX3D_PIPE(QP) hipLaunchKernelGGL((attn_pipe_kernel<T, D, QT, MINW, QP>), grid, block, 0, s, p, nqb, nwg)
+  switch (p.qpro) {
+    case QP_LN_R1: LUX3D_PIPE(QP_LN_R1); break;
+    case QP_RMS: LUX3D_PIPE(QP_RMS); break;
+    case QP_L2_R2: LUX3D_PIPE(QP_L2_R2); break;
+    default: LUX3D_PIPE(QP_NONE);
+  }
+#undef LUX3D_PIPE
+  return hipGetLastError();
+}
+
 template <typename T>
 hipError_t launch_generic(const AttnParams &p, hipStream_t s) {
   const int64_t rows = p.B * p.H * p.Lq;
@@ -1116,14 +1430,11 @@ hipError_t launch_f32x3(const AttnParams &p, hipStream_t s) {
   return hipGetLastError();
 }
 
-// D 128: K / V as direct global -> LDS loads (DMA) when every key offset of
-// a head fits the 32-bit buffer offsets (TripoSG 87.2 against 92.3 us,
-// TRELLIS.2 40k voxels 10.3 against 11.2 ms, bit-identical). D 64 stays
-// register-staged (with rotating inputs DMA gained nothing there):
-// 128-query workgroups (three per CU) or 256-query ones (the phased form,
-// two per CU), whichever leaves the busiest CU less work (below), also with
-// q's LayerNorm fused (VGGT frame 92.8 against 96.0 us); the exact-
-// probability kernel takes 128-query ones up to kShortQ queries.
+// D 64 and 128 run pipelined with K / V as direct global -> LDS loads when
+// every key offset of a head fits the 32-bit buffer offsets; D 64 in 128-query
+// workgroups (three per CU) or 256-query ones (two per CU), whichever leaves
+// the busiest CU less work (below). The exact-probability kernel takes
+// 128-query ones up to kShortQ queries.
 constexpr int64_t kShortQ = 4096;
 constexpr int64_t kCus = 256;  // MI355X
 
@@ -1133,13 +1444,14 @@ int64_t busiest_cu_time(int64_t nwg, int per_cu, const int *t) {
   const int64_t m = (nwg + kCus - 1) / kCus;
   return (m / per_cu) * t[per_cu] + t[m % per_cu];
 }
-// t: VGGT frames (1374 keys, D 64) timed with k workgroups resident per CU,
-// in 0.1 us: 128-query 20.4 / 32.5 / 45.4 us (k = 1 / 2 / 3), 256-query
-// 32.0 / 54.7 us (k = 1 / 2). The 256-query form must win by 3%; so set,
-// the rule picks the faster form at each of 2 to 8 frames, 1 / 2 / 4 x 2048
-// tokens and DINOv3's 1029 (both forms timed at each).
+// t: VGGT frames (1374 keys, D 64) with k workgroups of the pipelined kernel
+// resident per CU, in 0.1 us: 128-query 17.5 / 27.0 / 39.7 us (k = 1 / 2 / 3),
+// 256-query 28.0 / 49.0 us (k = 1 / 2). The 256-query form must win by 3%; so
+// set, the rule picks the faster form at each of 1 to 10 frames, 7 x 900, 10 x
+// 700, 2 / 4 / 6 / 8 frames as one sequence, 1 / 4 x 2048 and 2 x 1029 tokens
+// (both timed at each).
 bool use_256_query(const AttnParams &p) {
-  static const int t1[4] = {0, 204, 325, 454}, t2[3] = {0, 320, 547};
+  static const int t1[4] = {0, 175, 270, 397}, t2[3] = {0, 280, 490};
   const int64_t n1 = p.B * p.H * ((p.Lq + 127) / 128), n2 = p.B * p.H * ((p.Lq + 255) / 256);
   return 100 * busiest_cu_time(n2, 2, t2) < 97 * busiest_cu_time(n1, 3, t1);
 }
@@ -1151,8 +1463,8 @@ bool use_256_query(const AttnParams &p) {
 // workgroups, each wavefront with 1 / KS of the keys. These kernels are
 // VALU-bound (exact_sdpa_heads: about 370 VALU instructions per 64-key block
 // and wavefront against 32 MFMAs), so the busiest SIMD's share sets the
-// time; KS = 2 is taken while the doubled grid still fits three workgroups
-// per CU. Measured (exact_sdpa_heads bf16, D 64, us, KS = 1 / 2 / 4):
+// time; KS = 2 is taken while the doubled grid stays within max_grid: three
+// workgroups per CU, or one where the pipelined kernel is the other choice. Measured (exact_sdpa_heads bf16, D 64, us, KS = 1 / 2 / 4):
 // 16 heads x 1029 tokens 26.3 / 24.2 / 25.5, x 1024 22.6 / 17.3 / 16.4,
 // 8 x 1029 23.9 / 17.3 / 16.7, 2 x 16 x 1029 37.0 / 32.2 / 38.1, 4 x 4096
 // 78.3 / 55.0 / 50.5, 16 x 2048 45.7 / 43.2 / 50.9; KS = 4 (128-key blocks,
@@ -1160,9 +1472,9 @@ bool use_256_query(const AttnParams &p) {
 // elsewhere, so it is not chosen by default. Needs Lk >= the block (every
 // key group sees keys in block 0). LUX3D_ATTN_KS=1 / 2 / 4 forces a choice
 // (timing).
-int key_groups(const AttnParams &p) {
+int key_groups(const AttnParams &p, int64_t max_grid) {
   const int64_t tiles = p.B * p.H * ((p.Lq + 127) / 128);
-  int ks = 2 * tiles <= 3 * kCus ? 2 : 1;
+  int ks = 2 * tiles <= max_grid ? 2 : 1;
   if (const char *e = getenv("LUX3D_ATTN_KS")) ks = atoi(e);
   if (ks == 4 && p.Lk >= 128) return 4;
   if (ks == 2 && p.Lk >= 64) return 2;
@@ -1185,7 +1497,7 @@ hipError_t launch_t(const AttnParams &p, hipStream_t s) {
     // the generic kernel (f32 throughout)
     if constexpr (T::code == LUX3D_BF16) {
       if (p.mfma && p.D == 64) {
-        const int ks = key_groups(p);
+        const int ks = key_groups(p, 3 * kCus);
         if (ks == 4) return launch_mfma<T, 64, 1, 128, 2, true, false, false, false, true, 4>(p, s);
         if (ks == 2) return launch_mfma<T, 64, 1, 64, 3, true, false, false, false, true, 2>(p, s);
         if (p.Lq <= kShortQ) return launch_mfma<T, 64, 1, 64, 3, true, false, false, false, true>(p, s);
@@ -1200,16 +1512,27 @@ hipError_t launch_t(const AttnParams &p, hipStream_t s) {
   }
   if constexpr (T::code != LUX3D_F32) {
     if (p.mfma) {
+      const bool dma = dma_fits(p, 2);
       if (p.D == 64) {
-        const int ks = key_groups(p);
+        // key groups while their doubled grid leaves CUs idle (16 heads x 1024
+        // tokens: 13.7 us against 15.3 pipelined; x 1029, one more tile: 19.0
+        // / 16.3)
+        const int ks = key_groups(p, dma ? kCus : 3 * kCus);
         if (ks == 4) return launch_mfma<T, 64, 1, 128, 2, true, true, false, false, false, 4>(p, s);
         if (ks == 2) return launch_mfma<T, 64, 1, 64, 3, true, true, false, false, false, 2>(p, s);
-        if (!use_256_query(p))
-          return launch_mfma<T, 64, 1, 64, 3, true, true, false, false>(p, s);
-        return launch_mfma<T, 64, 2, 64, 2, true, true, true, false>(p, s);
+        if (use_256_query(p)) {
+          if (dma) return launch_pipe<T, 64, 2, 2>(p, s);
+          return launch_mfma<T, 64, 2, 64, 2, true, true, true, false>(p, s);
+        }
+        if (dma) return launch_pipe<T, 64, 1, 3>(p, s);
+        return launch_mfma<T, 64, 1, 64, 3, true, true, false, false>(p, s);
       }
       if (p.D == 128) {
-        if (dma_fits(p, 2)) return launch_mfma<T, 128, 1, 64, 2, true, true, false, true>(p, s);
+        // a few key blocks do not pay for the pipeline's first (2 x 16 x 2048
+        // queries: 64 keys 12.0 us against 12.8, 128 13.9 / 14.3, 256 18.3 /
+        // 18.1)
+        if (dma && p.Lk >= 256) return launch_pipe<T, 128, 1, 2>(p, s);
+        if (dma) return launch_mfma<T, 128, 1, 64, 2, true, true, false, true>(p, s);
         return launch_mfma<T, 128, 1, 64, 2, true, true, false, false>(p, s);
       }
     }

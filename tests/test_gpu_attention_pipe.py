@@ -1,0 +1,67 @@
+"""The pipelined attention kernel (D 64 / 128, bf16 / f16) at the edges of its
+key steps and stages, query tiles and dispatch rules, against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+TDT = {"bf16": torch.bfloat16, "f16": torch.float16}
+
+
+@pytest.fixture(scope="module")
+def dev():
+    if not torch.cuda.is_available():
+        pytest.skip("no ROCm device")
+    return torch.device("cuda:0")
+
+
+def _check(got, q, k, v, scale, dt):
+    """|error| <= 4 u max|v| + u |want| with u the type's unit roundoff: a probability's rounding changes a weight by
+    at most u of itself on both sides of the quotient, exponentials and f32 sums stay below another u, and the output
+    is rounded once."""
+    q, k, v = (t.double() for t in (q, k, v))
+    s = q @ k.transpose(-1, -2).contiguous() * scale
+    want = torch.softmax(s, -1) @ v
+    u = 2.0 ** -8 if dt == "bf16" else 2.0 ** -11
+    err = (got.double() - want).abs()
+    bound = 4 * u * v.abs().amax() + u * want.abs()
+    assert bool((err <= bound).all()), float((err / bound).max())
+
+
+# (b, h, lq, lk): 1-9 key blocks of 32 and their remainders, 256 keys (the shortest D 128 takes), one row, query tiles
+# of 128 / 256 and one more, and grids on both sides of each rule of the dispatch
+SHAPES = [(1, 3, 130, 1), (2, 80, 130, 31), (2, 80, 130, 33), (2, 80, 129, 64), (2, 80, 128, 95), (2, 80, 127, 96),
+          (2, 80, 1, 128), (2, 80, 130, 129), (2, 80, 130, 160), (2, 80, 130, 191), (2, 80, 130, 224), (2, 80, 130, 255),
+          (2, 80, 130, 256), (2, 80, 257, 257), (2, 80, 130, 289), (1, 16, 1024, 300), (1, 16, 1029, 300),
+          (4, 16, 2048, 70)]
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("b,h,lq,lk", SHAPES)
+def test_sdpa_pipelined(dev, b, h, lq, lk, d, dt):
+    from lux3d_fused import ops
+    print(f"\n[case] sdpa pipelined [{b},{h},{lq},{lk},{d}] {dt}", flush=True)
+    g = torch.Generator(device="cpu").manual_seed(lq * 7 + lk + d)
+    make = lambda n: torch.randn((b, n, h, d), generator=g).to(dev).to(TDT[dt]).transpose(1, 2)  # noqa: E731
+    q, k, v = make(lq), make(lk), make(lk)
+    k = k * 3    # maxima that move by more than the 2^8 that the running reference allows
+    scale = d ** -0.5
+    out = torch.full((b, h, lq, d), float("nan"), dtype=TDT[dt], device=dev)
+    ops.sdpa(q, k, v, scale, out=out)
+    _check(out, q, k, v, scale, dt)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_sdpa_pipelined_rising_scores(dev, d):
+    """Scores that rise along the keys, so that every block moves the reference maximum and rescales the sums, and a
+    last key that outweighs all others."""
+    from lux3d_fused import ops
+    print(f"\n[case] sdpa pipelined rising scores d={d}", flush=True)
+    b, h, lq, lk = 2, 40, 140, 333
+    g = torch.Generator(device="cpu").manual_seed(d)
+    q = torch.ones((b, h, lq, d)).to(dev).to(torch.bfloat16)
+    k = (torch.arange(lk).float()[None, None, :, None] * 0.25 / d * torch.ones((b, h, lk, d))).to(dev).to(torch.bfloat16)
+    k[:, :, -1] = 120.0 / d
+    v = torch.randn((b, h, lk, d), generator=g).to(dev).to(torch.bfloat16)
+    _check(ops.sdpa(q, k, v, 1.0), q, k, v, 1.0, "bf16")
