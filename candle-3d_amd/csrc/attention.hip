@@ -1004,6 +1004,52 @@ __global__ __launch_bounds__(256, MINW) void attn_pipe_kernel(AttnParams p, int6
   }
 }
 
+// f32 q of queries q0 .. q0 + 31 as the B operand in three bf16 terms: lane
+// holds Q[query l32][c * 16 + 8 * hh + e]. R3: DINOv3's rotate_half rotation
+// (QP_R3) applied with the head kernel's per-element arithmetic (rotate1), bit
+// for bit.
+template <int D, bool R3>
+__device__ __forceinline__ void load_q_f32x3(const AttnParams &p, const float *qbase, int64_t q0,
+                                             bf16x8_t (&q)[3][D / 16]) {
+  const int lane = threadIdx.x & 63, l32 = lane & 31, hh = lane >> 5;
+  int64_t qr = q0 + l32;
+  qr = qr < p.Lq ? qr : p.Lq - 1;
+  const float *qrow = qbase + qr * p.q_st;
+  float xq[D / 16][8];
+#pragma unroll
+  for (int c = 0; c < D / 16; ++c) Chunk<F32>::load<false>(qrow + c * 16 + 8 * hh, xq[c]);
+  if constexpr (R3) {
+    // element j = 16 c + 8 hh + e; its partner j ^ D/2 is element e of the
+    // lane's own chunk c ^ D/32; S = -sin for j < D/2. Tokens before the
+    // prefix pass through (table row clamped to 0, rotation discarded).
+    const bool rot = qr >= p.prefix;
+    const int64_t trow = (rot ? qr - p.prefix : 0) * p.tab_sN;
+    float yq[D / 16][8];
+#pragma unroll
+    for (int c = 0; c < D / 16; ++c) {
+      float C8[8], S8[8];
+      param8(p.tab_c, p.tab_dt, trow + c * 16 + 8 * hh, 1.f, C8);
+      param8(p.tab_s, p.tab_dt, trow + c * 16 + 8 * hh, 0.f, S8);
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        yq[c][e] = rot ? rotate1(xq[c][e], C8[e], xq[c ^ (D / 32)][e], c < D / 32 ? -S8[e] : S8[e]) : xq[c][e];
+    }
+#pragma unroll
+    for (int c = 0; c < D / 16; ++c)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) xq[c][e] = yq[c][e];
+  }
+#pragma unroll
+  for (int c = 0; c < D / 16; ++c) {
+    u32x4_t x1, x2, x3;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) split3_into(xq[c][2 * e], xq[c][2 * e + 1], x1, x2, x3, e);
+    q[0][c] = __builtin_bit_cast(bf16x8_t, x1);
+    q[1][c] = __builtin_bit_cast(bf16x8_t, x2);
+    q[2][c] = __builtin_bit_cast(bf16x8_t, x3);
+  }
+}
+
 // ---- f32 inputs on the bf16 matrix cores (three-term split) --------------------
 //
 // f32 q, k and v are split exactly into three bf16 terms each (x = x1 + x2 +
@@ -1020,8 +1066,6 @@ __global__ __launch_bounds__(256, MINW) void attn_pipe_kernel(AttnParams p, int6
 // of BKV keys are loaded as f32 (keys past Lk clamped to Lk - 1, their scores
 // masked), split in registers and stored as three bf16 planes each, [key][dim]
 // rows padded by 16 bytes, double-buffered.
-// R3: DINOv3's rotate_half rotation of q (QP_R3) applied in the Q load with
-// the head kernel's per-element arithmetic (rotate1), bit for bit.
 template <int D, int BKV, int MINW, bool R3 = false>
 __global__ __launch_bounds__(256, MINW) void attn_f32x3_kernel(AttnParams p, int64_t nqb, int64_t nwg) {
   using op_t = bf16x8_t;
@@ -1045,46 +1089,8 @@ __global__ __launch_bounds__(256, MINW) void attn_f32x3_kernel(AttnParams p, int
   const int l32 = lane & 31, hh = lane >> 5;
   const int64_t Lq = p.Lq, Lk = p.Lk;
 
-  // Q as the B operand, three terms: lane holds Q[query l32][c * 16 + 8 * hh + e]
-  op_t q1[D / 16], q2[D / 16], q3[D / 16];
-  {
-    int64_t qr = qb * BQ + wave * 32 + l32;
-    qr = qr < Lq ? qr : Lq - 1;
-    const float *qrow = qbase + qr * p.q_st;
-    float xq[D / 16][8];
-#pragma unroll
-    for (int c = 0; c < D / 16; ++c) Chunk<F32>::load<false>(qrow + c * 16 + 8 * hh, xq[c]);
-    if constexpr (R3) {
-      // element j = 16 c + 8 hh + e; its partner j ^ D/2 is element e of the
-      // lane's own chunk c ^ D/32; S = -sin for j < D/2. Tokens before the
-      // prefix pass through (table row clamped to 0, rotation discarded).
-      const bool rot = qr >= p.prefix;
-      const int64_t trow = (rot ? qr - p.prefix : 0) * p.tab_sN;
-      float yq[D / 16][8];
-#pragma unroll
-      for (int c = 0; c < D / 16; ++c) {
-        float C8[8], S8[8];
-        param8(p.tab_c, p.tab_dt, trow + c * 16 + 8 * hh, 1.f, C8);
-        param8(p.tab_s, p.tab_dt, trow + c * 16 + 8 * hh, 0.f, S8);
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          yq[c][e] = rot ? rotate1(xq[c][e], C8[e], xq[c ^ (D / 32)][e], c < D / 32 ? -S8[e] : S8[e]) : xq[c][e];
-      }
-#pragma unroll
-      for (int c = 0; c < D / 16; ++c)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) xq[c][e] = yq[c][e];
-    }
-#pragma unroll
-    for (int c = 0; c < D / 16; ++c) {
-      u32x4_t x1, x2, x3;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) split3_into(xq[c][2 * e], xq[c][2 * e + 1], x1, x2, x3, e);
-      q1[c] = __builtin_bit_cast(op_t, x1);
-      q2[c] = __builtin_bit_cast(op_t, x2);
-      q3[c] = __builtin_bit_cast(op_t, x3);
-    }
-  }
+  op_t q[3][D / 16];
+  load_q_f32x3<D, R3>(p, qbase, qb * BQ + wave * 32, q);
   // staging: chunk c = t + 256 i holds K / V row c / (D/4), floats 4 (c % (D/4)) ..
   int s_row[KCH], s_c4[KCH];
 #pragma unroll
@@ -1166,12 +1172,12 @@ __global__ __launch_bounds__(256, MINW) void attn_f32x3_kernel(AttnParams p, int
         const op_t a1 = *reinterpret_cast<const op_t *>(K1 + off);
         const op_t a2 = *reinterpret_cast<const op_t *>(K2 + off);
         const op_t a3 = *reinterpret_cast<const op_t *>(K3 + off);
-        s[kt] = M::run(a3, q1[c], s[kt]);
-        s[kt] = M::run(a2, q2[c], s[kt]);
-        s[kt] = M::run(a1, q3[c], s[kt]);
-        s[kt] = M::run(a2, q1[c], s[kt]);
-        s[kt] = M::run(a1, q2[c], s[kt]);
-        s[kt] = M::run(a1, q1[c], s[kt]);
+        s[kt] = M::run(a3, q[0][c], s[kt]);
+        s[kt] = M::run(a2, q[1][c], s[kt]);
+        s[kt] = M::run(a1, q[2][c], s[kt]);
+        s[kt] = M::run(a2, q[0][c], s[kt]);
+        s[kt] = M::run(a1, q[1][c], s[kt]);
+        s[kt] = M::run(a1, q[0][c], s[kt]);
       }
     }
     if constexpr (MASK) {
@@ -1247,6 +1253,281 @@ __global__ __launch_bounds__(256, MINW) void attn_f32x3_kernel(AttnParams p, int
   const int64_t nfull = tail ? nkv - 1 : nkv;
   for (int64_t j = 0; j < nfull; ++j) step(j, std::false_type{});
   if (tail) step(nkv - 1, std::true_type{});
+
+  // out[query][dim] (f32): lane holds dims dt * 32 + 8 * g + 4 * hh + {0..3}, g = 0..3
+  const int64_t qr = qb * BQ + wave * 32 + l32;
+  const float inv = 1.f / half_swap_sum(l);
+  if (qr < Lq) {
+    float *orow = obase + qr * p.o_st;
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<float4 *>(orow + dt * 32 + 8 * g + 4 * hh) =
+            make_float4(o[dt][4 * g] * inv, o[dt][4 * g + 1] * inv, o[dt][4 * g + 2] * inv, o[dt][4 * g + 3] * inv);
+  }
+}
+
+// The same arithmetic for D 64, pipelined as attn_pipe_kernel: step j is one
+// straight line of 48 MFMAs,
+//   scores of block j + 1, between them block j's exponentials and the split of
+//   its probabilities,
+//   O += P V of block j, between them the maximum of block j + 1 and the split
+//   of K's block j + 2 and V's block j + 1 from registers into LDS,
+// so that a single wavefront per SIMD overlaps the two where there are few
+// workgroups (DINOv3: 16 heads x 9 query tiles on 256 CUs). About 280 VALU
+// instructions per step go into the gaps, in chains of two or more (a lone
+// dependent chain takes 8.5 cycles per instruction). K and V are
+// double-buffered planes of 32 rows of 128 bytes, swizzled (k_swz, v_swz); one
+// barrier per step. Before / after, us: 16 x 1029 x 64 52.7 / 43.0 (1.2 us per
+// step and wavefront, half of it MFMAs; 144 of 256 CUs have work), 8 x 16 x
+// 1374 x 64 347 / 330 (1126 TFLOP/s in bf16 products; large bf16 matrix
+// products reach 1230-1580 here).
+template <bool R3>
+__global__ __launch_bounds__(256, 2) void attn_f32x3_pipe_kernel(AttnParams p, int64_t nqb, int64_t nwg) {
+  using op_t = bf16x8_t;
+  using M = Mma<BF16>;
+  constexpr int D = 64, BQ = 128, BK = 32, NC = D / 16, NDT = D / 32;
+  constexpr int RB = 2 * D, PL = BK * RB, BUF = 3 * PL, V0 = 2 * BUF;  // bytes: plane row, plane, buffer, V's first
+  __shared__ __align__(16) char smem[4 * BUF];                         // K buffers 0, 1, V buffers 0, 1
+
+  const int64_t lid = xcd_logical_id(blockIdx.x, nwg);
+  const int64_t bh = lid / nqb, qb = lid % nqb;
+  const int64_t bi = bh / p.H, hi = bh % p.H;
+  const float *qbase = reinterpret_cast<const float *>(p.q) + bi * p.q_sb + hi * p.q_sh;
+  const float *kbase = reinterpret_cast<const float *>(p.k) + bi * p.k_sb + hi * p.k_sh;
+  const float *vbase = reinterpret_cast<const float *>(p.v) + bi * p.v_sb + hi * p.v_sh;
+  float *obase = reinterpret_cast<float *>(p.o) + bi * p.o_sb + hi * p.o_sh;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int l32 = lane & 31, hh = lane >> 5;
+  const int64_t Lq = p.Lq, Lk = p.Lk;
+
+  op_t q[3][NC];
+  load_q_f32x3<D, R3>(p, qbase, qb * BQ + wave * 32, q);
+
+  // staging: thread t holds floats 4 (t % 16) .. + 3 of rows t / 16 and t / 16 + 16 of a block of K and of V
+  const int srow = t >> 4, sc4 = t & 15;
+  int kw[2], vw[2];  // byte offsets of its 8 bytes in a plane
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int r = srow + 16 * i;
+    kw[i] = r * RB + (((sc4 >> 1) ^ k_swz<D>(r)) << 4) + (sc4 & 1) * 8;
+    vw[i] = V0 + r * RB + (((sc4 >> 1) ^ v_swz<D>(r)) << 4) + (sc4 & 1) * 8;
+  }
+  float raw[4][4];  // K's two rows, V's two rows
+  // rows of block b, those past Lk clamped to Lk - 1 (their scores are masked);
+  // at: the thread's first row of block b while the blocks are whole
+  auto load_rows = [&](const float *base, const float *&at, int64_t st, int64_t b, float (&r0)[4], float (&r1)[4]) {
+    const float *a0 = at, *a1 = at + 16 * st;
+    if ((b + 1) * BK > Lk) {
+      const int64_t k0 = b * BK + srow;
+      a0 = base + (k0 < Lk ? k0 : Lk - 1) * st + sc4 * 4;
+      a1 = base + (k0 + 16 < Lk ? k0 + 16 : Lk - 1) * st + sc4 * 4;
+    }
+    at += BK * st;
+    const float4 u = *reinterpret_cast<const float4 *>(a0);
+    const float4 w = *reinterpret_cast<const float4 *>(a1);
+    r0[0] = u.x, r0[1] = u.y, r0[2] = u.z, r0[3] = u.w;
+    r1[0] = w.x, r1[1] = w.y, r1[2] = w.z, r1[3] = w.w;
+  };
+  const float *kat = kbase + srow * p.k_st + sc4 * 4, *vat = vbase + srow * p.v_st + sc4 * 4;
+  // split3_bf16 of x[0..3] in 22 items of one instruction, two pairs side by
+  // side: an instruction that waits for the one before it takes 8.5 cycles, an
+  // independent one 5 (one wavefront per SIMD)
+  uint32_t tmp[4];
+  auto split_item = [&](int n, float (&x)[4], uint32_t (&t)[3][2]) {
+    const int term = n < 10 ? 0 : n < 20 ? 1 : 2, r = n - 10 * term;
+    if (r < 2) t[term][r] = pack_bf16x2(x[2 * r], x[2 * r + 1]);
+    else if (r < 6) tmp[r - 2] = (r & 1) ? t[term][(r - 2) / 2] & 0xffff0000u : t[term][(r - 2) / 2] << 16;
+    else x[r - 6] -= __uint_as_float(tmp[r - 6]);
+  };
+  uint32_t stt[3][2];
+  // staging item n of row w: the split, then the three writes
+  auto stage_item = [&](int w, int n, int buf) {
+    if (n < 22) {
+      split_item(n, raw[w], stt);
+    } else {
+      char *dst = smem + buf * BUF + (w < 2 ? kw[w] : vw[w - 2]);
+      *reinterpret_cast<uint2 *>(dst + (n - 22) * PL) = make_uint2(stt[n - 22][0], stt[n - 22][1]);
+    }
+  };
+  auto stage_all = [&](int w, int buf) {
+#pragma unroll
+    for (int n = 0; n < 25; ++n) stage_item(w, n, buf);
+  };
+  int kfo[NC], vfo[NDT];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) kfo[c] = l32 * RB + (((2 * c + hh) ^ k_swz<D>(l32)) << 4);
+  const int vr0 = 4 * hh + ((lane & 15) >> 2), vc0 = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt) {
+    const int col = dt * 32 + vc0;
+    vfo[dt] = V0 + vr0 * RB + (((col >> 3) ^ v_swz<D>(vr0)) << 4) + (col & 7) * 2;
+  }
+  typedef short s16x4_t __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s16x4_t lds_s16x4_t;
+  auto kfrag = [&](int buf, int pl, int c) {
+    return *reinterpret_cast<const op_t *>(smem + buf * BUF + pl * PL + kfo[c]);
+  };
+  auto vfrag = [&](int buf, int pl, int dt, int jj) {
+    const char *a = smem + buf * BUF + pl * PL + vfo[dt] + 16 * jj * RB;
+    const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t *)a);
+    const s16x4_t hi2 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t *)(a + 8 * RB));
+    return __builtin_bit_cast(op_t, __builtin_shufflevector(lo, hi2, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+
+  f32x16_t o[NDT], sa, sb;
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt) o[dt] = f32x16_t{};
+  float m = -INFINITY, l = 0.f, alpha = 1.f, mx = -INFINITY;
+  const float c2 = p.scale * kLog2e;
+  const int64_t nkv = (Lk + BK - 1) / BK;
+  auto mask = [&](int64_t j, f32x16_t &s) {
+    const int lim = (int)(Lk - j * BK) - 4 * hh;
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      if (8 * (i >> 2) + (i & 3) >= lim) s[i] = -INFINITY;
+  };
+  auto max_item = [&](const f32x16_t &s, int i) {
+    if (i < 8) {
+      mx = i == 0 ? fmaxf(s[0], s[1]) : fmaxf(fmaxf(mx, s[2 * i]), s[2 * i + 1]);
+    } else {
+      const float cand = half_swap_max(mx) * c2;
+      float mn = m;
+      if (cand > mn + 8.f) mn = cand;
+      alpha = __builtin_amdgcn_exp2f(m - mn);
+      m = mn;
+    }
+  };
+  // smallest terms first: (x3 y1, x2 y2, x1 y3), (x2 y1, x1 y2), x1 y1
+  constexpr int tx[6] = {2, 1, 0, 1, 0, 0}, ty[6] = {0, 1, 2, 0, 1, 0};
+
+  // prologue: K's blocks 0 and 1, V's block 0, scores and maximum of block 0
+  load_rows(kbase, kat, p.k_st, 0, raw[0], raw[1]);
+  load_rows(vbase, vat, p.v_st, 0, raw[2], raw[3]);
+#pragma unroll
+  for (int w = 0; w < 4; ++w) stage_all(w, 0);
+  load_rows(kbase, kat, p.k_st, 1, raw[0], raw[1]);
+  stage_all(0, 1);
+  stage_all(1, 1);
+  load_rows(kbase, kat, p.k_st, 2, raw[0], raw[1]);
+  load_rows(vbase, vat, p.v_st, 1, raw[2], raw[3]);
+  lds_barrier();
+  sa = f32x16_t{};
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int u = 0; u < 6; ++u) sa = M::run(kfrag(0, tx[u], c), q[ty[u]][c], sa);
+  if (nkv == 1) mask(0, sa);
+#pragma unroll
+  for (int i = 0; i < 9; ++i) max_item(sa, i);
+
+  auto step = [&](int64_t j, int buf, f32x16_t &s, f32x16_t &sn, auto next_c, auto masked_c) {
+    constexpr bool NEXT = decltype(next_c)::value, MASKED = decltype(masked_c)::value;
+    lds_barrier();  // what the last step staged is there, and what this one overwrites has been read
+    if (__builtin_amdgcn_ballot_w64(alpha != 1.f)) {
+      l *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt) o[dt] *= alpha;
+    }
+    float ls = 0.f;
+    u32x4_t pp[3][2];  // the three terms of the probabilities of 16 keys each
+    op_t vf[2][3];
+    // block j's exponentials, their sum and their split, four scores at a time
+    // in 34 items: 4 FMAs, 4 exponentials, 4 additions, 22 of the split
+    float x[4], part[2];
+    uint32_t xt[3][2];
+    auto exp_item = [&](int n) {
+      const int e0 = 4 * (n / 34), r = n % 34;
+      if (r < 4) x[r] = __builtin_fmaf(s[e0 + r], c2, -m);
+      else if (r < 8) x[r - 4] = __builtin_amdgcn_exp2f(x[r - 4]);
+      else if (r < 10) part[r - 8] = x[2 * (r - 8)] + x[2 * (r - 8) + 1];
+      else if (r < 12) ls += part[r - 10];
+      else {
+        split_item(r - 12, x, xt);
+        if (r == 33) {
+#pragma unroll
+          for (int q = 0; q < 3; ++q)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) pp[q][e0 / 8][e0 / 2 % 4 + h] = xt[q][h];
+        }
+      }
+    };
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (NEXT) {
+      op_t a[2][3];
+#pragma unroll
+      for (int pl = 0; pl < 3; ++pl) a[0][pl] = kfrag(buf ^ 1, 2 - pl, 0);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < 24; ++u) {
+        const int c = u / 6, v = u % 6;
+        if (v == 0 && c + 1 < NC) {
+#pragma unroll
+          for (int pl = 0; pl < 3; ++pl) a[(c + 1) & 1][pl] = kfrag(buf ^ 1, 2 - pl, c + 1);
+        }
+        sn = M::run(a[c & 1][2 - tx[v]], q[ty[v]][c], u == 0 ? f32x16_t{} : sn);
+#pragma unroll
+        for (int n = 6 * u; n < 6 * u + 6; ++n)
+          if (n < 136) exp_item(n);
+        if (u >= 18 && u < 21) vf[0][u - 18] = vfrag(buf, 20 - u, 0, 0);  // V's first fragments
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (MASKED) mask(j + 1, sn);
+    } else {
+#pragma unroll
+      for (int n = 0; n < 136; ++n) exp_item(n);
+    }
+    l += ls;
+    if constexpr (!NEXT) {
+#pragma unroll
+      for (int pl = 0; pl < 3; ++pl) vf[0][pl] = vfrag(buf, 2 - pl, 0, 0);
+    }
+#pragma unroll
+    for (int u = 0; u < 24; ++u) {
+      const int g = u / 6, w = u % 6, jj = g / NDT, dt = g % NDT;
+      if (w == 0 && g + 1 < 2 * NDT) {
+#pragma unroll
+        for (int pl = 0; pl < 3; ++pl) vf[(g + 1) & 1][pl] = vfrag(buf, 2 - pl, (g + 1) % NDT, (g + 1) / NDT);
+      }
+      o[dt] = M::run(vf[g & 1][2 - tx[w]], __builtin_bit_cast(op_t, pp[ty[w]][jj]), o[dt]);
+      if constexpr (NEXT) {
+        // the maximum after the first MFMAs, then the four staged rows
+        if (u < 4) {
+          max_item(sn, 2 * u);
+          max_item(sn, 2 * u + 1);
+        } else if (u == 4) {
+          max_item(sn, 8);
+        } else {
+#pragma unroll
+          for (int n = 6 * (u - 5); n < 6 * (u - 5) + 6; ++n)
+            if (n < 100) stage_item(n / 25, n % 25, n / 25 < 2 ? buf : buf ^ 1);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if constexpr (NEXT) {
+      load_rows(kbase, kat, p.k_st, j + 3, raw[0], raw[1]);
+      load_rows(vbase, vat, p.v_st, j + 2, raw[2], raw[3]);
+    }
+  };
+  constexpr std::true_type yes{};
+  constexpr std::false_type no{};
+  int64_t j = 0;
+  for (; j + 3 < nkv; j += 2) {  // blocks j + 1 and j + 2 are not the last
+    step(j, 0, sa, sb, yes, no);
+    step(j + 1, 1, sb, sa, yes, no);
+  }
+  if (j + 2 < nkv) {  // an odd number of blocks: one more step, then the next starts from buffer 1
+    step(j, 0, sa, sb, yes, no);
+    step(j + 1, 1, sb, sa, yes, yes);
+    step(j + 2, 0, sa, sb, no, no);
+  } else if (j + 1 < nkv) {
+    step(j, 0, sa, sb, yes, yes);
+    step(j + 1, 1, sb, sa, no, no);
+  } else {
+    step(j, 0, sa, sb, no, no);
+  }
 
   // out[query][dim] (f32): lane holds dims dt * 32 + 8 * g + 4 * hh + {0..3}, g = 0..3
   const int64_t qr = qb * BQ + wave * 32 + l32;
@@ -1418,15 +1699,22 @@ bool dma_fits(const AttnParams &p, int eb) {
   return p.k_st >= 0 && p.v_st >= 0 && ((p.Lk + 64) * st + p.D) * eb < (int64_t(1) << 31);
 }
 
-template <int D, int BKV, int MINW>
 hipError_t launch_f32x3(const AttnParams &p, hipStream_t s) {
   const int64_t nqb = (p.Lq + 127) / 128;
   const int64_t nwg = p.B * p.H * nqb;
   if (nwg > INT32_MAX) return hipErrorInvalidValue;
-  if (p.qpro == QP_R3)
-    hipLaunchKernelGGL((attn_f32x3_kernel<D, BKV, MINW, true>), dim3((unsigned)nwg), dim3(256), 0, s, p, nqb, nwg);
-  else
-    hipLaunchKernelGGL((attn_f32x3_kernel<D, BKV, MINW>), dim3((unsigned)nwg), dim3(256), 0, s, p, nqb, nwg);
+  const dim3 grid((unsigned)nwg), block(256);
+  const bool r3 = p.qpro == QP_R3;
+  if (p.D == 64 && p.Lk >= 192) {  // fewer keys do not pay for the pipeline's start (2 x 50: 6.3 us against 7.4; 16 x 201: 14.1 / 13.8)
+    if (r3) hipLaunchKernelGGL((attn_f32x3_pipe_kernel<true>), grid, block, 0, s, p, nqb, nwg);
+    else hipLaunchKernelGGL((attn_f32x3_pipe_kernel<false>), grid, block, 0, s, p, nqb, nwg);
+  } else if (p.D == 64) {
+    if (r3) hipLaunchKernelGGL((attn_f32x3_kernel<64, 32, 2, true>), grid, block, 0, s, p, nqb, nwg);
+    else hipLaunchKernelGGL((attn_f32x3_kernel<64, 32, 2, false>), grid, block, 0, s, p, nqb, nwg);
+  } else {
+    if (r3) hipLaunchKernelGGL((attn_f32x3_kernel<128, 32, 1, true>), grid, block, 0, s, p, nqb, nwg);
+    else hipLaunchKernelGGL((attn_f32x3_kernel<128, 32, 1, false>), grid, block, 0, s, p, nqb, nwg);
+  }
   return hipGetLastError();
 }
 
@@ -1539,12 +1827,10 @@ hipError_t launch_t(const AttnParams &p, hipStream_t s) {
   } else {
     if (p.mfma) {
       // f32 on the bf16 matrix cores (three-term splits), 32-key blocks: at
-      // D 64 55 KB of LDS and 181 VGPRs, two workgroups per CU; at D 128
-      // 104 KB, one. Against the f32 MFMA kernel this replaced (same box,
+      // D 64 two workgroups per CU, at D 128 (104 KB of LDS) one. Against the f32 MFMA kernel this replaced (same box,
       // graph-timed): VGGT frame 342 against 541 us, TripoSG 401 against 523,
       // DINOv3 52.5 against 86.0
-      if (p.D == 64) return launch_f32x3<64, 32, 2>(p, s);
-      if (p.D == 128) return launch_f32x3<128, 32, 1>(p, s);
+      if (p.D == 64 || p.D == 128) return launch_f32x3(p, s);
     }
   }
   return launch_generic<T>(p, s);

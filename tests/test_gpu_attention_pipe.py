@@ -65,3 +65,48 @@ def test_sdpa_pipelined_rising_scores(dev, d):
     k[:, :, -1] = 120.0 / d
     v = torch.randn((b, h, lk, d), generator=g).to(dev).to(torch.bfloat16)
     _check(ops.sdpa(q, k, v, 1.0), q, k, v, 1.0, "bf16")
+
+
+@pytest.mark.parametrize("lk", [192, 193, 223, 224, 225, 256, 287, 300])
+@pytest.mark.parametrize("rotate", [False, True])
+def test_sdpa_f32_pipelined(dev, lk, rotate):
+    """The pipelined f32 kernel (D 64) over odd and even numbers of 32-key blocks and their remainders, against 64
+    bits: |error| <= (d + lk) 2^-22 max|v|, an f32 sum's last place per product in scores and output."""
+    from lux3d_fused import ops
+    print(f"\n[case] sdpa f32 pipelined lk={lk} rotate={rotate}", flush=True)
+    b, h, d, lq = 1, 3, 64, lk
+    g = torch.Generator(device="cpu").manual_seed(lk)
+    q, k, v = (torch.randn((b, lk, h, d), generator=g).to(dev).transpose(1, 2) for _ in range(3))
+    out = torch.full((b, h, lq, d), float("nan"), device=dev)
+    qd = q.double()
+    if rotate:
+        ang = torch.randn((lq - 5, d), generator=g).to(dev)
+        cos, sin = torch.cos(ang), torch.sin(ang)
+        ops.sdpa_dinov3_rope(q, cos, sin, 5, k, v, 0.125, out=out)
+        t = qd[:, :, 5:]
+        turned = torch.cat([-t[..., d // 2:], t[..., :d // 2]], -1)
+        qd = torch.cat([qd[:, :, :5], t * cos.double() + turned * sin.double()], 2)
+    else:
+        ops.sdpa(q, k, v, 0.125, out=out)
+    want = torch.softmax(qd @ k.double().transpose(-1, -2).contiguous() * 0.125, -1) @ v.double()
+    err = (out.double() - want).abs().max()
+    assert float(err) <= (d + lk) * 2.0 ** -22 * float(v.abs().max())
+
+
+def test_sdpa_f32_pipelined_reversed_keys(dev):
+    """A negative token stride addresses the same keys backwards: the same softmax up to the order of the sums."""
+    from lux3d_fused import _lib, ops
+    print("\n[case] sdpa f32 pipelined reversed keys", flush=True)
+    b, h, lk, d = 1, 2, 333, 64
+    g = torch.Generator(device="cpu").manual_seed(3)
+    q, k, v = (torch.randn((b, h, lk, d), generator=g).to(dev) for _ in range(3))
+
+    def backwards(t):
+        return _lib.descriptor(t.data_ptr() + (lk - 1) * d * 4, _lib.F32, list(t.shape), [h * lk * d, lk * d, -d, 1])
+
+    import ctypes
+    out = torch.empty_like(q)
+    _lib.call("lux3d_sdpa", ops.desc(q), ctypes.pointer(backwards(k)), ctypes.pointer(backwards(v)), 0.125,
+              ops.desc(out), torch.cuda.current_stream().cuda_stream)
+    want = ops.sdpa(q, k.flip(2).contiguous(), v.flip(2).contiguous(), 0.125)
+    assert torch.equal(out, want)
