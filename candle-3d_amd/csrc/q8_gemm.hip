@@ -13,7 +13,9 @@
 // are only 2-byte aligned, into int8 [N, K] row-major plus f32 scales
 // [N, K/32], so the GEMM streams them with 16-byte loads.
 //
-// Three GEMM kernels (each one rounding of the f32 sum per output):
+// Four GEMM kernels (each one rounding of the f32 sum per output):
+// - q8_0_few_rows_kernel (K % 64 == 0, up to 16 rows or few tiles): workgroups of
+//   16 weight rows whose wavefronts split k.
 // - q8_0_gemm_ring_kernel (K % 64 == 0, the common case): a workgroup of NW
 //   wavefronts (8, or 4 for small shapes) computes a BM x 32 NW tile; x, the
 //   int8 weights and the scales stream through a 3-stage LDS ring by direct
@@ -678,6 +680,144 @@ __global__ __launch_bounds__(kX3Threads, 1) void q8_0_gemm_x3_kernel(Q8GemmParam
   }
 }
 
+// ---- few rows --------------------------------------------------------------------
+//
+// One modulation or conditioning vector per batch element, short sequences: the
+// weights' bytes bound them, and tiles of 128 rows leave most CUs idle (72
+// workgroups at N 9216) behind a serial k loop. A workgroup owns 16 weight rows
+// and 16 MT rows of x; its NW wavefronts take pairs of 64-deep chunks of k in
+// turn, each keeping the loads of U chunks in flight, and their sums
+// (v_mfma_f32_16x16x32_bf16: x rows x weight rows) are added in wavefront order
+// through LDS. k order inside a chunk: lane group g = lane / 16 holds weights
+// 16 g .. 16 g + 15 of its row as one 16-byte load (one Q8_0 block, one scale),
+// bytes 8 s .. + 7 in MFMA s, and x alike. XF32: f32 x in three exact bf16
+// terms, the int8 weights exact, one MFMA per term and Q8_0 block (lane group
+// g: weights 8 g .. + 7), the block's sum scaled by d, as q8_0_gemm_x3_kernel
+// does. Before / after, us: M 2, K 1536 -> N 9216 16.9 / 8.0 in bf16 (16 MB of
+// weights: 3.1 us at the copy rate) and 71 / 10.8 in f32; M 64, K 8192 -> N
+// 2048 68 / 38 and 363 / 69.
+template <typename OUT, bool XF32, int NW, int MT>
+__global__ __launch_bounds__(64 * NW) void q8_0_few_rows_kernel(Q8GemmParams p) {
+  typedef float f32x4_t __attribute__((ext_vector_type(4)));
+  constexpr int U = MT == 1 ? (XF32 ? 4 : 8) : 2;  // chunks in flight
+  __shared__ float part[NW][MT * 256];
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), g = lane >> 4;
+  const int64_t n0 = (int64_t)blockIdx.x * 16, m0 = (int64_t)blockIdx.y * 16 * MT;
+  // rows past N and M are clamped: loaded, computed, never stored
+  const int64_t n = n0 + (lane & 15) < p.N ? n0 + (lane & 15) : p.N - 1;
+  const int64_t nch = p.K / 64;
+  const int8_t *wr = p.qs + n * p.K;
+  const float *sr = p.scales + n * (p.K / 32);
+  const char *xr[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int64_t m = m0 + 16 * i + (lane & 15);
+    xr[i] = reinterpret_cast<const char *>(p.x) + (m < p.M ? m : p.M - 1) * p.ldx * (XF32 ? 4 : 2);
+  }
+  f32x4_t acc[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) acc[i] = f32x4_t{};
+  // chunks go to the wavefronts in pairs: whole 128-byte lines of the weights
+  for (int64_t c0 = 2 * wave; c0 < nch; c0 += U * NW) {
+    auto chunk = [&](int u) { return c0 + (int64_t)(u / 2) * 2 * NW + (u & 1); };
+    if constexpr (!XF32) {
+      uint4 w[U], x[U][MT][2];
+      float d[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t c = chunk(u) < nch ? chunk(u) : c0;
+        w[u] = ld16<false>(wr + c * 64 + 16 * g);
+        d[u] = sr[c * 2 + (g >> 1)];
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+          x[u][i][0] = ld16<false>(xr[i] + (c * 64 + 16 * g) * 2);
+          x[u][i][1] = ld16<false>(xr[i] + (c * 64 + 16 * g) * 2 + 16);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (chunk(u) >= nch) break;  // uniform
+        const bf16x8_t b0 = dequant8(w[u].x, w[u].y, d[u]), b1 = dequant8(w[u].z, w[u].w, d[u]);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x[u][i][0]), b0, acc[i], 0, 0, 0);
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x[u][i][1]), b1, acc[i], 0, 0, 0);
+        }
+      }
+    } else {
+      uint2 w[U][2];
+      float d[U][2], x[U][2][MT][8];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t c = chunk(u) < nch ? chunk(u) : c0;
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          w[u][b] = *reinterpret_cast<const uint2 *>(wr + c * 64 + 32 * b + 8 * g);
+          d[u][b] = sr[c * 2 + b];
+#pragma unroll
+          for (int i = 0; i < MT; ++i) Chunk<F32>::load<false>(xr[i] + (c * 64 + 32 * b + 8 * g) * 4, x[u][b][i]);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (chunk(u) >= nch) break;  // uniform
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          const bf16x8_t q = dequant8(w[u][b].x, w[u][b].y, 1.f);
+#pragma unroll
+          for (int i = 0; i < MT; ++i) {
+            uint32_t x1[4], x2[4], x3[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const Split3 r = split3_bf16(x[u][b][i][2 * e], x[u][b][i][2 * e + 1]);
+              x1[e] = r.t1;
+              x2[e] = r.t2;
+              x3[e] = r.t3;
+            }
+            f32x4_t blk = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                __builtin_bit_cast(bf16x8_t, u32x4_t{x3[0], x3[1], x3[2], x3[3]}), q, f32x4_t{}, 0, 0, 0);
+            blk = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                __builtin_bit_cast(bf16x8_t, u32x4_t{x2[0], x2[1], x2[2], x2[3]}), q, blk, 0, 0, 0);
+            blk = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                __builtin_bit_cast(bf16x8_t, u32x4_t{x1[0], x1[1], x1[2], x1[3]}), q, blk, 0, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[i][e] = __builtin_fmaf(blk[e], d[u][b], acc[i][e]);
+          }
+        }
+      }
+    }
+  }
+  // lane holds rows 4 g + e, column lane % 16 of each 16-row tile
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) part[wave][i * 256 + e * 64 + lane] = acc[i][e];
+  __syncthreads();
+  for (int o = t; o < MT * 256; o += 64 * NW) {
+    const int64_t row = m0 + o / 256 * 16 + 4 * ((o & 63) >> 4) + (o >> 6 & 3), col = n0 + (o & 15);
+    if (row >= p.M || col >= p.N) continue;
+    float v = part[0][o];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) v += part[w][o];
+    store1<OUT>(p.y, row * p.ldy + col, v + (p.bias ? p.bias[col] : 0.f));
+  }
+}
+
+template <typename OUT, bool XF32, int MT>
+hipError_t launch_few_rows(const Q8GemmParams &p, hipStream_t s) {
+  // 2048 wavefronts (two per SIMD), or as many as k has chunk pairs
+  const int64_t tn = (p.N + 15) / 16, tm = (p.M + 16 * MT - 1) / (16 * MT);
+  if (tn > INT32_MAX || tm > 65535) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)tn, (unsigned)tm);
+  if (tn * tm * 4 >= 2048 || p.K <= 512)
+    hipLaunchKernelGGL((q8_0_few_rows_kernel<OUT, XF32, 4, MT>), grid, dim3(256), 0, s, p);
+  else if (tn * tm * 8 >= 2048 || p.K <= 1024)
+    hipLaunchKernelGGL((q8_0_few_rows_kernel<OUT, XF32, 8, MT>), grid, dim3(512), 0, s, p);
+  else
+    hipLaunchKernelGGL((q8_0_few_rows_kernel<OUT, XF32, 16, MT>), grid, dim3(1024), 0, s, p);
+  return hipGetLastError();
+}
+
 // The ring kernel's buffer descriptors span one tile (at most 256 rows of x,
 // 256 weight rows and their scales) and must stay below 2^31 bytes; its
 // per-lane offsets are 32-bit.
@@ -700,6 +840,18 @@ constexpr int64_t kRingMinTiles = 256;  // MI355X compute units
 
 template <typename OUT>
 hipError_t launch_tiles(const Q8GemmParams &p, hipStream_t s) {
+  // Few rows: always up to 16; beyond, while the grid of 64 x 16 tiles is below
+  // the line where the 128-row tiles' serial k loop takes as long (bf16 512
+  // tiles: K 1024, N 4096 at 64 / 128 / 200 rows 7.0 / 11.6 / 18.1 us against
+  // 12.0 / 12.3 / 12.5; K 8192, N 2048 at 128 / 200 37.8 / 72.7 against 70.9 /
+  // 70.1; f32 1280 tiles: K 1536, N 9216 at 128 / 200 64.2 / 100.5 against 74.9
+  // / 75.1; K 8192, N 2048 at 512 270 against 366).
+  if (p.K % 64 == 0) {
+    const int64_t tiles64 = (p.M + 63) / 64 * ((p.N + 15) / 16);
+    if (p.M <= 16) return p.x_f32 ? launch_few_rows<OUT, true, 1>(p, s) : launch_few_rows<OUT, false, 1>(p, s);
+    if (p.x_f32 && tiles64 <= 1280) return launch_few_rows<OUT, true, 4>(p, s);
+    if (!p.x_f32 && tiles64 < 512) return launch_few_rows<OUT, false, 4>(p, s);
+  }
   if (p.x_f32) {
     // f32 activations (K % 64 == 0, checked by the caller)
     const int64_t tiles_m = (p.M + 127) / 128, tiles_n = (p.N + 255) / 256;
