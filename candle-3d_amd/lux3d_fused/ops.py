@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import ctypes
 import math
+import struct
 from dataclasses import dataclass
 from typing import Optional
 
@@ -25,17 +26,42 @@ _DT = {torch.float32: _lib.F32, torch.bfloat16: _lib.BF16, torch.float16: _lib.F
 
 def desc(t: Optional[torch.Tensor]):
     """lux3d_tensor_t pointer for a torch tensor (None -> NULL)."""
+    return None if t is None else ctypes.pointer(_d(t))
+
+
+# A call's host time is mostly its descriptors and outputs, and below about 1k
+# rows the call is as long as its host time. Each descriptor is packed at once
+# (the fields of _lib.Tensor: data, dtype, rank, shape[5], stride[5]) and passed
+# by reference: 1.1 us against 3.2 on one CPU core for a store per field. residual_layer_norm of
+# 1029 x 1024: 18.9 -> 10.0 us a call.
+_PACK = [struct.Struct(f"=Qii{r}q{8 * (_lib.MAX_RANK - r)}x{r}q{8 * (_lib.MAX_RANK - r)}x").pack
+         for r in range(_lib.MAX_RANK + 1)]
+
+
+def _d(t: Optional[torch.Tensor]):
+    """lux3d_tensor_t of a torch tensor, to be passed by reference (None -> NULL)."""
     if t is None:
         return None
-    if t.dtype not in _DT:
+    code = _DT.get(t.dtype)
+    if code is None:
         raise TypeError(f"unsupported dtype {t.dtype}")
-    if t.dim() == 0:
-        t = t.reshape(1)
-    d = _lib.descriptor(t.data_ptr(), _DT[t.dtype], list(t.shape), list(t.stride()))
-    return ctypes.pointer(d)
+    shape, stride = t.shape, t.stride()
+    if not shape:
+        shape = stride = (1,)
+    rank = len(shape)
+    return _lib.Tensor.from_buffer_copy(_PACK[rank](t.data_ptr(), code, rank, *shape, *stride))
+
+
+def _new(x: torch.Tensor) -> torch.Tensor:
+    """A new contiguous plain tensor of x's shape, dtype and device."""
+    if type(x) is torch.Tensor:
+        return torch.empty_like(x, memory_format=torch.contiguous_format)
+    return torch.empty(x.shape, dtype=x.dtype, device=x.device)
 
 
 def _stream(t: torch.Tensor) -> int:
+    if t.is_cuda:  # the handle itself, without a torch.cuda.Stream around it
+        return torch._C._cuda_getCurrentRawStream(t.get_device())
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
@@ -53,8 +79,8 @@ def layer_norm(x: torch.Tensor, weight: Optional[torch.Tensor], bias: Optional[t
     """candle_nn::ops::layer_norm(x, w, b, eps) (upstream candle-nn), the op
     behind every `layer_norm(dim, eps, vb)` LayerNorm::forward in the
     reference (e.g. runtime/pi3_encoder.rs:67, runtime/vggt.rs:104)."""
-    y = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-    _lib.call("lux3d_layer_norm", desc(x), desc(weight), desc(bias), eps, desc(y), _stream(x))
+    y = _new(x)
+    _lib.call("lux3d_layer_norm", _d(x), _d(weight), _d(bias), eps, _d(y), _stream(x))
     return y
 
 
@@ -69,10 +95,10 @@ def residual_layer_norm(x: torch.Tensor, a: torch.Tensor, ls_gamma: Optional[tor
     """`h = x + ls(a)`, `y = norm(h)`: LayerScale::forward
     (runtime/nn_blocks.rs:210-214) + residual + LayerNorm::forward as in
     VggtBlock::forward (runtime/vggt.rs:113-124). Returns (h, y)."""
-    h = torch.empty(x.shape, dtype=x.dtype, device=x.device) if h_out is None else h_out
-    y = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-    _lib.call("lux3d_residual_layer_norm", desc(x), desc(a), desc(ls_gamma), desc(weight), desc(bias),
-              eps, desc(h), desc(y), _stream(x))
+    h = _new(x) if h_out is None else h_out
+    y = _new(x)
+    _lib.call("lux3d_residual_layer_norm", _d(x), _d(a), _d(ls_gamma), _d(weight), _d(bias),
+              eps, _d(h), _d(y), _stream(x))
     return h, y
 
 
@@ -84,9 +110,9 @@ def adaln_modulate(x: torch.Tensor, shift: torch.Tensor, scale: torch.Tensor,
     `gate*(...) + x`), per batch element or ragged segment:
     runtime/trellis2_blocks.rs:617-630 (with `modulation + t_emb` via the
     *_base vectors) and runtime/vggt.rs:399-405 (gate variant)."""
-    y = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-    _lib.call("lux3d_adaln_modulate", desc(x), desc(seg_offsets), desc(shift), desc(shift_base),
-              desc(scale), desc(scale_base), desc(gate), desc(gate_base), eps, desc(y), _stream(x))
+    y = _new(x)
+    _lib.call("lux3d_adaln_modulate", _d(x), _d(seg_offsets), _d(shift), _d(shift_base),
+              _d(scale), _d(scale_base), _d(gate), _d(gate_base), eps, _d(y), _stream(x))
     return y
 
 
@@ -94,9 +120,9 @@ def gated_residual(x: torch.Tensor, h: torch.Tensor, gate: torch.Tensor, *, gate
                    seg_offsets: Optional[torch.Tensor] = None,
                    out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """`xs.add(h.broadcast_mul(gate))` (runtime/trellis2_blocks.rs:632-633)."""
-    o = torch.empty(x.shape, dtype=x.dtype, device=x.device) if out is None else out
-    _lib.call("lux3d_gated_residual", desc(x), desc(h), desc(seg_offsets), desc(gate), desc(gate_base),
-              desc(o), _stream(x))
+    o = _new(x) if out is None else out
+    _lib.call("lux3d_gated_residual", _d(x), _d(h), _d(seg_offsets), _d(gate), _d(gate_base),
+              _d(o), _stream(x))
     return o
 
 
@@ -109,11 +135,11 @@ def gated_residual_adaln_modulate(x: torch.Tensor, h: torch.Tensor, gate: Option
     followed by `layer_norm_no_affine(xs)*(1 + scale) + shift`
     (runtime/trellis2_blocks.rs:708-713 sparse block, :637-642 dense block).
     Returns (x_out, y); x_out may be x (in-place residual update)."""
-    xo = torch.empty(x.shape, dtype=x.dtype, device=x.device) if x_out is None else x_out
-    y = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-    _lib.call("lux3d_gated_residual_adaln_modulate", desc(x), desc(h), desc(seg_offsets), desc(gate),
-              desc(gate_base), desc(shift), desc(shift_base), desc(scale), desc(scale_base), eps, desc(xo),
-              desc(y), _stream(x))
+    xo = _new(x) if x_out is None else x_out
+    y = _new(x)
+    _lib.call("lux3d_gated_residual_adaln_modulate", _d(x), _d(h), _d(seg_offsets), _d(gate),
+              _d(gate_base), _d(shift), _d(shift_base), _d(scale), _d(scale_base), eps, _d(xo),
+              _d(y), _stream(x))
     return xo, y
 
 
@@ -154,12 +180,8 @@ class Rope2d:
         b, n, _ = positions.shape
         cos = torch.empty((b, 1, n, token_dim), dtype=torch.float32, device=positions.device)
         sin = torch.empty_like(cos)
-        _lib.call("lux3d_rope2d_tables", desc(positions), self.base, desc(cos), desc(sin), _stream(cos))
+        _lib.call("lux3d_rope2d_tables", _d(positions), self.base, _d(cos), _d(sin), _stream(cos))
         return RopeEmbeddings(cos, sin)
-
-
-def _heads_out(q: torch.Tensor) -> torch.Tensor:
-    return torch.empty(q.shape, dtype=q.dtype, device=q.device)
 
 
 def layernorm_rope_fused(q: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, eps: float,
@@ -167,17 +189,17 @@ def layernorm_rope_fused(q: torch.Tensor, weight: torch.Tensor, bias: torch.Tens
     """candle_nn::ops::layernorm_rope_fused (the fork's CustomOp3, routed at
     runtime/attention_math.rs:139-146): LN(64)+affine then 2D RoPE on a
     (possibly strided) [b, h, n, d] head view; contiguous output."""
-    out = _heads_out(q)
-    _lib.call("lux3d_qk_layernorm_rope2d", desc(q), desc(weight), desc(bias), None, None, None, eps,
-              desc(cos_full), desc(sin_alt_full), desc(out), None, _stream(q))
+    out = _new(q)
+    _lib.call("lux3d_qk_layernorm_rope2d", _d(q), _d(weight), _d(bias), None, None, None, eps,
+              _d(cos_full), _d(sin_alt_full), _d(out), None, _stream(q))
     return out
 
 
 def rope_fused(x: torch.Tensor, cos_full: torch.Tensor, sin_alt_full: torch.Tensor) -> torch.Tensor:
     """candle_nn::ops::rope_fused (runtime/attention_math.rs:162)."""
-    out = _heads_out(x)
-    _lib.call("lux3d_qk_layernorm_rope2d", desc(x), None, None, None, None, None, 0.0,
-              desc(cos_full), desc(sin_alt_full), desc(out), None, _stream(x))
+    out = _new(x)
+    _lib.call("lux3d_qk_layernorm_rope2d", _d(x), None, None, None, None, None, 0.0,
+              _d(cos_full), _d(sin_alt_full), _d(out), None, _stream(x))
     return out
 
 
@@ -201,13 +223,13 @@ def qk_layernorm_rope2d(q: torch.Tensor, k: torch.Tensor, q_norm, k_norm,
     with `positions`, computed in-kernel (no table traffic)."""
     qw, qb, eps = q_norm
     kw, kb, _ = k_norm
-    qo, ko = _heads_out(q), _heads_out(k)
+    qo, ko = _new(q), _new(k)
     if positions is not None:
-        _lib.call("lux3d_qk_layernorm_rope2d_pos", desc(q), desc(qw), desc(qb), desc(k), desc(kw), desc(kb),
-                  eps, desc(positions), base, desc(qo), desc(ko), _stream(q))
+        _lib.call("lux3d_qk_layernorm_rope2d_pos", _d(q), _d(qw), _d(qb), _d(k), _d(kw), _d(kb),
+                  eps, _d(positions), base, _d(qo), _d(ko), _stream(q))
     else:
-        _lib.call("lux3d_qk_layernorm_rope2d", desc(q), desc(qw), desc(qb), desc(k), desc(kw), desc(kb),
-                  eps, desc(embeddings.cos_full), desc(embeddings.sin_alt_full), desc(qo), desc(ko),
+        _lib.call("lux3d_qk_layernorm_rope2d", _d(q), _d(qw), _d(qb), _d(k), _d(kw), _d(kb),
+                  eps, _d(embeddings.cos_full), _d(embeddings.sin_alt_full), _d(qo), _d(ko),
                   _stream(q))
     return qo, ko
 
@@ -221,10 +243,10 @@ def rms_norm_heads(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6,
     """RmsNormHeads::rms_norm_heads (runtime/triposg_dit.rs:509-522) on a
     [B, H, L, D] head view (strided views accepted: the transpose/contiguous
     before it is fused). With `k`, both norms run in one launch."""
-    qo = _heads_out(x)
-    ko = _heads_out(k) if k is not None else None
-    _lib.call("lux3d_rms_norm_heads", desc(x), desc(weight), desc(k), desc(k_weight), eps, desc(qo),
-              desc(ko), _stream(x))
+    qo = _new(x)
+    ko = _new(k) if k is not None else None
+    _lib.call("lux3d_rms_norm_heads", _d(x), _d(weight), _d(k), _d(k_weight), eps, _d(qo),
+              _d(ko), _stream(x))
     return qo if k is None else (qo, ko)
 
 
@@ -239,9 +261,9 @@ class Trellis2QkRmsNorm:
         self.gamma = gamma
 
     def forward(self, xs: torch.Tensor) -> torch.Tensor:
-        out = _heads_out(xs)
-        _lib.call("lux3d_qk_l2norm_rope3d", desc(xs), desc(self.gamma), None, None, None, None, None, 0.0,
-                  desc(out), None, _stream(xs))
+        out = _new(xs)
+        _lib.call("lux3d_qk_l2norm_rope3d", _d(xs), _d(self.gamma), None, None, None, None, None, 0.0,
+                  _d(out), None, _stream(xs))
         return out
 
 
@@ -257,14 +279,14 @@ class Trellis2Rope3d:
         n = coords.shape[0]
         cos = torch.empty((n, self.head_dim // 2), dtype=torch.float32, device=coords.device)
         sin = torch.empty_like(cos)
-        _lib.call("lux3d_rope3d_tables", desc(coords), self.head_dim, self.rope_base, desc(cos), desc(sin),
+        _lib.call("lux3d_rope3d_tables", _d(coords), self.head_dim, self.rope_base, _d(cos), _d(sin),
                   _stream(cos))
         return cos, sin
 
     def apply(self, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
-        out = _heads_out(x)
-        _lib.call("lux3d_qk_l2norm_rope3d", desc(x), None, None, None, desc(cos), desc(sin), None, 0.0,
-                  desc(out), None, _stream(x))
+        out = _new(x)
+        _lib.call("lux3d_qk_l2norm_rope3d", _d(x), None, None, None, _d(cos), _d(sin), None, 0.0,
+                  _d(out), None, _stream(x))
         return out
 
 
@@ -274,18 +296,18 @@ def qk_l2norm_rope3d(q: torch.Tensor, k: torch.Tensor, q_gamma: Optional[torch.T
                      rope_base: float = 10000.0):
     """Trellis2SelfAttention::attention's q/k stage
     (runtime/trellis2_blocks.rs:423-430) on [B, L, H, D] views, one launch."""
-    qo, ko = _heads_out(q), _heads_out(k)
-    _lib.call("lux3d_qk_l2norm_rope3d", desc(q), desc(q_gamma), desc(k), desc(k_gamma), desc(cos), desc(sin),
-              desc(coords), rope_base, desc(qo), desc(ko), _stream(q))
+    qo, ko = _new(q), _new(k)
+    _lib.call("lux3d_qk_l2norm_rope3d", _d(q), _d(q_gamma), _d(k), _d(k_gamma), _d(cos), _d(sin),
+              _d(coords), rope_base, _d(qo), _d(ko), _stream(q))
     return qo, ko
 
 
 def apply_rotary_to_patches(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
                             num_prefix: int):
     """apply_rotary_to_patches (runtime/trellis2_dino.rs:406-436)."""
-    qo, ko = _heads_out(q), _heads_out(k)
-    _lib.call("lux3d_dinov3_rope", desc(q), desc(k), desc(cos), desc(sin), int(num_prefix), desc(qo),
-              desc(ko), _stream(q))
+    qo, ko = _new(q), _new(k)
+    _lib.call("lux3d_dinov3_rope", _d(q), _d(k), _d(cos), _d(sin), int(num_prefix), _d(qo),
+              _d(ko), _stream(q))
     return qo, ko
 
 
@@ -294,8 +316,8 @@ def apply_rotary_to_patches(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor,
 # ---------------------------------------------------------------------------
 
 def _act(name: str, x: torch.Tensor, out: Optional[torch.Tensor]) -> torch.Tensor:
-    y = torch.empty(x.shape, dtype=x.dtype, device=x.device) if out is None else out
-    _lib.call(name, desc(x), desc(y), _stream(x))
+    y = _new(x) if out is None else out
+    _lib.call(name, _d(x), _d(y), _stream(x))
     return y
 
 
@@ -340,8 +362,8 @@ def timestep_embedding(t: torch.Tensor, dim: int, cos_first: bool = True,
     or TripoSgDiT::timestep_embedding (runtime/triposg_dit.rs:280-297, sin
     first) for a batch of f32 timesteps t [n] -> [n, dim] f32."""
     out = torch.empty((t.numel(), dim), dtype=torch.float32, device=t.device)
-    _lib.call("lux3d_timestep_embedding", desc(t.reshape(-1)), desc(freqs), int(dim), 1 if cos_first else 0,
-              desc(out), _stream(t))
+    _lib.call("lux3d_timestep_embedding", _d(t.reshape(-1)), _d(freqs), int(dim), 1 if cos_first else 0,
+              _d(out), _stream(t))
     return out
 
 
@@ -349,7 +371,7 @@ def dequantize_q8_0(blocks: torch.Tensor, shape, dtype=torch.bfloat16) -> torch.
     """QTensor::dequantize for a GGML Q8_0 tensor (runtime/nn_blocks.rs:140):
     u8 blocks [nblocks*34] -> dtype tensor of `shape`, bit-exact."""
     y = torch.empty(tuple(shape), dtype=dtype, device=blocks.device)
-    _lib.call("lux3d_dequant_q8_0", desc(blocks.reshape(-1)), desc(y), _stream(y))
+    _lib.call("lux3d_dequant_q8_0", _d(blocks.reshape(-1)), _d(y), _stream(y))
     return y
 
 
@@ -363,7 +385,7 @@ def q8_0_repack(blocks: torch.Tensor, n: int, k: int):
     (qs int8 [n, k], scales f32 [n, k/32]), exact."""
     qs = torch.empty((n, k), dtype=torch.int8, device=blocks.device)
     scales = torch.empty((n, k // 32), dtype=torch.float32, device=blocks.device)
-    _lib.call("lux3d_q8_0_repack", desc(blocks.reshape(-1)), int(n), int(k), desc(qs), desc(scales),
+    _lib.call("lux3d_q8_0_repack", _d(blocks.reshape(-1)), int(n), int(k), _d(qs), _d(scales),
               _stream(blocks))
     return qs, scales
 
@@ -375,7 +397,7 @@ def q8_0_linear(x: torch.Tensor, qs: torch.Tensor, scales: torch.Tensor, bias: O
     (f32 x: the weights dequantized exactly to f32, k a multiple of 64)."""
     n = qs.shape[0]
     y = torch.empty(tuple(x.shape[:-1]) + (n,), dtype=out_dtype, device=x.device)
-    _lib.call("lux3d_q8_0_linear", desc(x), desc(qs), desc(scales), desc(bias), desc(y), _stream(x))
+    _lib.call("lux3d_q8_0_linear", _d(x), _d(qs), _d(scales), _d(bias), _d(y), _stream(x))
     return y
 
 
@@ -387,7 +409,7 @@ def q8_0_quantize(x: torch.Tensor):
     k = x.shape[-1]
     rows = x.numel() // k
     xq, xd = _q8_workspace(rows, k, x.device)
-    _lib.call("lux3d_q8_0_quantize", desc(x), desc(xq), desc(xd), _stream(x))
+    _lib.call("lux3d_q8_0_quantize", _d(x), _d(xq), _d(xd), _stream(x))
     return xq, xd[:, :rows].t()
 
 
@@ -409,7 +431,7 @@ def q8_0_linear_int8(x: torch.Tensor, qs: torch.Tensor, scales: torch.Tensor,
     rows = x.numel() // k
     xq, xd = _q8_workspace(rows, k, x.device)
     y = torch.empty(tuple(x.shape[:-1]) + (n,), dtype=torch.float32, device=x.device)
-    _lib.call("lux3d_q8_0_linear_int8", desc(x), desc(qs), desc(scales), desc(bias), desc(xq), desc(xd), desc(y),
+    _lib.call("lux3d_q8_0_linear_int8", _d(x), _d(qs), _d(scales), _d(bias), _d(xq), _d(xd), _d(y),
               _stream(x))
     return y
 
@@ -436,8 +458,8 @@ def sdpa(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float,
     [B, H, Lq, D]) may be any view with a unit inner stride, e.g. the
     [B, Lq, H, D] layout the caller transposes to next."""
     if out is None:
-        out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-    _lib.call("lux3d_sdpa", desc(q), desc(k), desc(v), float(scale), desc(out), _stream(q))
+        out = _new(q)
+    _lib.call("lux3d_sdpa", _d(q), _d(k), _d(v), float(scale), _d(out), _stream(q))
     return out
 
 
@@ -449,9 +471,9 @@ def sdpa_layernorm_rope2d(q_raw: torch.Tensor, q_norm, embeddings: "RopeEmbeddin
     normalised and rotated."""
     w, b, eps = q_norm
     if out is None:
-        out = torch.empty(q_raw.shape, dtype=q_raw.dtype, device=q_raw.device)
-    _lib.call("lux3d_sdpa_layernorm_rope2d", desc(q_raw), desc(w), desc(b), float(eps), desc(embeddings.cos_full),
-              desc(embeddings.sin_alt_full), desc(k), desc(v), float(scale), desc(out), _stream(q_raw))
+        out = _new(q_raw)
+    _lib.call("lux3d_sdpa_layernorm_rope2d", _d(q_raw), _d(w), _d(b), float(eps), _d(embeddings.cos_full),
+              _d(embeddings.sin_alt_full), _d(k), _d(v), float(scale), _d(out), _stream(q_raw))
     return out
 
 
@@ -461,9 +483,9 @@ def sdpa_rms_norm_heads(q_raw: torch.Tensor, q_w: torch.Tensor, eps: float, k: t
     (triposg_dit.rs:446-455) with q's per-head RMSNorm done in the attention
     kernel's Q load; k already normalised."""
     if out is None:
-        out = torch.empty(q_raw.shape, dtype=q_raw.dtype, device=q_raw.device)
-    _lib.call("lux3d_sdpa_rms_norm_heads", desc(q_raw), desc(q_w), float(eps), desc(k), desc(v), float(scale),
-              desc(out), _stream(q_raw))
+        out = _new(q_raw)
+    _lib.call("lux3d_sdpa_rms_norm_heads", _d(q_raw), _d(q_w), float(eps), _d(k), _d(v), float(scale),
+              _d(out), _stream(q_raw))
     return out
 
 
@@ -475,9 +497,9 @@ def sdpa_l2norm_rope3d(q_raw: torch.Tensor, q_gamma: torch.Tensor, cos: torch.Te
     scale) with q's L2 norm (gamma [H, D]) and 3D RoPE (tables [L, D/2]) done
     in the attention kernel's Q load; k already normalised and rotated."""
     if out is None:
-        out = torch.empty(q_raw.shape, dtype=q_raw.dtype, device=q_raw.device)
-    _lib.call("lux3d_sdpa_l2norm_rope3d", desc(q_raw), desc(q_gamma), desc(cos), desc(sin), desc(k), desc(v),
-              float(scale), desc(out), _stream(q_raw))
+        out = _new(q_raw)
+    _lib.call("lux3d_sdpa_l2norm_rope3d", _d(q_raw), _d(q_gamma), _d(cos), _d(sin), _d(k), _d(v),
+              float(scale), _d(out), _stream(q_raw))
     return out
 
 
@@ -487,9 +509,9 @@ def sdpa_dinov3_rope(q_raw: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, 
     (trellis2_dino.rs:385-393) with q's rotate_half RoPE done in the
     attention kernel's Q load; k already rotated."""
     if out is None:
-        out = torch.empty(q_raw.shape, dtype=q_raw.dtype, device=q_raw.device)
-    _lib.call("lux3d_sdpa_dinov3_rope", desc(q_raw), desc(cos), desc(sin), int(num_prefix), desc(k), desc(v),
-              float(scale), desc(out), _stream(q_raw))
+        out = _new(q_raw)
+    _lib.call("lux3d_sdpa_dinov3_rope", _d(q_raw), _d(cos), _d(sin), int(num_prefix), _d(k), _d(v),
+              float(scale), _d(out), _stream(q_raw))
     return out
 
 
@@ -503,8 +525,8 @@ def exact_sdpa_heads(q, k, v, scale: float, out: Optional[torch.Tensor] = None) 
     """attention_math.rs:244-259: f32 arithmetic whatever q's dtype, output
     in q's dtype (default) or in `out`, which may also be f32."""
     if out is None:
-        out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-    _lib.call("lux3d_sdpa_heads_f32", desc(q), desc(k), desc(v), float(scale), desc(out), _stream(q))
+        out = _new(q)
+    _lib.call("lux3d_sdpa_heads_f32", _d(q), _d(k), _d(v), float(scale), _d(out), _stream(q))
     return out
 
 
@@ -528,7 +550,7 @@ def sparse_neighbors(coords: torch.Tensor, bad_coords: Optional[torch.Tensor] = 
     keys = torch.empty(cap, dtype=torch.int64, device=coords.device)
     vals = torch.empty(cap, dtype=torch.int32, device=coords.device)
     nbr = torch.empty((n, 27), dtype=torch.int32, device=coords.device)
-    _lib.call("lux3d_sparse_neighbors", desc(coords), desc(keys), desc(vals), desc(nbr), desc(bad_coords),
+    _lib.call("lux3d_sparse_neighbors", _d(coords), _d(keys), _d(vals), _d(nbr), _d(bad_coords),
               _stream(coords))
     return nbr
 
@@ -538,7 +560,7 @@ def sparse_neighbors_noalloc(coords: torch.Tensor, nbr: torch.Tensor,
     """sparse_neighbors into a caller-provided `nbr` (int32 [N, 27]) with the
     hash table in the library's per-device static array: the library
     allocates nothing. N <= 2^20; calls that overlap on one GPU race."""
-    _lib.call("lux3d_sparse_neighbors_noalloc", desc(coords), desc(nbr), desc(bad_coords), _stream(coords))
+    _lib.call("lux3d_sparse_neighbors_noalloc", _d(coords), _d(nbr), _d(bad_coords), _stream(coords))
     return nbr
 
 
@@ -547,7 +569,7 @@ def _sparse_order(nbr: torch.Tensor, passes: int) -> torch.Tensor:
     n = nbr.shape[0]
     table = torch.empty((passes, n, 27 // passes + 1), dtype=torch.int32, device=nbr.device)
     ws = torch.empty(3 << 9, dtype=torch.int32, device=nbr.device)
-    _lib.call("lux3d_sparse_order", desc(nbr), desc(table), desc(ws), _stream(nbr))
+    _lib.call("lux3d_sparse_order", _d(nbr), _d(table), _d(ws), _stream(nbr))
     return table
 
 
@@ -571,8 +593,8 @@ class SparseConv3d:
             if self._ordered(feats, rb.nbr.shape[0]):
                 self._forward_ordered(rb.tables[_order_passes(feats.shape[0], self.in_channels)], feats, out)
             else:
-                _lib.call("lux3d_sparse_conv3d_rulebook", desc(feats), desc(rb.pairs), desc(rb.counts),
-                          desc(self.weight27), desc(self.bias), desc(out), _stream(feats))
+                _lib.call("lux3d_sparse_conv3d_rulebook", _d(feats), _d(rb.pairs), _d(rb.counts),
+                          _d(self.weight27), _d(self.bias), _d(out), _stream(feats))
             return out
         nbr = coords_or_nbr if coords_or_nbr.shape[-1] == 27 else sparse_neighbors(coords_or_nbr)
         n, cin = nbr.shape[0], self.in_channels
@@ -585,7 +607,7 @@ class SparseConv3d:
                 and self._ordered(feats, n)):
             self._forward_ordered(_sparse_order(nbr, _order_passes(n, cin)), feats, out)
         else:
-            _lib.call("lux3d_sparse_conv3d", desc(feats), desc(nbr), desc(self.weight27), desc(self.bias), desc(out),
+            _lib.call("lux3d_sparse_conv3d", _d(feats), _d(nbr), _d(self.weight27), _d(self.bias), _d(out),
                       _stream(feats))
         return out
 
@@ -605,8 +627,8 @@ class SparseConv3d:
 
     def _forward_ordered(self, table: torch.Tensor, feats: torch.Tensor, out: torch.Tensor):
         planes = torch.empty(self._planes_numel(), dtype=torch.bfloat16, device=feats.device)
-        _lib.call("lux3d_sparse_conv3d_ordered", desc(feats), desc(table), desc(self.weight27), desc(planes),
-                  desc(self.bias), desc(out), _stream(feats))
+        _lib.call("lux3d_sparse_conv3d_ordered", _d(feats), _d(table), _d(self.weight27), _d(planes),
+                  _d(self.bias), _d(out), _stream(feats))
 
 
 def _order_passes(n: int, cin: int) -> int:
@@ -627,7 +649,7 @@ class SparseRulebook:
         self.nbr = nbr
         self.pairs = torch.empty((27, n, 2), dtype=torch.int32, device=nbr.device)
         self.counts = torch.empty(27, dtype=torch.int32, device=nbr.device)
-        _lib.call("lux3d_sparse_rulebook", desc(nbr), desc(self.pairs), desc(self.counts), _stream(nbr))
+        _lib.call("lux3d_sparse_rulebook", _d(nbr), _d(self.pairs), _d(self.counts), _stream(nbr))
         self.tables = {p: _sparse_order(nbr, p) for p in {_order_passes(n, 64), _order_passes(n, 1024)}}
 
 
@@ -635,7 +657,7 @@ def index_select_rows(feats: torch.Tensor, ids: torch.Tensor, bad_ids: Optional[
     """index_select_rows (trellis2_sparse.rs:117-131): feats[ids] along dim 0.
     `bad_ids` (int32 [1]) receives the number of ids outside [0, rows)."""
     out = torch.empty((ids.shape[0],) + tuple(feats.shape[1:]), dtype=feats.dtype, device=feats.device)
-    _lib.call("lux3d_index_select_rows", desc(feats), desc(ids), desc(out), desc(bad_ids), _stream(feats))
+    _lib.call("lux3d_index_select_rows", _d(feats), _d(ids), _d(out), _d(bad_ids), _stream(feats))
     return out
 
 
@@ -651,7 +673,7 @@ def channel_to_spatial(coords: torch.Tensor, feats: torch.Tensor, subdiv_logits:
     of = torch.empty((8 * n, c // 8), dtype=feats.dtype, device=dev)
     sub = torch.empty((n, 8), dtype=torch.float32, device=dev)
     cnt = torch.empty(1, dtype=torch.int32, device=dev)
-    _lib.call("lux3d_channel_to_spatial", desc(coords), desc(feats), desc(subdiv_logits), desc(ws), desc(oc),
-              desc(src), desc(of), desc(sub), desc(cnt), _stream(feats))
+    _lib.call("lux3d_channel_to_spatial", _d(coords), _d(feats), _d(subdiv_logits), _d(ws), _d(oc),
+              _d(src), _d(of), _d(sub), _d(cnt), _stream(feats))
     m = int(cnt.item())
     return oc[:m], of[:m], sub
