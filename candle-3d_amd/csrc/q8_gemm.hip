@@ -457,9 +457,12 @@ __global__ __launch_bounds__(64 * NW, 1) void q8_0_gemm_ring_kernel(Q8GemmParams
 // a ring kernel on v_mfma_f32_32x32x2_f32 (4096 x 2048 -> 8192: 994 -> 430
 // us, same-box A/B).
 //
-// 128 x 256 tiles, 8 wavefronts as 2 (rows) x 4 (columns), 64 x 64 each.
+// 128 x 256 tiles, 8 wavefronts as 2 (rows) x 4 (columns), 64 x 64 each; where
+// those would leave CUs idle, 64 x 128 or 32 x 128 tiles of 4 wavefronts, whose
+// KG groups take every KG th k-step into rings of their own and add their sums
+// in LDS at the end (a step's chain of MFMAs, not memory, bounds a lone tile).
 // 32-deep k-steps through a 4-stage LDS ring filled by direct global -> LDS
-// loads: x (128 rows x 128 bytes, row-major), the int8 weights (32 columns x
+// loads: x (BM rows x 128 bytes, row-major), the int8 weights (32 columns x
 // 32 bytes per 1 KB segment; lane l holds column l % 32, bytes 16 (l / 32)
 // .. + 15) and the scales (32 columns per wavefront, both lane halves). Each
 // step one cooperative pass splits the next stage's x into three bf16 planes
@@ -468,17 +471,25 @@ __global__ __launch_bounds__(64 * NW, 1) void q8_0_gemm_ring_kernel(Q8GemmParams
 // lane half h holds k = 16 h + 8 s + e on both operands. One barrier per
 // step: wait for stage kt + 1, barrier, issue stage kt + 3, split stage
 // kt + 1, compute stage kt.
-constexpr int kX3Stages = 4, kX3Threads = 512;
-constexpr int kX3XL = 128 * 128, kX3WB = 256 * 32, kX3SB = 8 * 256;
-constexpr int kX3Stage = kX3XL + kX3WB + kX3SB;  // 26,624 bytes
-constexpr int kX3Plane = 128 * 64;               // one bf16 plane of 128 rows x 32 k
-constexpr int kX3Ops = 4;                        // direct loads per wavefront per stage
+constexpr int kX3Stages = 4;
 
-template <typename OUT, int GM>
-__global__ __launch_bounds__(kX3Threads, 1) void q8_0_gemm_x3_kernel(Q8GemmParams p, int tiles_m, int tiles_n) {
-  constexpr int BM = 128, BN = 256, BK = 32, NS = kX3Stages;
-  __shared__ __align__(16) char lds[NS * kX3Stage + 2 * 3 * kX3Plane];
-  char *const planes = lds + NS * kX3Stage;
+// KG groups of WM x WN wavefronts, each wavefront TI x TJ tiles of 32 x 32.
+template <int WM, int WN, int TI, int TJ>
+struct X3Tile {
+  static constexpr int NW = WM * WN, BM = 32 * WM * TI, BN = 32 * WN * TJ;
+  static constexpr int SX = BM / 8 / NW, SW = BN / 32 / NW;  // 1 KB segments of x and of the weights a wavefront loads
+  static constexpr int XL = BM * 128, WB = BN * 32, SB = BN * 8, STAGE = XL + WB + SB;
+  static constexpr int PLANE = BM * 64;                      // one bf16 plane of BM rows x 32 k
+  static constexpr int OPS = SX + 2 * SW;                    // direct loads per wavefront per stage
+  static constexpr int LDS = kX3Stages * STAGE + 2 * 3 * PLANE;
+  static_assert(BM % (8 * NW) == 0 && BN % (32 * NW) == 0, "whole segments per wavefront");
+};
+
+template <typename OUT, int GM, int WM, int WN, int TI, int TJ, int KG>
+__global__ __launch_bounds__(64 * WM * WN * KG, 1) void q8_0_gemm_x3_kernel(Q8GemmParams p, int tiles_m, int tiles_n) {
+  using T = X3Tile<WM, WN, TI, TJ>;
+  constexpr int BM = T::BM, BN = T::BN, BK = 32, NS = kX3Stages;
+  __shared__ __align__(16) char lds_all[KG * T::LDS];
 
   const int G = tiles_m * tiles_n, bid = (int)blockIdx.x;
   const int per = G / 8, rem = G % 8, xcd = bid % 8, pos = bid / 8;
@@ -488,77 +499,88 @@ __global__ __launch_bounds__(kX3Threads, 1) void q8_0_gemm_x3_kernel(Q8GemmParam
   const int in_group = lid - group * GM * tiles_n;
   const int tm = first_m + in_group % gsize, tn = in_group / gsize;
 
-  const int t = threadIdx.x;
+  const int kg = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * T::NW)) : 0;
+  const int t = KG > 1 ? threadIdx.x - kg * 64 * T::NW : threadIdx.x;
   const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), h = lane >> 5, l32 = lane & 31;
-  const int wm = wave >> 2, wn = wave & 3;
+  const int wm = wave / WN, wn = wave % WN;
+  char *const lds = lds_all + kg * T::LDS, *const planes = lds + NS * T::STAGE;
   const int64_t m0 = (int64_t)tm * BM, c0 = (int64_t)tn * BN;
   const int64_t nblk = p.K / 32;
-  const int nk = (int)nblk;
+  const int nk = (int)nblk, nit = (nk + KG - 1) / KG;  // group kg takes steps kg, kg + KG, ...
 
   // direct-load offsets (rows and columns past the matrix clamp to the last)
-  uint32_t xoff[2];
+  uint32_t xoff[T::SX];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int r = 8 * (2 * wave + i) + (lane >> 3);
+  for (int i = 0; i < T::SX; ++i) {
+    const int r = 8 * (T::SX * wave + i) + (lane >> 3);
     const int64_t gr = m0 + r < p.M ? m0 + r : p.M - 1;
     xoff[i] = (uint32_t)(((gr - m0) * p.ldx + 4 * (lane & 7)) * 4);
   }
   const int64_t last_row = p.M - 1 - m0 < BM - 1 ? p.M - 1 - m0 : BM - 1;
   const int64_t ncols = p.N - c0 < BN ? p.N - c0 : BN;
-  const int64_t wcol = c0 + 32 * wave + l32, wc = wcol < p.N ? wcol : p.N - 1;
   const i32x4_t xr = buffer_rsrc(reinterpret_cast<const char *>(p.x) + m0 * p.ldx * 4, (last_row * p.ldx + p.K) * 4);
   const i32x4_t wr = buffer_rsrc(p.qs + c0 * p.K, ncols * p.K);
   const i32x4_t sr = buffer_rsrc(p.scales + c0 * nblk, ncols * nblk * 4);
-  const uint32_t woff = (uint32_t)((wc - c0) * p.K + 16 * h);
-  const uint32_t soff = (uint32_t)((wc - c0) * nblk * 4);
+  uint32_t woff[T::SW], soff[T::SW];
+#pragma unroll
+  for (int i = 0; i < T::SW; ++i) {
+    const int64_t col = c0 + 32 * (T::SW * wave + i) + l32, wc = col < p.N ? col : p.N - 1;
+    woff[i] = (uint32_t)((wc - c0) * p.K + 16 * h);
+    soff[i] = (uint32_t)((wc - c0) * nblk * 4);
+  }
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)lds;
-  auto issue = [&](int kt, int slot) {
-    const uint32_t st = lds0 + slot * kX3Stage;
+  auto issue = [&](int it, int slot) {
+    const int step = it * KG + kg, kt = step < nk ? step : nk - 1;
+    const uint32_t st = lds0 + slot * T::STAGE;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-      lds_load16(xr, xoff[i], (uint32_t)kt * BK * 4, __builtin_amdgcn_readfirstlane(st + (2 * wave + i) * 1024));
-    lds_load16(wr, woff, (uint32_t)kt * BK, __builtin_amdgcn_readfirstlane(st + kX3XL + wave * 1024));
-    lds_load4(sr, soff, (uint32_t)kt * 4, __builtin_amdgcn_readfirstlane(st + kX3XL + kX3WB + wave * 256));
+    for (int i = 0; i < T::SX; ++i)
+      lds_load16(xr, xoff[i], (uint32_t)kt * BK * 4, __builtin_amdgcn_readfirstlane(st + (T::SX * wave + i) * 1024));
+#pragma unroll
+    for (int i = 0; i < T::SW; ++i) {
+      const int seg = T::SW * wave + i;
+      lds_load16(wr, woff[i], (uint32_t)kt * BK, __builtin_amdgcn_readfirstlane(st + T::XL + seg * 1024));
+      lds_load4(sr, soff[i], (uint32_t)kt * 4, __builtin_amdgcn_readfirstlane(st + T::XL + T::WB + seg * 256));
+    }
   };
-  // the split pass: thread t takes 16-byte chunks t and t + 512 of the stage's
-  // x (row q / 8, k 4 (q % 8) .. + 3)
+  // the split pass: thread t of a group takes every 64 NW th 16-byte chunk of
+  // the stage's x from t (row q / 8, k 4 (q % 8) .. + 3)
   auto split = [&](int slot, int pb) {
-    const char *xs = lds + slot * kX3Stage;
-    char *pl = planes + pb * 3 * kX3Plane;
+    const char *xs = lds + slot * T::STAGE;
+    char *pl = planes + pb * 3 * T::PLANE;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int q = t + i * 512, r = q >> 3, c = q & 7;
+    for (int i = 0; i < BM * 8 / (64 * T::NW); ++i) {
+      const int q = t + i * 64 * T::NW, r = q >> 3, c = q & 7;
       const float4 v = *reinterpret_cast<const float4 *>(xs + q * 16);
       const Split3 lo = split3_bf16(v.x, v.y), hi = split3_bf16(v.z, v.w);
       const int off = r * 64 + (((c >> 1) ^ ((r >> 2) & 3)) << 4) + (c & 1) * 8;
       *reinterpret_cast<uint2 *>(pl + off) = make_uint2(lo.t1, hi.t1);
-      *reinterpret_cast<uint2 *>(pl + kX3Plane + off) = make_uint2(lo.t2, hi.t2);
-      *reinterpret_cast<uint2 *>(pl + 2 * kX3Plane + off) = make_uint2(lo.t3, hi.t3);
+      *reinterpret_cast<uint2 *>(pl + T::PLANE + off) = make_uint2(lo.t2, hi.t2);
+      *reinterpret_cast<uint2 *>(pl + 2 * T::PLANE + off) = make_uint2(lo.t3, hi.t3);
     }
   };
-  // fragment offsets: A rows wm * 64 + i * 32 + l32, chunk 2 h + s
-  int aoff[2][2];
+  // fragment offsets: A rows (wm TI + i) * 32 + l32, chunk 2 h + s
+  int aoff[TI][2];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int r = wm * 64 + i * 32 + l32;
+  for (int i = 0; i < TI; ++i) {
+    const int r = (wm * TI + i) * 32 + l32;
 #pragma unroll
     for (int s2 = 0; s2 < 2; ++s2) aoff[i][s2] = r * 64 + (((2 * h + s2) ^ ((r >> 2) & 3)) << 4);
   }
-  f32x16_t acc[2][2];
+  f32x16_t acc[TI][TJ];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < TI; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x16_t{};
+    for (int j = 0; j < TJ; ++j) acc[i][j] = f32x16_t{};
   auto compute = [&](int slot, int pb) {
-    const char *st = lds + slot * kX3Stage;
-    const char *pl = planes + pb * 3 * kX3Plane;
-    // weights of columns wn * 64 + j * 32 + l32: 16 int8 -> two bf16x8 (sub-steps)
-    bf16x8_t b[2][2];
-    float d[2];
+    const char *st = lds + slot * T::STAGE;
+    const char *pl = planes + pb * 3 * T::PLANE;
+    // weights of columns (wn TJ + j) * 32 + l32: 16 int8 -> two bf16x8 (sub-steps)
+    bf16x8_t b[TJ][2];
+    float d[TJ];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const uint4 w = *reinterpret_cast<const uint4 *>(st + kX3XL + (2 * wn + j) * 1024 + lane * 16);
-      d[j] = *reinterpret_cast<const float *>(st + kX3XL + kX3WB + (2 * wn + j) * 256 + l32 * 4);
+    for (int j = 0; j < TJ; ++j) {
+      const uint4 w = *reinterpret_cast<const uint4 *>(st + T::XL + (wn * TJ + j) * 1024 + lane * 16);
+      d[j] = *reinterpret_cast<const float *>(st + T::XL + T::WB + (wn * TJ + j) * 256 + l32 * 4);
       const uint32_t wv[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
       for (int s2 = 0; s2 < 2; ++s2) {
@@ -573,14 +595,14 @@ __global__ __launch_bounds__(kX3Threads, 1) void q8_0_gemm_x3_kernel(Q8GemmParam
       }
     }
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < TI; ++i) {
       bf16x8_t a[3][2];
 #pragma unroll
       for (int q = 0; q < 3; ++q)
 #pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) a[q][s2] = *reinterpret_cast<const bf16x8_t *>(pl + q * kX3Plane + aoff[i][s2]);
+        for (int s2 = 0; s2 < 2; ++s2) a[q][s2] = *reinterpret_cast<const bf16x8_t *>(pl + q * T::PLANE + aoff[i][s2]);
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int j = 0; j < TJ; ++j) {
         // block sum, smallest terms first, then scaled by the column's d
         f32x16_t blk = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2][0], b[j][0], f32x16_t{}, 0, 0, 0);
         blk = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2][1], b[j][1], blk, 0, 0, 0);
@@ -595,44 +617,74 @@ __global__ __launch_bounds__(kX3Threads, 1) void q8_0_gemm_x3_kernel(Q8GemmParam
   };
 
 #pragma unroll
-  for (int s2 = 0; s2 < NS - 1; ++s2) issue(s2 < nk ? s2 : nk - 1, s2);
-  __builtin_amdgcn_s_waitcnt(waitcnt_vm((NS - 2) * kX3Ops));
+  for (int s2 = 0; s2 < NS - 1; ++s2) issue(s2, s2);
+  __builtin_amdgcn_s_waitcnt(waitcnt_vm((NS - 2) * T::OPS));
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
   split(0, 0);
-  for (int kt = 0; kt < nk; ++kt) {
-    // stage kt + 1 landed (kt + 2 may be in flight); every wavefront is done
-    // with compute(kt - 1) and split(kt)
-    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(kX3Ops));
+  for (int it = 0; it < nit; ++it) {
+    // stage it + 1 landed (it + 2 may be in flight); every wavefront is done
+    // with compute(it - 1) and split(it)
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(T::OPS));
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    issue(kt + NS - 1 < nk ? kt + NS - 1 : nk - 1, (kt + NS - 1) % NS);
+    issue(it + NS - 1, (it + NS - 1) % NS);
     __builtin_amdgcn_sched_barrier(0);
-    if (kt + 1 < nk) split((kt + 1) % NS, (kt + 1) & 1);
-    compute(kt % NS, kt & 1);
+    if (it + 1 < nit) split((it + 1) % NS, (it + 1) & 1);
+    if (KG == 1 || it * KG + kg < nk) compute(it % NS, it & 1);
   }
   __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));
   __builtin_amdgcn_s_barrier();  // every wavefront is done with the ring and the planes
 
-  // epilogue: each wavefront's 64 x 64 block through LDS, bias added, one
+  if constexpr (KG > 1) {
+    // the groups' sums in group order, through LDS
+    constexpr int PART = TI * TJ * 16 * 64;
+    static_assert((KG - 1) * T::NW * PART * 4 <= KG * T::LDS, "partial sums fit");
+    float *const part = reinterpret_cast<float *>(lds_all) + wave * PART;
+    if (kg > 0) {
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; ++e)
+            part[(kg - 1) * T::NW * PART + ((i * TJ + j) * 16 + e) * 64 + lane] = acc[i][j][e];
+    }
+    __syncthreads();
+    if (kg == 0) {
+#pragma unroll
+      for (int g = 1; g < KG; ++g)
+#pragma unroll
+        for (int i = 0; i < TI; ++i)
+#pragma unroll
+          for (int j = 0; j < TJ; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+              acc[i][j][e] += part[(g - 1) * T::NW * PART + ((i * TJ + j) * 16 + e) * 64 + lane];
+    }
+    __syncthreads();
+    if (kg > 0) return;
+  }
+
+  // epilogue: each wavefront's 32 TI x 32 TJ block through LDS, bias added, one
   // rounding, 16-byte row pieces
   char *ybase = reinterpret_cast<char *>(p.y);
   constexpr int EB = OUT::code == LUX3D_F32 ? 4 : 2;
-  float bias[2];
+  float bias[TJ];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int64_t col = c0 + wn * 64 + j * 32 + l32;
+  for (int j = 0; j < TJ; ++j) {
+    const int64_t col = c0 + (wn * TJ + j) * 32 + l32;
     bias[j] = (p.bias && col < p.N) ? p.bias[col] : 0.f;
   }
   if (((uintptr_t)p.y % 16 == 0) && ((p.ldy * EB) % 16 == 0)) {
-    constexpr int ROW_B = 64 * EB, LROW = ROW_B + 16, CPR = ROW_B / 16, EPC = 16 / EB;
-    constexpr int REGION = 64 * LROW;
-    static_assert(8 * REGION <= (int)sizeof(lds), "epilogue staging fits");
+    constexpr int ROW_B = 32 * TJ * EB, LROW = ROW_B + 16, CPR = ROW_B / 16, EPC = 16 / EB;
+    constexpr int REGION = 32 * TI * LROW;
+    static_assert(T::NW * REGION <= T::LDS, "epilogue staging fits");
     char *reg = lds + wave * REGION;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < TI; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < TJ; ++j)
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
           const int r = i * 32 + 8 * (e >> 2) + 4 * h + (e & 3), cl = j * 32 + l32;
@@ -642,9 +694,9 @@ __global__ __launch_bounds__(kX3Threads, 1) void q8_0_gemm_x3_kernel(Q8GemmParam
             *reinterpret_cast<uint16_t *>(reg + r * LROW + cl * 2) = (uint16_t)(pack_bf16x2(v, 0.f) & 0xFFFFu);
           else *reinterpret_cast<uint16_t *>(reg + r * LROW + cl * 2) = (uint16_t)(pack_f16x2(v, 0.f) & 0xFFFFu);
         }
-    const int64_t r0 = m0 + wm * 64, cw = c0 + wn * 64;
+    const int64_t r0 = m0 + wm * TI * 32, cw = c0 + wn * TJ * 32;
 #pragma unroll
-    for (int it = 0; it < 64 * CPR / 64; ++it) {
+    for (int it = 0; it < 32 * TI * CPR / 64; ++it) {
       const int q = it * 64 + lane, r = q / CPR, part = q % CPR;
       const int64_t row = r0 + r, col = cw + part * EPC;
       if (row >= p.M || col >= p.N) continue;
@@ -666,14 +718,14 @@ __global__ __launch_bounds__(kX3Threads, 1) void q8_0_gemm_x3_kernel(Q8GemmParam
   }
   // y rows not 16-byte aligned: one element per store
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int64_t col = c0 + wn * 64 + j * 32 + l32;
+  for (int j = 0; j < TJ; ++j) {
+    const int64_t col = c0 + (wn * TJ + j) * 32 + l32;
     if (col >= p.N) continue;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < TI; ++i)
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const int64_t row = m0 + wm * 64 + i * 32 + 8 * (e >> 2) + 4 * h + (e & 3);
+        const int64_t row = m0 + (wm * TI + i) * 32 + 8 * (e >> 2) + 4 * h + (e & 3);
         if (row >= p.M) continue;
         store1<OUT>(ybase, row * p.ldy + col, acc[i][j][e] + bias[j]);
       }
@@ -818,6 +870,51 @@ hipError_t launch_few_rows(const Q8GemmParams &p, hipStream_t s) {
   return hipGetLastError();
 }
 
+template <typename OUT, int WM, int WN, int TI, int TJ, int KG>
+hipError_t launch_x3(const Q8GemmParams &p, hipStream_t s) {
+  using T = X3Tile<WM, WN, TI, TJ>;
+  const int64_t tiles_m = (p.M + T::BM - 1) / T::BM, tiles_n = (p.N + T::BN - 1) / T::BN;
+  if (tiles_m * tiles_n > 0x7FFFFFFF) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((q8_0_gemm_x3_kernel<OUT, 8, WM, WN, TI, TJ, KG>), dim3((unsigned)(tiles_m * tiles_n)),
+                     dim3(64 * T::NW * KG), 0, s, p, (int)tiles_m, (int)tiles_n);
+  return hipGetLastError();
+}
+
+// f32 activations: the kernel and tile that take the shortest time by these
+// measured costs, linear in the 32-deep steps of k (ns; one round = every CU
+// busy once, alone or, for the 64 x 128 tiles, with two workgroups):
+//   few rows      64 x 16     262 steps + 2000 a round
+//   1 x 4, KG 3   32 x 128    345 steps + 3500 a round
+//   2 x 2, KG 2   64 x 128    570 steps + 4500 a round
+//   2 x 2         64 x 128   1050 steps + 4000 for two a CU, 760 steps + 4000 for one
+//   2 x 4        128 x 256   1500 steps + 5000 a round
+// With 128 x 256 tiles alone a product of 1029 rows left most CUs idle or took
+// a second round for a few tiles: 1029 x 4096 -> 1024 154 -> 76 us, 1029 x 1536
+// -> 1536 76 -> 34, 512 x 8192 -> 2048 268 -> 91, 2049 x 1024 -> 4096 109 -> 91,
+// 256 x 1024 -> 4096 36.7 -> 16.1.
+template <typename OUT>
+hipError_t launch_f32(const Q8GemmParams &p, hipStream_t s) {
+  if (p.M <= 16) return launch_few_rows<OUT, true, 1>(p, s);
+  auto tiles = [&](int64_t bm, int64_t bn) { return (double)((p.M + bm - 1) / bm) * (double)((p.N + bn - 1) / bn); };
+  auto rounds = [](double t) { return __builtin_ceil(t / 256); };
+  const double steps = (double)(p.K / 32), mid = tiles(64, 128);
+  const double few = p.M > 65535 * 64 ? __builtin_inf() : rounds(tiles(64, 16)) * (262 * steps + 2000);  // its grid
+  const double k3 = rounds(tiles(32, 128)) * (345 * steps + 3500);
+  const double k2 = rounds(mid) * (570 * steps + 4500);
+  // two a CU; the tiles past the last full round run as on half-empty CUs
+  const double pair = 1050 * steps + 4000, one = 760 * steps + 4000, full = __builtin_floor(mid / 512);
+  const double k1 = mid <= 256 ? one
+                    : mid <= 512 ? pair
+                    : mid / 512 * pair + (mid > full * 512 ? (full < 2 ? 0.75 : 0.5) * one : 0);
+  const double large = rounds(tiles(128, 256)) * (1500 * steps + 5000);
+  const double best = __builtin_fmin(__builtin_fmin(__builtin_fmin(few, k3), __builtin_fmin(k2, k1)), large);
+  if (best == large) return launch_x3<OUT, 2, 4, 2, 2, 1>(p, s);
+  if (best == k1) return launch_x3<OUT, 2, 2, 1, 2, 1>(p, s);
+  if (best == k2) return launch_x3<OUT, 2, 2, 1, 2, 2>(p, s);
+  if (best == k3) return launch_x3<OUT, 1, 4, 1, 1, 3>(p, s);
+  return launch_few_rows<OUT, true, 4>(p, s);
+}
+
 // The ring kernel's buffer descriptors span one tile (at most 256 rows of x,
 // 256 weight rows and their scales) and must stay below 2^31 bytes; its
 // per-lane offsets are 32-bit.
@@ -840,25 +937,15 @@ constexpr int64_t kRingMinTiles = 256;  // MI355X compute units
 
 template <typename OUT>
 hipError_t launch_tiles(const Q8GemmParams &p, hipStream_t s) {
+  // f32 activations (K % 64 == 0, checked by the caller)
+  if (p.x_f32) return launch_f32<OUT>(p, s);
   // Few rows: always up to 16; beyond, while the grid of 64 x 16 tiles is below
-  // the line where the 128-row tiles' serial k loop takes as long (bf16 512
-  // tiles: K 1024, N 4096 at 64 / 128 / 200 rows 7.0 / 11.6 / 18.1 us against
-  // 12.0 / 12.3 / 12.5; K 8192, N 2048 at 128 / 200 37.8 / 72.7 against 70.9 /
-  // 70.1; f32 1280 tiles: K 1536, N 9216 at 128 / 200 64.2 / 100.5 against 74.9
-  // / 75.1; K 8192, N 2048 at 512 270 against 366).
+  // the line where the 128-row tiles' serial k loop takes as long (512 tiles: K
+  // 1024, N 4096 at 64 / 128 / 200 rows 7.0 / 11.6 / 18.1 us against 12.0 / 12.3
+  // / 12.5; K 8192, N 2048 at 128 / 200 37.8 / 72.7 against 70.9 / 70.1).
   if (p.K % 64 == 0) {
-    const int64_t tiles64 = (p.M + 63) / 64 * ((p.N + 15) / 16);
-    if (p.M <= 16) return p.x_f32 ? launch_few_rows<OUT, true, 1>(p, s) : launch_few_rows<OUT, false, 1>(p, s);
-    if (p.x_f32 && tiles64 <= 1280) return launch_few_rows<OUT, true, 4>(p, s);
-    if (!p.x_f32 && tiles64 < 512) return launch_few_rows<OUT, false, 4>(p, s);
-  }
-  if (p.x_f32) {
-    // f32 activations (K % 64 == 0, checked by the caller)
-    const int64_t tiles_m = (p.M + 127) / 128, tiles_n = (p.N + 255) / 256;
-    if (tiles_m * tiles_n > 0x7FFFFFFF) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((q8_0_gemm_x3_kernel<OUT, 8>), dim3((unsigned)(tiles_m * tiles_n)), dim3(kX3Threads), 0, s, p,
-                       (int)tiles_m, (int)tiles_n);
-    return hipGetLastError();
+    if (p.M <= 16) return launch_few_rows<OUT, false, 1>(p, s);
+    if ((p.M + 63) / 64 * ((p.N + 15) / 16) < 512) return launch_few_rows<OUT, false, 4>(p, s);
   }
   if (ring_fits(p)) {
     const int64_t tiles_n = (p.N + 255) / 256, tiles_m256 = (p.M + 255) / 256;
