@@ -17,7 +17,8 @@
 // - q8_0_few_rows_kernel (K % 64 == 0, up to 16 rows or few tiles): workgroups of
 //   16 weight rows whose wavefronts split k.
 // - q8_0_gemm_ring_kernel (K % 64 == 0, the common case): a workgroup of NW
-//   wavefronts (8, or 4 for small shapes) computes a BM x 32 NW tile; x, the
+//   wavefronts (8, or 4 for small shapes) computes a BM x 32 NW tile (BM 32 to
+//   256); x, the
 //   int8 weights and the scales stream through a 3-stage LDS ring by direct
 //   global->LDS loads; each wavefront dequantises its own 32 weight columns
 //   once per k-step.
@@ -199,9 +200,9 @@ __global__ __launch_bounds__(kGemmThreads, MINW) void q8_0_gemm_kernel(Q8GemmPar
 
 // ---- GEMM through an LDS ring fed by direct loads ---------------------------
 //
-// One 512-thread workgroup per CU computes a BM x 256 tile of y (BM = 256,
-// or 128 for problems too small to give every CU a 256-row tile). Its eight
-// wavefronts each own 32 columns and all BM rows (BM / 32 MFMA tiles of
+// A workgroup of NW wavefronts computes a BM x 32 NW tile of y (256 x 256 where
+// the problem fills the chip with them, down to 32 x 128). Its wavefronts each
+// own 32 columns and all BM rows (BM / 32 MFMA tiles of
 // 32 x 32), so every weight element is dequantised by exactly one wavefront
 // and amortised over BM rows of x.
 //
@@ -924,56 +925,66 @@ bool ring_fits(const Q8GemmParams &p) {
          (p.M + 127) / 128 * ((p.N + 255) / 256) <= INT32_MAX;
 }
 
-// Kernel choice (measured on MI355X, graph-timed over rotating inputs):
-// the ring kernel whenever K % 64 == 0 (every shape of the models): 256-row
-// tiles when they cover every CU at least once (1,018 TFLOP/s at
-// 4096x2048x8192, 512 tiles), else 128-row tiles of 8 wavefronts when those
-// do, else tiles of 4 wavefronts: 160 x 128 when 128 x 128 ones would
-// outnumber the CUs but 160-row ones do not (1029x1024x4096: 7 x 32 tiles in
-// 19.2 us, against 23.5 us for 9 x 32 of 128 x 128, 26.8 us for 9 x 16 tiles
-// of 8 wavefronts, 22.4 us for 5 x 32 of 256 x 128), else 128 x 128. The
-// 128 x 128 kernel with 32-deep k-steps covers K % 64 == 32.
-constexpr int64_t kRingMinTiles = 256;  // MI355X compute units
+template <typename OUT, int BM, int NW>
+hipError_t launch_ring(const Q8GemmParams &p, hipStream_t s) {
+  const int64_t tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N + 32 * NW - 1) / (32 * NW);
+  if (tiles_m * tiles_n > INT32_MAX) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((q8_0_gemm_ring_kernel<OUT, 8, BM, NW>), dim3((unsigned)(tiles_m * tiles_n)), dim3(64 * NW), 0, s,
+                     p, (int)tiles_m, (int)tiles_n);
+  return hipGetLastError();
+}
+
+// bf16 activations: the kernel and tile that take the shortest time by these
+// measured costs, linear in the 64-deep steps of k (ns; a round is 256 tiles,
+// one for each CU, whether a CU holds one workgroup or several):
+//   few rows   64 x 16    280 steps + 2000 a round
+//   ring       32 x 128   410 steps a round + 2500
+//              64 x 128   450 steps + 1000 a round + 3000
+//             128 x 128   530 steps + 4000 for one round, else 610 steps + 2000 a round
+//             160 x 128   660 steps + 5000 a round
+//             128 x 256  1150 steps + 2000 a round
+//             256 x 256  1600 steps + 3000 a round
+// A lone small tile is bound by the latency of its serial k loop, and a 256 x
+// 256 tile reads each operand least. One rule for all sizes instead of the
+// first tile that covered every CU, us: 1029 x 1536 -> 9216 59 -> 46, 1536 x
+// 2048 -> 8192 75 -> 59, 512 x 8192 -> 2048 70 -> 56, 512 x 1536 -> 1536 17 ->
+// 13, 3000 x 1024 -> 3072 41 -> 31. Groups of wavefronts that share k gain
+// nothing here (512 x 8192 -> 2048: 61 us with four groups of 32 x 128): a
+// workgroup of any tile already takes what one CU loads.
+template <typename OUT>
+hipError_t launch_bf16(const Q8GemmParams &p, hipStream_t s) {
+  if (p.M <= 16) return launch_few_rows<OUT, false, 1>(p, s);
+  const double steps = (double)(p.K / 64);
+  auto rounds = [&](int64_t bm, int64_t bn) {
+    return __builtin_ceil((double)((p.M + bm - 1) / bm) * (double)((p.N + bn - 1) / bn) / 256);
+  };
+  const double r128 = rounds(128, 128);
+  const double cost[7] = {p.M > 65535 * 64 ? __builtin_inf() : rounds(64, 16) * (280 * steps + 2000),  // its grid
+                          rounds(32, 128) * 410 * steps + 2500,
+                          rounds(64, 128) * (450 * steps + 1000) + 3000,
+                          r128 == 1 ? 530 * steps + 4000 : r128 * (610 * steps + 2000),
+                          rounds(160, 128) * (660 * steps + 5000),
+                          rounds(128, 256) * (1150 * steps + 2000),
+                          rounds(256, 256) * (1600 * steps + 3000)};
+  int best = 6;  // the larger tile of two equal ones
+  for (int i = 5; i >= 0; --i)
+    if (cost[i] < cost[best]) best = i;
+  switch (best) {
+    case 0: return launch_few_rows<OUT, false, 4>(p, s);
+    case 1: return launch_ring<OUT, 32, 4>(p, s);
+    case 2: return launch_ring<OUT, 64, 4>(p, s);
+    case 3: return launch_ring<OUT, 128, 4>(p, s);
+    case 4: return launch_ring<OUT, 160, 4>(p, s);
+    case 5: return launch_ring<OUT, 128, 8>(p, s);
+  }
+  return launch_ring<OUT, 256, 8>(p, s);
+}
 
 template <typename OUT>
 hipError_t launch_tiles(const Q8GemmParams &p, hipStream_t s) {
-  // f32 activations (K % 64 == 0, checked by the caller)
-  if (p.x_f32) return launch_f32<OUT>(p, s);
-  // Few rows: always up to 16; beyond, while the grid of 64 x 16 tiles is below
-  // the line where the 128-row tiles' serial k loop takes as long (512 tiles: K
-  // 1024, N 4096 at 64 / 128 / 200 rows 7.0 / 11.6 / 18.1 us against 12.0 / 12.3
-  // / 12.5; K 8192, N 2048 at 128 / 200 37.8 / 72.7 against 70.9 / 70.1).
-  if (p.K % 64 == 0) {
-    if (p.M <= 16) return launch_few_rows<OUT, false, 1>(p, s);
-    if ((p.M + 63) / 64 * ((p.N + 15) / 16) < 512) return launch_few_rows<OUT, false, 4>(p, s);
-  }
-  if (ring_fits(p)) {
-    const int64_t tiles_n = (p.N + 255) / 256, tiles_m256 = (p.M + 255) / 256;
-    if (tiles_m256 * tiles_n >= kRingMinTiles) {
-      hipLaunchKernelGGL((q8_0_gemm_ring_kernel<OUT, 8, 256>), dim3((unsigned)(tiles_m256 * tiles_n)), dim3(kRingThreads),
-                         0, s, p, (int)tiles_m256, (int)tiles_n);
-    } else if ((p.M + 127) / 128 * tiles_n >= kRingMinTiles) {
-      const int64_t tiles_m = (p.M + 127) / 128;
-      hipLaunchKernelGGL((q8_0_gemm_ring_kernel<OUT, 8, 128>), dim3((unsigned)(tiles_m * tiles_n)), dim3(kRingThreads), 0,
-                         s, p, (int)tiles_m, (int)tiles_n);
-    } else if ((p.M + 127) / 128 * ((p.N + 127) / 128) > kRingMinTiles &&
-               (p.M + 159) / 160 * ((p.N + 127) / 128) <= kRingMinTiles) {
-      // fewer 128 x 256 tiles than CUs, more 128 x 128 ones: 160 x 128 tiles
-      // of four wavefronts, one per CU (the 128-row tiles would leave some CUs
-      // two; 1029 x 1024 -> 4096: 7 x 32 tiles in 19.2 us against 9 x 32 in
-      // 23.5 us)
-      const int64_t tiles_m = (p.M + 159) / 160, tiles_n128 = (p.N + 127) / 128;
-      hipLaunchKernelGGL((q8_0_gemm_ring_kernel<OUT, 8, 160, 4>), dim3((unsigned)(tiles_m * tiles_n128)), dim3(256), 0,
-                         s, p, (int)tiles_m, (int)tiles_n128);
-    } else {
-      // fewer 128 x 256 tiles than CUs: 128 x 128 tiles of four wavefronts
-      // (two workgroups per CU by LDS) spread the same wavefronts over more CUs
-      const int64_t tiles_m = (p.M + 127) / 128, tiles_n128 = (p.N + 127) / 128;
-      hipLaunchKernelGGL((q8_0_gemm_ring_kernel<OUT, 8, 128, 4>), dim3((unsigned)(tiles_m * tiles_n128)), dim3(256), 0,
-                         s, p, (int)tiles_m, (int)tiles_n128);
-    }
-    return hipGetLastError();
-  }
+  if (p.x_f32) return launch_f32<OUT>(p, s);  // K % 64 == 0, checked by the caller
+  if (ring_fits(p)) return launch_bf16<OUT>(p, s);
+  // K % 64 == 32, or rows too far apart for the ring's offsets
   const dim3 grid((unsigned)((p.N + 127) / 128), (unsigned)((p.M + 127) / 128));
   hipLaunchKernelGGL((q8_0_gemm_kernel<OUT, 128, 128, 32, 1>), grid, dim3(kGemmThreads), 0, s, p);
   return hipGetLastError();
