@@ -599,11 +599,11 @@ def _sdpa(dev, name, cfg, b, n, h, d, what, reps=50, dt=torch.bfloat16, heads_f3
     nbytes = 4 * b * h * n * d * esz
     f32 = dt == torch.float32
     if f32:
-        kern, arith = f"attn_f32x3_kernel<{d}>", "f32 (bf16 matrix cores, three-term splits)"
+        kern, arith = f"attn_f32x3_{'pipe_' if d == 64 else ''}kernel<{d}>", "f32 (bf16 matrix cores, three-term splits)"
     elif heads_f32:
         kern, arith = f"attn_mfma_kernel<BF16,{d},...,EXACTP>", "bf16 in, f32 probabilities (3 bf16 terms), bf16 out"
     else:
-        kern, arith = f"attn_mfma_kernel<BF16,{d}>", "bf16 -> f32 acc"
+        kern, arith = f"attn_pipe_kernel<BF16,{d}>", "bf16 -> f32 acc"
     wl = Workload(name, cfg, kern, arith, nbytes,
                   f"q,k,v [{b},{h},{n},{d}] from qkv [{b},{n},3,{h},{d}] ({what})", launch, n_sets,
                   flops=4 * b * h * n * n * d, reps=reps,
@@ -651,7 +651,7 @@ def cfg1_sdpa_frame_qln(dev) -> Workload:
         dq, dk, dv, do = descs[i % n_sets]
         _lib.call("lux3d_sdpa_layernorm_rope2d", dq, dw, db, 1e-6, dc, dsn, dk, dv, 0.125, do, _cur())
     nbytes = 4 * b * h * n * d * 2
-    wl = Workload("sdpa_frame_qln", 1, "attn_mfma_kernel<BF16,64,...,QLN>", "bf16 -> f32 acc", nbytes,
+    wl = Workload("sdpa_frame_qln", 1, "attn_pipe_kernel<BF16,64,...,QLN>", "bf16 -> f32 acc", nbytes,
                   f"raw q + normalised k, v [{b},{h},{n},{d}]: q LayerNorm + 2D RoPE in the Q load", launch,
                   n_sets, flops=4 * b * h * n * n * d, reps=50)
     wl._keep = (qkvs, outs, qw, qb, emb, ks, descs, dw, db, dc, dsn)
@@ -737,7 +737,7 @@ def _sdpa_qprologue(dev, name, cfg, kind, b, n, h, d, dt, fused=True, reps=50) -
     f32 = dt == torch.float32
     what = {"rms": "RMSNorm", "l2r2": "L2 norm + 3D RoPE", "r3": "rotate_half RoPE"}[kind]
     how = "in the Q load" if fused else "head op, then attention (two launches)"
-    wl = Workload(name, cfg, f"attn_{'f32x3' if f32 else 'mfma'}_kernel<{d}, q prologue>",
+    wl = Workload(name, cfg, f"attn_{'f32x3_pipe' if f32 else 'mfma' if kind == 'r3' else 'pipe'}_kernel<{d}, q prologue>",
                   "f32 (three-term splits)" if f32 else "bf16 -> f32 acc", 4 * b * h * n * d * esz,
                   f"q, k, v [{b},{h},{n},{d}]: q {what} {how}", launch, n_sets,
                   flops=4 * b * h * n * n * d, reps=reps, peak_tflops=2500.0 / 6 if f32 else 0.0)
