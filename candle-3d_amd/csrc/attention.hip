@@ -110,6 +110,9 @@ __device__ __forceinline__ void split3_into(float a, float b, u32x4_t &x1, u32x4
 template <int D> __device__ __forceinline__ int k_swz(int r) { return D == 128 ? r & 15 : (r >> 1) & 7; }
 template <int D> __device__ __forceinline__ int v_swz(int r) { return D == 128 ? (r & 3) << 2 : (r & 2) << 1; }
 
+// Counts as a use of x at this place.
+__device__ __forceinline__ void keep(const f32x16_t &x) { asm volatile("" ::"v"(x)); }
+
 // The value the partner lane (lane ^ 32) holds, paired with this lane's own:
 // v_permlane32_swap exchanges the two 32-lane halves.
 __device__ __forceinline__ float half_swap_max(float v) {
@@ -726,27 +729,36 @@ __global__ __launch_bounds__(256, MINW) void attn_mfma_kernel(AttnParams p, int6
 
 // ---- pipelined form -------------------------------------------------------------
 //
-// The same arithmetic (LAZY, DOT) with the parts of a key block that depend on
-// each other taken from different blocks. Each of the 4 wavefronts keeps QT
-// tiles of 32 queries; the keys go by 32 per step, and step j is one straight
-// line of MFMAs with everything else in the gaps between them:
-//   scores of block j + 1 (its K fragments were read one step ahead), between
-//   them the exponentials of block j and the reads of V's fragments,
-//   O += P V of block j, between them the last exponentials, the maximum of
-//   block j + 1 and the reads of the K fragments after it.
-// An MFMA takes 32 cycles and up to about 24 cycles of VALU work issue beside
-// it for free (4 FMAs and an exponential per MFMA: 34.8 against 32.5 cycles,
-// one wavefront per SIMD). The order is fenced instruction by instruction:
-// left alone, the scheduler gathers the MFMAs. D 128 (QT 1, two workgroups per
-// CU) is then bound by the matrix cores, about 66% busy, at the clock that
-// this load leaves (about 1.8 GHz); D 64 by the VALU: 32 scores per lane and
-// tile pair are 0.7 us of FMAs, exponentials, packs and sums against 0.5 us of
-// MFMAs per 1000 steps. Before / after, us: TRELLIS.2 12 x 40000 x 128 9354 /
-// 8505, TripoSG 2 x 16 x 2048 x 128 74.5 / 68.1, VGGT 8 frames (D 64) 81.6 /
-// 76.0, 8 frames as one sequence 561 / 529.
+// attn_mfma_kernel's arithmetic (LAZY, DOT, 64-key blocks) in its order, so that
+// the two give the same bits: the reference maximum may move once in 64 keys
+// and the row sum of 64 keys is formed before it joins the running one (one
+// chain over all keys has 16 times the rounding steps at 40,000 keys). The
+// parts that depend on each other are taken from different blocks. Each of the
+// 4 wavefronts keeps QT tiles of 32 queries; the keys go by 32 per step, two
+// steps to a pair, and step j is one straight line of MFMAs with everything
+// else in the gaps between them:
+//   scores of block j + 2 but for their last 16 dims (its K fragments were read
+//   one step ahead), between them the exponentials of block j and the reads of
+//   V's fragments,
+//   half of O += P V of block j, between them the last exponentials,
+//   the last 16 dims of the scores, into the registers that block j's scores
+//   leave: the two tiles of a pair and a third for the sums under way stay
+//   where they are, without copies,
+//   the rest of O += P V, between them the maximum, over both blocks of a pair,
+//   and the reads of the K fragments of block j + 3.
+// The order is fenced instruction by instruction: left alone, the scheduler
+// gathers the MFMAs. A pair takes 32 MFMAs of 32 cycles for 173 VALU
+// instructions at D 128 (QT 1, two workgroups per CU), for 296 at D 64 and QT
+// 2, 16 for 151 at QT 1: D 64 is bound by the VALU (an exponential takes as
+// long as four FMAs), D 128 by the matrix cores and the clock that their load
+// leaves. Against attn_mfma_kernel, us: TRELLIS.2 12 x 40000 x 128 9560 / 8736,
+// TripoSG 2 x 16 x 2048 x 128 75.3 / 71.2, VGGT 8 frames (D 64) 83.0 / 81.1, 8
+// frames as one sequence 553 / 546. (A maximum for every 32 keys needs two
+// tiles of scores instead of three and was 1 to 2% faster, but rounds other
+// probabilities.)
 //
 // K and V arrive by direct global -> LDS loads in two stages of 64 keys; stage
-// g holds V's blocks 2 g, 2 g + 1 and K's blocks 2 g + 2, 2 g + 3, as steps 2
+// g holds V's blocks 2 g, 2 g + 1 and K's blocks 2 g + 3, 2 g + 4, as steps 2
 // g and 2 g + 1 read them (what lies past Lk reads as zeros). One barrier per
 // stage; its successor's loads are issued behind it.
 template <typename T, int D, int QT, int MINW, int QP>
@@ -776,60 +788,63 @@ __global__ __launch_bounds__(256, MINW) void attn_pipe_kernel(AttnParams p, int6
   if constexpr (QP != QP_NONE) lds_barrier();
 
   const int nkv = (int)((Lk + BK - 1) / BK);
-  uint32_t dk_off[SEGW], dv_off[SEGW];
-#pragma unroll
-  for (int i = 0; i < SEGW; ++i) {
-    const int byte = (wave * SEGW + i) * 1024 + lane * 16, r = byte / (2 * D), sl = (byte % (2 * D)) / 16;
-    dk_off[i] = (uint32_t)(r * p.k_st * 2 + (sl ^ k_swz<D>(r)) * 16);
-    dv_off[i] = (uint32_t)(r * p.v_st * 2 + (sl ^ v_swz<D>(r)) * 16);
-  }
-  // the next two blocks of K and of V: their first byte, and the bytes from there to the head's last (none: all
-  // loads read zeros)
-  const char *knext = kbase, *vnext = vbase;
-  int64_t kleft = ((Lk - 1) * p.k_st + D) * 2, vleft = ((Lk - 1) * p.v_st + D) * 2;
-  const int64_t kstep = 2 * BK * p.k_st * 2, vstep = 2 * BK * p.v_st * 2;
+  // Load i of a wavefront fills 1 KB of two blocks, rows r0 + RS i: r0's bits
+  // below RS and the swizzle's bits from RS on do not overlap, so that the
+  // offsets of all loads follow from the first one's.
+  constexpr int RS = 512 / D;
+  const int r0 = wave * SEGW * RS + lane / (D / 8), sl = lane % (D / 8);
+  uint32_t krow = (uint32_t)(r0 * p.k_st * 2), kch = (uint32_t)((sl ^ k_swz<D>(r0)) * 16);
+  uint32_t vrow = (uint32_t)(r0 * p.v_st * 2 + (sl ^ v_swz<D>(r0)) * 16);
+  // two blocks of K or V from byte `from` of a head of `bytes` bytes on (what lies past the head reads as zeros)
+  const int64_t kbytes = ((Lk - 1) * p.k_st + D) * 2, vbytes = ((Lk - 1) * p.v_st + D) * 2;
+  const int64_t kblock = BK * p.k_st * 2, vblock = BK * p.v_st * 2;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)ring;
-  auto dma = [&](const char *&base, int64_t &left, int64_t step, const uint32_t (&off)[SEGW], uint32_t lds) {
-    const i32x4_t rs = buffer_rsrc(base, left > 0 ? left : 0);
+  auto load_k = [&](int64_t from, uint32_t lds) {
+    const i32x4_t rs = buffer_rsrc(kbase + from, kbytes > from ? kbytes - from : 0);
+    asm volatile("" : "+v"(krow), "+v"(kch));
 #pragma unroll
     for (int i = 0; i < SEGW; ++i)
-      lds_load16(rs, off[i], 0, __builtin_amdgcn_readfirstlane(lds + (wave * SEGW + i) * 1024));
-    base += step;
-    left -= step;
+      lds_load16(rs, krow + (uint32_t)(i * RS * p.k_st * 2) + (kch ^ (k_swz<D>(i * RS) * 16)), 0,
+                 __builtin_amdgcn_readfirstlane(lds + (wave * SEGW + i) * 1024));
   };
-  auto load_k = [&](int slot) { dma(knext, kleft, kstep, dk_off, lds0 + slot * STAGE + 2 * KB); };
-  auto load_stage = [&](int slot) {
-    dma(vnext, vleft, vstep, dv_off, lds0 + slot * STAGE);
-    load_k(slot);
-  };
-  // K fragment c of a block: rows l32, 16-byte chunk 2 c + hh
-  int kfo[NC];
+  auto load_v = [&](int64_t from, uint32_t lds) {
+    const i32x4_t rs = buffer_rsrc(vbase + from, vbytes > from ? vbytes - from : 0);
+    asm volatile("" : "+v"(vrow));
 #pragma unroll
-  for (int c = 0; c < NC; ++c) kfo[c] = 2 * KB + l32 * 2 * D + (((2 * c + hh) ^ k_swz<D>(l32)) << 4);
-  // at: byte offset of the block in its stage's half, slot * STAGE + (block & 1) * KB
-  auto kfrag = [&](int at, int c) { return *reinterpret_cast<const op_t *>(ring + at + kfo[c]); };
-  // V^T fragment (dim tile dt, keys 16 jj ..), half h (keys + 8 h): see attn_mfma_kernel
+    for (int i = 0; i < SEGW; ++i)
+      lds_load16(rs, vrow + (uint32_t)(i * RS * p.v_st * 2), 0,
+                 __builtin_amdgcn_readfirstlane(lds + (wave * SEGW + i) * 1024));
+  };
+  int64_t kfrom = 3 * kblock, vfrom = 0;
+  int slot = 0;
+  auto load_stage = [&](int to) {
+    load_v(vfrom, lds0 + to * STAGE);
+    load_k(kfrom, lds0 + to * STAGE + 2 * KB);
+    vfrom += 2 * vblock;
+    kfrom += 2 * kblock;
+  };
+  // K fragment c of a block: row l32, 16-byte chunk 2 c + hh; kfo and vfo hold the stage's slot, at is the block's
+  // byte offset in its half of the stage
+  int kfo = 2 * KB + l32 * 2 * D + ((hh ^ k_swz<D>(l32)) << 4);
+  auto kfrag = [&](int at, int c) { return *reinterpret_cast<const op_t *>(ring + at + (kfo ^ (c << 5))); };
+  // V^T fragment (dim tile dt, keys 16 jj ..), half h (keys + 8 h): see attn_mfma_kernel. Rows 16 jj + 8 h more keep
+  // the swizzle's row bits.
   typedef short s16x4_t __attribute__((ext_vector_type(4)));
   typedef __attribute__((address_space(3))) s16x4_t lds_s16x4_t;
   const int vr0 = 4 * hh + ((lane & 15) >> 2), vc0 = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-  int vfo[NDT];  // rows 16 jj + 8 h more keep the swizzle's row bits
-#pragma unroll
-  for (int dt = 0; dt < NDT; ++dt) {
-    const int col = dt * 32 + vc0;
-    vfo[dt] = vr0 * 2 * D + (((col >> 3) ^ v_swz<D>(vr0)) << 4) + (col & 7) * 2;
-  }
+  int vfo = vr0 * 2 * D + (((vc0 >> 3) ^ v_swz<D>(vr0)) << 4) + (vc0 & 7) * 2;
   auto vhalf = [&](int at, int dt, int jj, int h) {
     return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-        (lds_s16x4_t *)(ring + at + vfo[dt] + (16 * jj + 8 * h) * 2 * D));
+        (lds_s16x4_t *)(ring + at + (vfo ^ (dt << 6)) + (16 * jj + 8 * h) * 2 * D));
   };
 
   f32x16_t o[QT][NDT], sa[QT], sb[QT];
-  float m[QT], l[QT], alpha[QT];
+  float m[QT], l[QT], ls[QT], alpha[QT];
   op_t kf[NC], pf[QT][2];
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
     m[qt] = -INFINITY;
-    l[qt] = 0.f;
+    l[qt] = ls[qt] = 0.f;
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt) o[qt][dt] = f32x16_t{};
   }
@@ -845,10 +860,11 @@ __global__ __launch_bounds__(256, MINW) void attn_pipe_kernel(AttnParams p, int6
         for (int qt = 0; qt < QT; ++qt) s[qt][i] = -INFINITY;
       }
   };
-  // the maximum of tile qt in 8 steps, and the reference maximum it leads to
+  // the maximum of tile qt over the two blocks of a pair, 8 steps each, and the reference maximum it leads to
   float mx[QT];
-  auto max_step = [&](const f32x16_t (&s)[QT], int qt, int i) {
-    mx[qt] = i == 0 ? fmaxf(s[qt][0], s[qt][1]) : fmaxf(fmaxf(mx[qt], s[qt][2 * i]), s[qt][2 * i + 1]);
+  auto max_step = [&](const f32x16_t (&s)[QT], int qt, int i, bool first) {
+    if (first && i == 0) mx[qt] = fmaxf(s[qt][0], s[qt][1]);
+    else mx[qt] = fmaxf(fmaxf(mx[qt], s[qt][2 * i]), s[qt][2 * i + 1]);
   };
   auto max_done = [&](int qt) {
     const float cand = half_swap_max(mx[qt]) * c2;
@@ -857,54 +873,74 @@ __global__ __launch_bounds__(256, MINW) void attn_pipe_kernel(AttnParams p, int6
     alpha[qt] = __builtin_amdgcn_exp2f(m[qt] - mn);
     m[qt] = mn;
   };
+  // the pair's row sum joins the running one
+  auto sum_pair = [&](int qt) { l[qt] = __builtin_fmaf(l[qt], alpha[qt], ls[qt]); };
 
-  // prologue: K's blocks 0 and 1 into the slot of stage 1, stage 0, scores of block 0
-  load_k(1);
+  // prologue: K's blocks 0, 1 and 2, 3 into the slot of stage 1, stage 0; the
+  // scores of the first pair and its maximum
+  load_k(0, lds0 + STAGE + 2 * KB);
+  load_k(2 * kblock, lds0 + STAGE);
   load_stage(0);
   __builtin_amdgcn_s_waitcnt(waitcnt_vm(2 * SEGW));
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
+  auto scores = [&](f32x16_t (&s)[QT]) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) s[qt] = M::run(kf[c], qf[qt][c], c == 0 ? f32x16_t{} : s[qt]);
+  };
 #pragma unroll
   for (int c = 0; c < NC; ++c) kf[c] = kfrag(STAGE, c);
-#pragma unroll
-  for (int c = 0; c < NC; ++c)
-#pragma unroll
-    for (int qt = 0; qt < QT; ++qt) sa[qt] = M::run(kf[c], qf[qt][c], c == 0 ? f32x16_t{} : sa[qt]);
+  scores(sa);
 #pragma unroll
   for (int c = 0; c < NC; ++c) kf[c] = kfrag(STAGE + KB, c);
-  if (nkv == 1) mask(0, sa);
+  scores(sb);
+#pragma unroll
+  for (int c = 0; c < NC; ++c) kf[c] = kfrag(STAGE - 2 * KB, c);
+  if (nkv <= 2) {
+    mask(0, sa);
+    mask(1, sb);
+  }
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) max_step(sa, qt, i);
+    for (int i = 0; i < 8; ++i) max_step(sa, qt, i, true);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) max_step(sb, qt, i, false);
     max_done(qt);
   }
 
-  // One step. NEXT: there is a block j + 1; MASKED: it is the last one.
-  auto step = [&](int j, f32x16_t (&s)[QT], f32x16_t (&sn)[QT], auto next_c, auto masked_c) {
+  // One step on block j, of parity PAR, whose scores are in s. NEXT: there is a next pair, and the scores of block
+  // j + 2 replace them; MASKED: it may hold the last block.
+  auto step = [&](int j, f32x16_t (&s)[QT], auto par_c, auto next_c, auto masked_c) {
+    constexpr int PAR = decltype(par_c)::value;
     constexpr bool NEXT = decltype(next_c)::value, MASKED = decltype(masked_c)::value;
-    constexpr int NA = NEXT ? QT * NC : 0, NB = QT * 2 * NDT, NM = NA + NB;  // MFMAs: scores, P v
-    const int at = (j >> 1 & 1) * STAGE + (j & 1) * KB;
-    if ((j & 1) == 0) {
+    // MFMAs: the scores but for their last chunk, one half of P v, the scores' last chunk, the other half
+    constexpr int NA = NEXT ? QT * (NC - 1) : 0, NL = NEXT ? QT : 0, NB = QT * 2 * NDT, NM = NA + NB + NL;
+    constexpr int LAST = NA + NB / 2;  // the scores' last chunk
+    constexpr int at = PAR * KB;
+    if constexpr (PAR == 0) {
       // the stage landed, and every wavefront is done with the one before
       __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));
       __builtin_amdgcn_s_barrier();
       __builtin_amdgcn_sched_barrier(0);
-      load_stage((j >> 1 & 1) ^ 1);
-    }
-    bool any = false;
+      load_stage(slot ^ 1);
+      bool any = false;
 #pragma unroll
-    for (int qt = 0; qt < QT; ++qt) any = any || alpha[qt] != 1.f;
-    if (__builtin_amdgcn_ballot_w64(any)) {
+      for (int qt = 0; qt < QT; ++qt) any = any || alpha[qt] != 1.f;
+      if (__builtin_amdgcn_ballot_w64(any)) {
 #pragma unroll
-      for (int qt = 0; qt < QT; ++qt) {
-        l[qt] *= alpha[qt];
+        for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
-        for (int dt = 0; dt < NDT; ++dt) o[qt][dt] *= alpha[qt];
+          for (int dt = 0; dt < NDT; ++dt) o[qt][dt] *= alpha[qt];
       }
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) ls[qt] = 0.f;
     }
     __builtin_amdgcn_sched_barrier(0);
     s16x4_t vh[NDT][2][2];
+    f32x16_t sn[QT];
     // exponentials, two pairs of scores at a time: 4 FMAs, 4 exponentials, 2 packs, 2 sums
     auto exp_op = [&](int n) {
       const int g = n / 12, r = n % 12, qt = g / 4, e0 = 4 * (g % 4);
@@ -916,14 +952,13 @@ __global__ __launch_bounds__(256, MINW) void attn_pipe_kernel(AttnParams p, int6
         const int h = r & 1, pe = e0 / 2 + h;  // packed pair pe of the tile: element pe % 4 of fragment pe / 4
         u32x4_t pk = __builtin_bit_cast(u32x4_t, pf[qt][pe / 4]);
         if (r < 10) pk[pe % 4] = M::pack(s[qt][e0 + 2 * h], s[qt][e0 + 2 * h + 1]);
-        else l[qt] = M::sum2(pk[pe % 4], l[qt]);
+        else ls[qt] = M::sum2(pk[pe % 4], ls[qt]);
         pf[qt][pe / 4] = __builtin_bit_cast(op_t, pk);
       }
     };
-    constexpr int NEXP = 48 * QT, NMAX = NEXT ? 9 * QT : 0;  // VALU items per tile: 4 groups of 12; 8 steps and the end
-    // items are spread over the MFMAs: all exponentials by the first P v MFMA of tile 1, tile 0's by the first of
-    // tile 0; without scores of a next block they come first
-    constexpr int EXP_END = NEXT ? NA + NB / 2 : 0;
+    // VALU items: 4 groups of 12 per tile; 8 steps of the maximum per tile and the pair's end. The exponentials
+    // are spread over the MFMAs up to LAST (without a next pair they come first), the maximum over those behind it.
+    constexpr int NEXP = 48 * QT, NMT = PAR == 1 ? 9 : 8, NMAX = NEXT ? NMT * QT : 0, REST = NB / 2;
     if constexpr (!NEXT) {
 #pragma unroll
       for (int dt = 0; dt < NDT; ++dt)
@@ -939,12 +974,17 @@ __global__ __launch_bounds__(256, MINW) void attn_pipe_kernel(AttnParams p, int6
       if (u < NA) {
         const int c = u / QT, qt = u % QT;
         sn[qt] = M::run(kf[c], qf[qt][c], c == 0 ? f32x16_t{} : sn[qt]);
-        // V's 4 NDT fragment halves, spread over the score MFMAs
-        constexpr int PER = 4 * NDT / (NA ? NA : 1);
+        // V's 4 NDT fragment halves, spread over these MFMAs
 #pragma unroll
-        for (int w = u * PER; w < (u + 1) * PER; ++w) vh[w / 4][w / 2 % 2][w % 2] = vhalf(at, w / 4, w / 2 % 2, w % 2);
+        for (int w = 0; w < 4 * NDT; ++w)
+          if (w >= u * 4 * NDT / (NA ? NA : 1) && w < (u + 1) * 4 * NDT / (NA ? NA : 1))
+            vh[w / 4][w / 2 % 2][w % 2] = vhalf(at, w / 4, w / 2 % 2, w % 2);
+      } else if (u >= LAST && u < LAST + NL) {
+        const int qt = u - LAST;
+        s[qt] = M::run(kf[NC - 1], qf[qt][NC - 1], sn[qt]);
+        keep(sn[qt]);  // the product goes to s's registers, not to sn's and a copy
       } else {
-        const int b = u - NA, qt = b / (2 * NDT), jj = b / NDT % 2, dt = b % NDT;
+        const int b = u < LAST ? u - NA : u - NA - NL, qt = b / (2 * NDT), jj = b / NDT % 2, dt = b % NDT;
         const op_t a = __builtin_bit_cast(op_t, __builtin_shufflevector(vh[dt][jj][0], vh[dt][jj][1], 0, 1, 2, 3, 4, 5, 6, 7));
         o[qt][dt] = M::run(a, pf[qt][jj], o[qt][dt]);
         if (NEXT && b % QT == 0 && b / QT < NC) kf[b / QT] = kfrag(at, b / QT);
@@ -952,39 +992,46 @@ __global__ __launch_bounds__(256, MINW) void attn_pipe_kernel(AttnParams p, int6
       if constexpr (NEXT) {
 #pragma unroll
         for (int n = 0; n < NEXP; ++n)
-          if (n >= u * NEXP / EXP_END && n < (u + 1) * NEXP / EXP_END) exp_op(n);
-        if (MASKED && u == EXP_END - 1) mask(j + 1, sn);
+          if (n >= u * NEXP / LAST && n < (u + 1) * NEXP / LAST) exp_op(n);
+        if (PAR == 1 && u == LAST - 1) {
+#pragma unroll
+          for (int qt = 0; qt < QT; ++qt) sum_pair(qt);
+        }
+        if (MASKED && u == LAST + NL - 1) mask(j + 2, s);
+        const int r = u - LAST - NL;
 #pragma unroll
         for (int n = 0; n < NMAX; ++n)
-          if (u >= EXP_END && n >= (u - EXP_END) * NMAX / (NM - EXP_END) && n < (u - EXP_END + 1) * NMAX / (NM - EXP_END)) {
-            if (n % 9 < 8) max_step(sn, n / 9, n % 9);
-            else max_done(n / 9);
+          if (r >= 0 && n >= r * NMAX / REST && n < (r + 1) * NMAX / REST) {
+            if (n % NMT < 8) max_step(s, n / NMT, n % NMT, PAR == 0);
+            else max_done(n / NMT);
           }
       }
       __builtin_amdgcn_sched_barrier(0);
     }
+    if constexpr (PAR == 1) {
+      slot ^= 1;
+      kfo ^= STAGE;
+      vfo ^= STAGE;
+    }
   };
+  constexpr std::integral_constant<int, 0> even{};
+  constexpr std::integral_constant<int, 1> odd{};
   constexpr std::true_type yes{};
   constexpr std::false_type no{};
   int j = 0;
-  for (; j + 5 < nkv; j += 4) {  // blocks up to j + 4 are not the last; the stages' offsets are constants
-    step(0, sa, sb, yes, no);
-    step(1, sb, sa, yes, no);
-    step(2, sa, sb, yes, no);
-    step(3, sb, sa, yes, no);
+  for (; j + 4 < nkv; j += 2) {  // block j + 3 is not the last
+    step(j, sa, even, yes, no);
+    step(j + 1, sb, odd, yes, no);
   }
-  for (; j + 2 < nkv; ++j) {
-    step(j, sa, sb, yes, no);
+  if (j + 2 < nkv) {
+    step(j, sa, even, yes, yes);
+    step(j + 1, sb, odd, yes, yes);
+    j += 2;
+  }
+  step(j, sa, even, no, no);
+  if (j + 2 == nkv) step(j + 1, sb, odd, no, no);
 #pragma unroll
-    for (int qt = 0; qt < QT; ++qt) sa[qt] = sb[qt];
-  }
-  if (j + 1 < nkv) {
-    step(j, sa, sb, yes, yes);
-#pragma unroll
-    for (int qt = 0; qt < QT; ++qt) sa[qt] = sb[qt];
-    ++j;
-  }
-  step(j, sa, sb, no, no);
+  for (int qt = 0; qt < QT; ++qt) sum_pair(qt);
   __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));  // the trailing reloads
 
   // out[query][dim]: lane holds dims dt * 32 + 8 * g + 4 * hh + {0..3}, g = 0..3
@@ -1732,12 +1779,13 @@ int64_t busiest_cu_time(int64_t nwg, int per_cu, const int *t) {
   const int64_t m = (nwg + kCus - 1) / kCus;
   return (m / per_cu) * t[per_cu] + t[m % per_cu];
 }
-// t: VGGT frames (1374 keys, D 64) with k workgroups of the pipelined kernel
-// resident per CU, in 0.1 us: 128-query 17.5 / 27.0 / 39.7 us (k = 1 / 2 / 3),
-// 256-query 28.0 / 49.0 us (k = 1 / 2). The 256-query form must win by 3%; so
-// set, the rule picks the faster form at each of 1 to 10 frames, 7 x 900, 10 x
-// 700, 2 / 4 / 6 / 8 frames as one sequence, 1 / 4 x 2048 and 2 x 1029 tokens
-// (both timed at each).
+// t: costs of k workgroups of the pipelined kernel resident per CU, in 0.1 us
+// of VGGT frames (1374 keys, D 64): 128-query 17.5 / 27.0 / 39.7 us (k = 1 / 2
+// / 3), 256-query 28.0 / 49.0 us (k = 1 / 2). The 256-query form must win by
+// 3%; so set, the rule picks the faster form at each of 1 to 10 frames, 7 x
+// 900, 10 x 700, 2 / 4 / 6 / 8 frames as one sequence, 1 / 4 x 2048 and 2 x
+// 1029 tokens (128- / 256-query, us: 1 frame 21.4 / 31.2, 5 57.7 / 54.4, 8 83.8
+// / 81.5, 9 96.0 / 101, 8 as one sequence 594 / 562, 6 366 / 411).
 bool use_256_query(const AttnParams &p) {
   static const int t1[4] = {0, 175, 270, 397}, t2[3] = {0, 280, 490};
   const int64_t n1 = p.B * p.H * ((p.Lq + 127) / 128), n2 = p.B * p.H * ((p.Lq + 255) / 256);
@@ -1803,8 +1851,8 @@ hipError_t launch_t(const AttnParams &p, hipStream_t s) {
       const bool dma = dma_fits(p, 2);
       if (p.D == 64) {
         // key groups while their doubled grid leaves CUs idle (16 heads x 1024
-        // tokens: 13.7 us against 15.3 pipelined; x 1029, one more tile: 19.0
-        // / 16.3)
+        // tokens: 13.3 us against 15.5 pipelined; x 1029, one more tile: 18.2
+        // / 16.7)
         const int ks = key_groups(p, dma ? kCus : 3 * kCus);
         if (ks == 4) return launch_mfma<T, 64, 1, 128, 2, true, true, false, false, false, 4>(p, s);
         if (ks == 2) return launch_mfma<T, 64, 1, 64, 3, true, true, false, false, false, 2>(p, s);
@@ -1817,8 +1865,8 @@ hipError_t launch_t(const AttnParams &p, hipStream_t s) {
       }
       if (p.D == 128) {
         // a few key blocks do not pay for the pipeline's first (2 x 16 x 2048
-        // queries: 64 keys 12.0 us against 12.8, 128 13.9 / 14.3, 256 18.3 /
-        // 18.1)
+        // queries: 64 keys 12.2 us against 13.6, 192 15.5 / 16.7, 256 18.3 /
+        // 18.1, 512 25.8 / 25.5)
         if (dma && p.Lk >= 256) return launch_pipe<T, 128, 1, 2>(p, s);
         if (dma) return launch_mfma<T, 128, 1, 64, 2, true, true, false, true>(p, s);
         return launch_mfma<T, 128, 1, 64, 2, true, true, false, false>(p, s);

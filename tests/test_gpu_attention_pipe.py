@@ -110,3 +110,89 @@ def test_sdpa_f32_pipelined_reversed_keys(dev):
               ops.desc(out), torch.cuda.current_stream().cuda_stream)
     want = ops.sdpa(q, k.flip(2).contiguous(), v.flip(2).contiguous(), 0.125)
     assert torch.equal(out, want)
+
+
+def _backwards(t):
+    """Descriptor of [B, H, L, D] `t` with its tokens in reverse order: a negative stride, which the direct loads of
+    the pipelined kernel do not address, so that the register-staged kernel takes the call."""
+    from lux3d_fused import _lib
+    st = list(t.stride())
+    code = {torch.bfloat16: _lib.BF16, torch.float16: _lib.F16}[t.dtype]
+    return _lib.descriptor(t.data_ptr() + (t.shape[2] - 1) * st[2] * t.element_size(), code, list(t.shape),
+                           [st[0], st[1], -st[2], st[3]])
+
+
+# grids on both sides of the 128- / 256-query rule and beyond the key groups of either kernel; D 128 from the 256 keys
+# where the pipelined kernel starts, D 64 from one key; 1-6 pairs of 32-key blocks, whole, cut and with an odd block
+STAGED = [(400, 128, lk, 64, "") for lk in (1, 32, 33, 64, 65, 96, 130, 192, 224, 333)] \
+    + [(512, 256, lk, 64, "") for lk in (1, 33, 64, 95, 129, 192, 300)] \
+    + [(2, 130, lk, 128, "") for lk in (256, 257, 288, 289, 320, 383, 20000)] \
+    + [(h, lq, lk, d, pro) for h, lq, lk, d in ((400, 128, 130, 64), (512, 256, 95, 64), (2, 130, 289, 128))
+       for pro in ("_layernorm_rope2d", "_rms_norm_heads", "_l2norm_rope3d")]
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("h,lq,lk,d,pro", STAGED)
+def test_sdpa_pipelined_has_the_bits_of_the_register_staged_kernel(dev, h, lq, lk, d, pro, dt):
+    """The pipelined kernel does the arithmetic of the register-staged one in its order (a reference maximum and a row
+    sum for each 64 keys), with each of the q prologues: the same keys through either give the same bits. Scores vary
+    enough to move the reference maximum."""
+    from lux3d_fused import _lib, ops
+    print(f"\n[case] pipelined / staged {pro} [{h},{lq},{lk},{d}] {dt}", flush=True)
+    g = torch.Generator(device="cpu").manual_seed(lq + lk + d)
+    q = (torch.randn((1, h, lq, d), generator=g) * 1.5).to(dev).to(TDT[dt])
+    k, v = (torch.randn((1, h, lk, d), generator=g).to(dev).to(TDT[dt]) for _ in range(2))
+    k = k * 3
+    w, b = (1 + 0.1 * torch.randn(d, generator=g)).to(dev), (0.1 * torch.randn(d, generator=g)).to(dev)
+    scale, stream = d ** -0.5, torch.cuda.current_stream().cuda_stream
+    if pro == "_l2norm_rope3d":
+        ang = torch.randn((lq, d // 2), generator=g).to(dev)
+        head = (q, (1 + 0.1 * torch.randn((h, d), generator=g)).to(dev), torch.cos(ang), torch.sin(ang))
+    elif pro == "_layernorm_rope2d":
+        ang = torch.randn((1, 1, lq, d), generator=g).to(dev)
+        head = (q, w, b, 1e-6, torch.cos(ang), torch.sin(ang))
+    else:
+        head = (q, w, 1e-6) if pro else (q,)
+
+    def run(kd, vd):
+        out = torch.full_like(q, float("nan"))
+        _lib.call("lux3d_sdpa" + pro, *(ops._d(a) if torch.is_tensor(a) else a for a in head), kd, vd, scale,
+                  ops._d(out), stream)
+        return out
+    kf, vf = k.flip(2).contiguous(), v.flip(2).contiguous()
+    pipelined, staged = run(ops._d(kf), ops._d(vf)), run(_backwards(k), _backwards(v))
+    assert not bool(torch.isnan(staged).any())
+    assert torch.equal(pipelined, staged)
+
+
+@pytest.mark.parametrize("first", [31, 32, 50, 63])
+@pytest.mark.parametrize("h,lq,d", [(400, 128, 64), (512, 256, 64), (2, 130, 128)])
+def test_sdpa_pipelined_first_keys_masked_by_infinity(dev, h, lq, d, first):
+    """Keys masked by a score of -inf, fewer than the 64 of the first reference maximum, weigh nothing."""
+    from lux3d_fused import ops
+    print(f"\n[case] sdpa -inf first={first} h={h} lq={lq} d={d}", flush=True)
+    g = torch.Generator(device="cpu").manual_seed(first + d)
+    lk = 300
+    q, k, v = (torch.randn((1, h, n, d), generator=g).to(dev).to(torch.bfloat16) for n in (lq, lk, lk))
+    q[..., 0], k[..., 0] = 1, 0
+    masked = k.clone()
+    masked[:, :, :first, 0] = float("-inf")
+    out = ops.sdpa(q, masked, v, d ** -0.5)
+    _check(out, q, k[:, :, first:], v[:, :, first:], d ** -0.5, "bf16")
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("h,lq,d", [(400, 128, 64), (512, 256, 64), (2, 130, 128)])
+@pytest.mark.parametrize("lk", [257, 289, 300, 320, 350])
+def test_sdpa_pipelined_keys_past_lk_are_not_read(dev, h, lq, lk, d, dt):
+    """K and V are views into a buffer whose 160 rows past Lk of every head are NaN (the pipeline loads up to 160 rows
+    ahead): none reaches the output, with even and odd numbers of blocks and whole and cut last ones."""
+    from lux3d_fused import ops
+    print(f"\n[case] pipelined nan tail [{h},{lq},{lk},{d}] {dt}", flush=True)
+    g = torch.Generator(device="cpu").manual_seed(lk * 3 + d)
+    buf = torch.full((2, 1, h, lk + 160, d), float("nan"))
+    buf[:, :, :, :lk] = torch.randn((2, 1, h, lk, d), generator=g)
+    buf = buf.to(dev).to(TDT[dt])
+    k, v = buf[0, :, :, :lk], buf[1, :, :, :lk]
+    q = torch.randn((1, h, lq, d), generator=g).to(dev).to(TDT[dt])
+    _check(ops.sdpa(q, k, v, d ** -0.5), q, k, v, d ** -0.5, dt)
