@@ -33,6 +33,7 @@
 // deterministic.
 #include "common.hpp"
 #include "kernels.hpp"
+#include "q8_tiles.hpp"
 
 namespace lux3d {
 
@@ -230,7 +231,6 @@ __global__ __launch_bounds__(kGemmThreads, MINW) void q8_0_gemm_kernel(Q8GemmPar
 // (bias added, rounded once) and writes whole 16-byte row pieces.
 
 constexpr int kRingStages = 3;
-constexpr int kRingThreads = 512;
 
 // 8 int8 (two dwords) -> bf16(f32(q) * d), RNE; q * d is exact in f32
 __device__ __forceinline__ bf16x8_t dequant8(uint32_t lo, uint32_t hi, float d) {
@@ -881,39 +881,13 @@ hipError_t launch_x3(const Q8GemmParams &p, hipStream_t s) {
   return hipGetLastError();
 }
 
-// f32 activations: the kernel and tile that take the shortest time by these
-// measured costs, linear in the 32-deep steps of k (ns; one round = every CU
-// busy once, alone or, for the 64 x 128 tiles, with two workgroups):
-//   few rows      64 x 16     262 steps + 2000 a round
-//   1 x 4, KG 3   32 x 128    345 steps + 3500 a round
-//   2 x 2, KG 2   64 x 128    570 steps + 4500 a round
-//   2 x 2         64 x 128   1050 steps + 4000 for two a CU, 760 steps + 4000 for one
-//   2 x 4        128 x 256   1500 steps + 5000 a round
-// With 128 x 256 tiles alone a product of 1029 rows left most CUs idle or took
-// a second round for a few tiles: 1029 x 4096 -> 1024 154 -> 76 us, 1029 x 1536
-// -> 1536 76 -> 34, 512 x 8192 -> 2048 268 -> 91, 2049 x 1024 -> 4096 109 -> 91,
-// 256 x 1024 -> 4096 36.7 -> 16.1.
 template <typename OUT>
 hipError_t launch_f32(const Q8GemmParams &p, hipStream_t s) {
-  if (p.M <= 16) return launch_few_rows<OUT, true, 1>(p, s);
-  auto tiles = [&](int64_t bm, int64_t bn) { return (double)((p.M + bm - 1) / bm) * (double)((p.N + bn - 1) / bn); };
-  auto rounds = [](double t) { return __builtin_ceil(t / 256); };
-  const double steps = (double)(p.K / 32), mid = tiles(64, 128);
-  const double few = p.M > 65535 * 64 ? __builtin_inf() : rounds(tiles(64, 16)) * (262 * steps + 2000);  // its grid
-  const double k3 = rounds(tiles(32, 128)) * (345 * steps + 3500);
-  const double k2 = rounds(mid) * (570 * steps + 4500);
-  // two a CU; the tiles past the last full round run as on half-empty CUs
-  const double pair = 1050 * steps + 4000, one = 760 * steps + 4000, full = __builtin_floor(mid / 512);
-  const double k1 = mid <= 256 ? one
-                    : mid <= 512 ? pair
-                    : mid / 512 * pair + (mid > full * 512 ? (full < 2 ? 0.75 : 0.5) * one : 0);
-  const double large = rounds(tiles(128, 256)) * (1500 * steps + 5000);
-  const double best = __builtin_fmin(__builtin_fmin(__builtin_fmin(few, k3), __builtin_fmin(k2, k1)), large);
-  if (best == large) return launch_x3<OUT, 2, 4, 2, 2, 1>(p, s);
-  if (best == k1) return launch_x3<OUT, 2, 2, 1, 2, 1>(p, s);
-  if (best == k2) return launch_x3<OUT, 2, 2, 1, 2, 2>(p, s);
-  if (best == k3) return launch_x3<OUT, 1, 4, 1, 1, 3>(p, s);
-  return launch_few_rows<OUT, true, 4>(p, s);
+  const Q8Tile tile = q8_tile_f32(p.M, p.N, p.K);
+  if (tile.few()) return tile.rows == 16 ? launch_few_rows<OUT, true, 1>(p, s) : launch_few_rows<OUT, true, 4>(p, s);
+  if (tile.rows == 128) return launch_x3<OUT, 2, 4, 2, 2, 1>(p, s);
+  if (tile.rows == 32) return launch_x3<OUT, 1, 4, 1, 1, 3>(p, s);
+  return tile.groups == 1 ? launch_x3<OUT, 2, 2, 1, 2, 1>(p, s) : launch_x3<OUT, 2, 2, 1, 2, 2>(p, s);
 }
 
 // The ring kernel's buffer descriptors span one tile (at most 256 rows of x,
@@ -934,50 +908,17 @@ hipError_t launch_ring(const Q8GemmParams &p, hipStream_t s) {
   return hipGetLastError();
 }
 
-// bf16 activations: the kernel and tile that take the shortest time by these
-// measured costs, linear in the 64-deep steps of k (ns; a round is 256 tiles,
-// one for each CU, whether a CU holds one workgroup or several):
-//   few rows   64 x 16    280 steps + 2000 a round
-//   ring       32 x 128   410 steps a round + 2500
-//              64 x 128   450 steps + 1000 a round + 3000
-//             128 x 128   530 steps + 4000 for one round, else 610 steps + 2000 a round
-//             160 x 128   660 steps + 5000 a round
-//             128 x 256  1150 steps + 2000 a round
-//             256 x 256  1600 steps + 3000 a round
-// A lone small tile is bound by the latency of its serial k loop, and a 256 x
-// 256 tile reads each operand least. One rule for all sizes instead of the
-// first tile that covered every CU, us: 1029 x 1536 -> 9216 59 -> 46, 1536 x
-// 2048 -> 8192 75 -> 59, 512 x 8192 -> 2048 70 -> 56, 512 x 1536 -> 1536 17 ->
-// 13, 3000 x 1024 -> 3072 41 -> 31. Groups of wavefronts that share k gain
-// nothing here (512 x 8192 -> 2048: 61 us with four groups of 32 x 128): a
-// workgroup of any tile already takes what one CU loads.
 template <typename OUT>
 hipError_t launch_bf16(const Q8GemmParams &p, hipStream_t s) {
-  if (p.M <= 16) return launch_few_rows<OUT, false, 1>(p, s);
-  const double steps = (double)(p.K / 64);
-  auto rounds = [&](int64_t bm, int64_t bn) {
-    return __builtin_ceil((double)((p.M + bm - 1) / bm) * (double)((p.N + bn - 1) / bn) / 256);
-  };
-  const double r128 = rounds(128, 128);
-  const double cost[7] = {p.M > 65535 * 64 ? __builtin_inf() : rounds(64, 16) * (280 * steps + 2000),  // its grid
-                          rounds(32, 128) * 410 * steps + 2500,
-                          rounds(64, 128) * (450 * steps + 1000) + 3000,
-                          r128 == 1 ? 530 * steps + 4000 : r128 * (610 * steps + 2000),
-                          rounds(160, 128) * (660 * steps + 5000),
-                          rounds(128, 256) * (1150 * steps + 2000),
-                          rounds(256, 256) * (1600 * steps + 3000)};
-  int best = 6;  // the larger tile of two equal ones
-  for (int i = 5; i >= 0; --i)
-    if (cost[i] < cost[best]) best = i;
-  switch (best) {
-    case 0: return launch_few_rows<OUT, false, 4>(p, s);
-    case 1: return launch_ring<OUT, 32, 4>(p, s);
-    case 2: return launch_ring<OUT, 64, 4>(p, s);
-    case 3: return launch_ring<OUT, 128, 4>(p, s);
-    case 4: return launch_ring<OUT, 160, 4>(p, s);
-    case 5: return launch_ring<OUT, 128, 8>(p, s);
+  const Q8Tile tile = q8_tile_bf16(p.M, p.N, p.K);
+  if (tile.few()) return tile.rows == 16 ? launch_few_rows<OUT, false, 1>(p, s) : launch_few_rows<OUT, false, 4>(p, s);
+  if (tile.cols == 256) return tile.rows == 256 ? launch_ring<OUT, 256, 8>(p, s) : launch_ring<OUT, 128, 8>(p, s);
+  switch (tile.rows) {
+    case 32: return launch_ring<OUT, 32, 4>(p, s);
+    case 64: return launch_ring<OUT, 64, 4>(p, s);
+    case 128: return launch_ring<OUT, 128, 4>(p, s);
   }
-  return launch_ring<OUT, 256, 8>(p, s);
+  return launch_ring<OUT, 160, 4>(p, s);
 }
 
 template <typename OUT>

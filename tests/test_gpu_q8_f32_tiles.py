@@ -7,11 +7,16 @@ pytestmark = pytest.mark.gpu
 TDT = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}
 
 
+# k of 2, 30, 32 and 34 steps of 32; two groups are taken from 4 steps on
+TILES = [(tile, m, n, k) for tile, m, n in (("32x128 / 3", 129, 1500), ("32x128 / 3", 160, 1537), ("64x128", 700, 1500),
+                                            ("64x128 / 2", 700, 1500), ("64x128", 1100, 2060),
+                                            ("64x128, aligned", 1088, 2176), ("128x256", 1100, 4100))
+         for k in ((64,) if (tile, m) == ("64x128", 700) else
+                   (128 if tile == "64x128 / 2" else 64, 960, 1024, 1088))]
+
+
 @pytest.mark.parametrize("ydt", ["f32", "bf16", "f16"])
-@pytest.mark.parametrize("k", [64, 960, 1024, 1088])     # 2, 30, 32 and 34 steps of 32
-@pytest.mark.parametrize("tile,m,n", [("32x128 / 3", 129, 1500), ("32x128 / 3", 160, 1537), ("64x128 / 2", 700, 1500),
-                                      ("64x128", 1100, 2060), ("64x128, aligned", 1088, 2176),
-                                      ("128x256", 1100, 4100)])
+@pytest.mark.parametrize("tile,m,n,k", TILES)
 def test_q8_linear_f32_tiles(tile, m, n, k, ydt):
     """|error| <= (k / 32 + 40) 2^-23 sum |x w| (an f32 sum's last place per MFMA, block and group) plus the result's
     rounding."""

@@ -15,9 +15,13 @@ def _weights(n, k, seed, dev):
 
 
 # k: one chunk, one pair, an odd number of chunks, and what 4, 8 and 16 wavefronts cover in one and more turns
+KS = [64, 128, 192, 576, 1088, 2112, 4160]
+SIZES = [(1, 1), (2, 15), (15, 16), (16, 33), (17, 17), (63, 40), (64, 16), (65, 50), (130, 31)]
+
+
 @pytest.mark.parametrize("xdt,ydt", [("bf16", "bf16"), ("bf16", "f32"), ("f32", "f32"), ("f32", "f16")])
-@pytest.mark.parametrize("k", [64, 128, 192, 576, 1088, 2112, 4160])
-@pytest.mark.parametrize("m,n", [(1, 1), (2, 15), (15, 16), (16, 33), (17, 17), (63, 40), (64, 16), (65, 50), (130, 31)])
+@pytest.mark.parametrize("k", KS)
+@pytest.mark.parametrize("m,n", SIZES)
 def test_q8_linear_few_rows(m, n, k, xdt, ydt):
     """|error| <= (k / 32 + 40) 2^-23 sum |x w| (an f32 sum's last place per MFMA, block and wavefront) plus the
     result's rounding."""

@@ -6,12 +6,14 @@ import torch
 pytestmark = pytest.mark.gpu
 TDT = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}
 
+TILES = [(tile, m, n, k) for k in (960, 1024) for tile, m, n in (
+         ("32x128", 129, 1500), ("32x128", 160, 1537), ("64x128", 700, 1500), ("64x128", 704, 1601),
+         ("128x128", 1400, 1500), ("128x128, two a CU", 7100, 1100), ("160x128", 1400, 3100), ("128x256", 1100, 7000),
+         ("256x256", 1500, 6000))]
+
 
 @pytest.mark.parametrize("ydt", ["bf16", "f32", "f16"])
-@pytest.mark.parametrize("k", [960, 1024])
-@pytest.mark.parametrize("tile,m,n", [("32x128", 129, 1500), ("32x128", 160, 1537), ("64x128", 700, 1500),
-                                      ("64x128", 704, 1601), ("128x128", 1400, 1500), ("128x128, two a CU", 7100, 1100),
-                                      ("160x128", 1400, 3100), ("128x256", 1100, 7000), ("256x256", 1500, 6000)])
+@pytest.mark.parametrize("tile,m,n,k", TILES)
 def test_q8_linear_ring_tiles(tile, m, n, k, ydt):
     """|error| <= (k / 32 + 40) 2^-23 sum |x w| (an f32 sum's last place per MFMA) plus the result's rounding."""
     from lux3d_fused import ops
