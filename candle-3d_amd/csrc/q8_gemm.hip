@@ -739,9 +739,12 @@ __global__ __launch_bounds__(64 * WM * WN * KG, 1) void q8_0_gemm_x3_kernel(Q8Ge
 // weights' bytes bound them, and tiles of 128 rows leave most CUs idle (72
 // workgroups at N 9216) behind a serial k loop. A workgroup owns 16 weight rows
 // and 16 MT rows of x; its NW wavefronts take pairs of 64-deep chunks of k in
-// turn, each keeping the loads of U chunks in flight, and their sums
-// (v_mfma_f32_16x16x32_bf16: x rows x weight rows) are added in wavefront order
-// through LDS. k order inside a chunk: lane group g = lane / 16 holds weights
+// turn, and their sums (v_mfma_f32_16x16x32_bf16: x rows x weight rows) are
+// added in wavefront order through LDS. A turn of the loop takes U chunks, but
+// as compiled a wavefront waits for each chunk's loads and multiplies before it
+// issues the next chunk's (the branch after each chunk keeps them apart: 51
+// VGPRs): one chunk is in flight per wavefront, and only the other wavefronts
+// of the SIMD cover its latency. k order inside a chunk: lane group g = lane / 16 holds weights
 // 16 g .. 16 g + 15 of its row as one 16-byte load (one Q8_0 block, one scale),
 // bytes 8 s .. + 7 in MFMA s, and x alike. XF32: f32 x in three exact bf16
 // terms, the int8 weights exact, one MFMA per term and Q8_0 block (lane group
@@ -752,7 +755,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, 1) void q8_0_gemm_x3_kernel(Q8Ge
 template <typename OUT, bool XF32, int NW, int MT>
 __global__ __launch_bounds__(64 * NW) void q8_0_few_rows_kernel(Q8GemmParams p) {
   typedef float f32x4_t __attribute__((ext_vector_type(4)));
-  constexpr int U = MT == 1 ? (XF32 ? 4 : 8) : 2;  // chunks in flight
+  constexpr int U = MT == 1 ? (XF32 ? 4 : 8) : 2;  // chunks per turn
   __shared__ float part[NW][MT * 256];
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), g = lane >> 4;
   const int64_t n0 = (int64_t)blockIdx.x * 16, m0 = (int64_t)blockIdx.y * 16 * MT;
