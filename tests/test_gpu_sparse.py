@@ -108,6 +108,20 @@ def test_sparse_conv3d_reference_cases(dev, ops, orc):
         assert np.array_equal(got, want), k
 
 
+def _run_conv(ops, conv, nbr, x, path):
+    """The convolution through the C entry of one path, whichever route SparseConv3d.forward takes at the size."""
+    from lux3d_fused import _lib
+    d, stream = ops.desc, torch.cuda.current_stream().cuda_stream
+    out = torch.full((x.shape[0], conv.out_channels), float("nan"), device=x.device)
+    if path == "rulebook":
+        rb = ops.SparseRulebook(nbr)
+        _lib.call("lux3d_sparse_conv3d_rulebook", d(x), d(rb.pairs), d(rb.counts), d(conv.weight27), d(conv.bias), d(out),
+                  stream)
+    else:
+        _lib.call("lux3d_sparse_conv3d", d(x), d(nbr), d(conv.weight27), d(conv.bias), d(out), stream)
+    return out
+
+
 @pytest.mark.parametrize("n,cin,cout,res,surface", [
     (3000, 64, 96, 32, False),
     (5000, 128, 128, 64, True),
@@ -129,8 +143,7 @@ def test_sparse_conv3d_mfma(dev, ops, orc, n, cin, cout, res, surface, path):
     wt = torch.from_numpy(w27).permute(1, 0, 2).contiguous()  # back to [Cout, 27, Cin]
     conv = ops.SparseConv3d(wt.to(dev), torch.from_numpy(bias).to(dev), cin, cout)
     nbr_d = ops.sparse_neighbors(torch.from_numpy(coords).to(dev))
-    arg = ops.SparseRulebook(nbr_d) if path == "rulebook" else nbr_d
-    out = conv.forward(arg, torch.from_numpy(x).to(dev))
+    out = _run_conv(ops, conv, nbr_d, torch.from_numpy(x).to(dev), path)
     torch.cuda.synchronize()
     nbr = orc.sparse_neighbors(coords)
     rows = np.arange(n) if n * cin * cout <= 5e8 else np.sort(np.random.default_rng(1).choice(n, 600, replace=False))
@@ -258,7 +271,7 @@ def test_sparse_conv3d_rulebook_matches_reference_order(dev, ops, orc, cin, cout
     conv = ops.SparseConv3d(torch.from_numpy(w27).permute(1, 0, 2).contiguous().to(dev), torch.from_numpy(bias).to(dev),
                             cin, cout)
     nbr = ops.sparse_neighbors(torch.from_numpy(coords).to(dev))
-    got = conv.forward(ops.SparseRulebook(nbr), torch.from_numpy(x).to(dev)).cpu().numpy()
+    got = _run_conv(ops, conv, nbr, torch.from_numpy(x).to(dev), "rulebook").cpu().numpy()
     want = orc.sparse_conv3d(x, orc.sparse_neighbors(coords), w27, bias)
     assert np.array_equal(got, want)
 

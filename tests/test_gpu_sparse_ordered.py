@@ -71,6 +71,75 @@ def test_sparse_conv3d_ordered(dev, ops, orc, n, cin, cout, passes):
     bound = (6 * 27 * cin / 16 + 64) * 2.0 ** -23 * mag.astype(np.float64) + 2.0 ** -23 * np.abs(want) + 1e-30
     err = np.abs(out[rows].astype(np.float64) - want)
     assert (err <= bound).all(), f"worst {np.max(err / bound):.3f} of the bound"
+    # the bound of one output allows more than a lost third term costs. Over all outputs: an f32 chain's rounding steps
+    # of 2^-25 each (root mean square) on partial sums no larger than the result's scale stay near 2e-7, without the
+    # third terms of x and w, or without the product of the second ones, the relative error is 2e-6 and more
+    exact = np.zeros((len(rows), cout))
+    for k in range(27):
+        has = valid[:, k] >= 0
+        exact[has] += x[valid[has, k]].astype(np.float64) @ w27[k].astype(np.float64).T
+    if bias is not None:
+        exact += bias
+    assert np.linalg.norm(out[rows] - exact) <= 1e-6 * np.linalg.norm(exact)
+
+
+@pytest.mark.parametrize("passes", [3, 9])
+@pytest.mark.parametrize("n,cin,cout", [(129, 64, 64), (127, 64, 128), (1000, 96, 200), (64 * 1024 + 5, 64, 100),
+                                        (8 * 1024, 128, 2049)])
+def test_sparse_conv3d_ordered_keeps_all_bits(dev, ops, n, cin, cout, passes):
+    """One product per output, of a value with 24 significant bits and a power of two, is exact: every term of x and
+    of the weights takes part, in every tile shape."""
+    print(f"\n[case] ordered conv, one product n={n} cin={cin} cout={cout} passes={passes}", flush=True)
+    rng = np.random.default_rng(n + cout)
+    nbr = _table(n, n + cin, n < 500)
+    tap, chan = rng.integers(0, 27, cout), rng.integers(0, cin, cout)
+    full = lambda s: ((rng.integers(1 << 23, 1 << 24, s) | 1) * 2.0 ** -23 * rng.choice([-1, 1], s))  # noqa: E731
+    power = lambda s: 2.0 ** rng.integers(-3, 4, s)  # noqa: E731
+    table = ops._sparse_order(torch.from_numpy(nbr).to(dev), passes)
+    for x, w in ((full((n, cin)), power(cout)), (power((n, cin)), full(cout))):
+        x, w = x.astype(np.float32), w.astype(np.float32)
+        w27 = np.zeros((27, cout, cin), dtype=np.float32)
+        w27[tap, np.arange(cout), chan] = w
+        conv = ops.SparseConv3d(torch.from_numpy(w27).permute(1, 0, 2).contiguous().to(dev), None, cin, cout)
+        out = torch.full((n, cout), float("nan"), device=dev)
+        conv._forward_ordered(table, torch.from_numpy(x).to(dev), out)
+        src = nbr[:, tap]
+        has = (src >= 0) & (src < n)
+        want = np.where(has, x[np.where(has, src, 0), chan] * w, np.float32(0))
+        assert np.array_equal(out.cpu().numpy(), want)
+
+
+def test_sparse_conv3d_ordered_under_capture(dev, ops):
+    """forward() captured from a rulebook and from a neighbour table: every replay has the eager result, with eager
+    work between replays and new features in the captured buffer."""
+    print("\n[case] ordered conv under capture", flush=True)
+    coords = random_coords(9000, 64, 5, True)
+    n, cin, cout = len(coords), 128, 96
+    g = torch.Generator(device="cpu").manual_seed(n)
+    x = torch.randn((n, cin), generator=g).to(dev)
+    conv = ops.SparseConv3d((torch.randn((cout, 27, cin), generator=g) / (27 * cin) ** 0.5).to(dev), None, cin, cout)
+    nbr = ops.sparse_neighbors(torch.from_numpy(coords).to(dev))
+    rb = ops.SparseRulebook(nbr)
+    conv.forward(rb, x), conv.forward(nbr, x)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        a, b = conv.forward(rb, x), conv.forward(nbr, x)
+    for i in range(4):
+        x.normal_()
+        want = conv.forward(rb, x), conv.forward(nbr, x)
+        a.fill_(float("nan")), b.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(a, want[0]) and torch.equal(b, want[1]), i
+
+
+def test_sparse_rulebook_of_no_voxels(dev, ops):
+    print("\n[case] rulebook and ordered conv without voxels", flush=True)
+    rb = ops.SparseRulebook(torch.empty((0, 27), dtype=torch.int32, device=dev))
+    conv = ops.SparseConv3d(torch.zeros((64, 27, 64), device=dev), None, 64, 64)
+    assert conv.forward(rb, torch.empty((0, 64), device=dev)).shape == (0, 64)
+    assert rb.counts.cpu().tolist() == [0] * 27
 
 
 @pytest.mark.parametrize("passes", [3, 9])
