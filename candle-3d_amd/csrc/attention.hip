@@ -1326,10 +1326,9 @@ __global__ __launch_bounds__(256, MINW) void attn_f32x3_kernel(AttnParams p, int
 // instructions per step go into the gaps, in chains of two or more (a lone
 // dependent chain takes 8.5 cycles per instruction). K and V are
 // double-buffered planes of 32 rows of 128 bytes, swizzled (k_swz, v_swz); one
-// barrier per step. Before / after, us: 16 x 1029 x 64 52.7 / 43.0 (1.2 us per
-// step and wavefront, half of it MFMAs; 144 of 256 CUs have work), 8 x 16 x
-// 1374 x 64 347 / 330 (1126 TFLOP/s in bf16 products; large bf16 matrix
-// products reach 1230-1580 here).
+// barrier per step. Needs two blocks or more. Against attn_f32x3_kernel, us: 16
+// x 1029 x 64 with q's rotation 52.9 / 44.4 (144 of 256 CUs have work), 8 x 16
+// x 1374 x 64 339 / 323 (1150 TFLOP/s in bf16 products).
 template <bool R3>
 __global__ __launch_bounds__(256, 2) void attn_f32x3_pipe_kernel(AttnParams p, int64_t nqb, int64_t nwg) {
   using op_t = bf16x8_t;
@@ -1465,7 +1464,6 @@ __global__ __launch_bounds__(256, 2) void attn_f32x3_pipe_kernel(AttnParams p, i
   for (int c = 0; c < NC; ++c)
 #pragma unroll
     for (int u = 0; u < 6; ++u) sa = M::run(kfrag(0, tx[u], c), q[ty[u]][c], sa);
-  if (nkv == 1) mask(0, sa);
 #pragma unroll
   for (int i = 0; i < 9; ++i) max_item(sa, i);
 
@@ -1569,11 +1567,9 @@ __global__ __launch_bounds__(256, 2) void attn_f32x3_pipe_kernel(AttnParams p, i
     step(j, 0, sa, sb, yes, no);
     step(j + 1, 1, sb, sa, yes, yes);
     step(j + 2, 0, sa, sb, no, no);
-  } else if (j + 1 < nkv) {
+  } else {
     step(j, 0, sa, sb, yes, yes);
     step(j + 1, 1, sb, sa, no, no);
-  } else {
-    step(j, 0, sa, sb, no, no);
   }
 
   // out[query][dim] (f32): lane holds dims dt * 32 + 8 * g + 4 * hh + {0..3}, g = 0..3
@@ -1746,13 +1742,18 @@ bool dma_fits(const AttnParams &p, int eb) {
   return p.k_st >= 0 && p.v_st >= 0 && ((p.Lk + 64) * st + p.D) * eb < (int64_t(1) << 31);
 }
 
+constexpr int64_t kCus = 256;  // MI355X
+
 hipError_t launch_f32x3(const AttnParams &p, hipStream_t s) {
   const int64_t nqb = (p.Lq + 127) / 128;
   const int64_t nwg = p.B * p.H * nqb;
   if (nwg > INT32_MAX) return hipErrorInvalidValue;
   const dim3 grid((unsigned)nwg), block(256);
   const bool r3 = p.qpro == QP_R3;
-  if (p.D == 64 && p.Lk >= 192) {  // fewer keys do not pay for the pipeline's start (2 x 50: 6.3 us against 7.4; 16 x 201: 14.1 / 13.8)
+  // Fewer keys do not pay for the pipeline's start (us, attn_f32x3_kernel / pipelined: 16 heads x 160 11.9 / 12.4, x
+  // 201 14.8 / 15.1, x 261 18.1 / 17.8), which two workgroups on a CU partly hide for the former: 160 x 261 29.8 /
+  // 31.4, 160 x 350 36.6 / 37.7, 128 x 400 42.0 / 42.3, 160 x 400 58.9 / 56.7, 128 x 512 51.7 / 50.5.
+  if (p.D == 64 && p.Lk >= (nwg <= kCus ? 224 : 400)) {
     if (r3) hipLaunchKernelGGL((attn_f32x3_pipe_kernel<true>), grid, block, 0, s, p, nqb, nwg);
     else hipLaunchKernelGGL((attn_f32x3_pipe_kernel<false>), grid, block, 0, s, p, nqb, nwg);
   } else if (p.D == 64) {
@@ -1771,7 +1772,6 @@ hipError_t launch_f32x3(const AttnParams &p, hipStream_t s) {
 // the busiest CU less work (below). The exact-probability kernel takes
 // 128-query ones up to kShortQ queries.
 constexpr int64_t kShortQ = 4096;
-constexpr int64_t kCus = 256;  // MI355X
 
 // Time of the busiest CU when nwg workgroups spread evenly over the CUs and
 // per_cu of them run at once; t[k] is the time of k resident workgroups.
@@ -1799,8 +1799,16 @@ bool use_256_query(const AttnParams &p) {
 // workgroups, each wavefront with 1 / KS of the keys. These kernels are
 // VALU-bound (exact_sdpa_heads: about 370 VALU instructions per 64-key block
 // and wavefront against 32 MFMAs), so the busiest SIMD's share sets the
-// time; KS = 2 is taken while the doubled grid stays within max_grid: three
-// workgroups per CU, or one where the pipelined kernel is the other choice. Measured (exact_sdpa_heads bf16, D 64, us, KS = 1 / 2 / 4):
+// time; KS = 2 is taken while the doubled grid fits three workgroups per CU
+// and, where the pipelined kernel is the other choice (pipe), only
+// - while its 64-query workgroups leave every CU one at most (16 heads x 1024
+//   tokens 13.3 us against 15.5 pipelined, 48 x 300 7.6 / 8.4; with more, x
+//   1029 18.2 / 16.7, 80 x 300 9.8 / 9.0), or
+// - where they fit two a CU and the pipelined kernel's 128-query ones do not
+//   fit one a CU: it would take a second round for a few (30 heads x 1029 22.5
+//   us against 26.2, 96 x 300 10.2 / 11.9, 44 x 700 15.1 / 18.1; with 64-query
+//   ones past two a CU, 32 x 1029 24.3 / 24.2, 60 x 550 16.5 / 16.2).
+// Measured (exact_sdpa_heads bf16, D 64, us, KS = 1 / 2 / 4):
 // 16 heads x 1029 tokens 26.3 / 24.2 / 25.5, x 1024 22.6 / 17.3 / 16.4,
 // 8 x 1029 23.9 / 17.3 / 16.7, 2 x 16 x 1029 37.0 / 32.2 / 38.1, 4 x 4096
 // 78.3 / 55.0 / 50.5, 16 x 2048 45.7 / 43.2 / 50.9; KS = 4 (128-key blocks,
@@ -1808,9 +1816,9 @@ bool use_256_query(const AttnParams &p) {
 // elsewhere, so it is not chosen by default. Needs Lk >= the block (every
 // key group sees keys in block 0). LUX3D_ATTN_KS=1 / 2 / 4 forces a choice
 // (timing).
-int key_groups(const AttnParams &p, int64_t max_grid) {
-  const int64_t tiles = p.B * p.H * ((p.Lq + 127) / 128);
-  int ks = 2 * tiles <= max_grid ? 2 : 1;
+int key_groups(const AttnParams &p, bool pipe) {
+  const int64_t tiles = p.B * p.H * ((p.Lq + 127) / 128), tiles64 = p.B * p.H * ((p.Lq + 63) / 64);
+  int ks = 2 * tiles <= 3 * kCus && (!pipe || tiles64 <= kCus || (tiles > kCus && tiles64 <= 2 * kCus)) ? 2 : 1;
   if (const char *e = getenv("LUX3D_ATTN_KS")) ks = atoi(e);
   if (ks == 4 && p.Lk >= 128) return 4;
   if (ks == 2 && p.Lk >= 64) return 2;
@@ -1833,7 +1841,7 @@ hipError_t launch_t(const AttnParams &p, hipStream_t s) {
     // the generic kernel (f32 throughout)
     if constexpr (T::code == LUX3D_BF16) {
       if (p.mfma && p.D == 64) {
-        const int ks = key_groups(p, 3 * kCus);
+        const int ks = key_groups(p, false);
         if (ks == 4) return launch_mfma<T, 64, 1, 128, 2, true, false, false, false, true, 4>(p, s);
         if (ks == 2) return launch_mfma<T, 64, 1, 64, 3, true, false, false, false, true, 2>(p, s);
         if (p.Lq <= kShortQ) return launch_mfma<T, 64, 1, 64, 3, true, false, false, false, true>(p, s);
@@ -1850,10 +1858,7 @@ hipError_t launch_t(const AttnParams &p, hipStream_t s) {
     if (p.mfma) {
       const bool dma = dma_fits(p, 2);
       if (p.D == 64) {
-        // key groups while their doubled grid leaves CUs idle (16 heads x 1024
-        // tokens: 13.3 us against 15.5 pipelined; x 1029, one more tile: 18.2
-        // / 16.7)
-        const int ks = key_groups(p, dma ? kCus : 3 * kCus);
+        const int ks = key_groups(p, dma);
         if (ks == 4) return launch_mfma<T, 64, 1, 128, 2, true, true, false, false, false, 4>(p, s);
         if (ks == 2) return launch_mfma<T, 64, 1, 64, 3, true, true, false, false, false, 2>(p, s);
         if (use_256_query(p)) {

@@ -33,7 +33,7 @@ def _check(got, q, k, v, scale, dt):
 SHAPES = [(1, 3, 130, 1), (2, 80, 130, 31), (2, 80, 130, 33), (2, 80, 129, 64), (2, 80, 128, 95), (2, 80, 127, 96),
           (2, 80, 1, 128), (2, 80, 130, 129), (2, 80, 130, 160), (2, 80, 130, 191), (2, 80, 130, 224), (2, 80, 130, 255),
           (2, 80, 130, 256), (2, 80, 257, 257), (2, 80, 130, 289), (1, 16, 1024, 300), (1, 16, 1029, 300),
-          (4, 16, 2048, 70)]
+          (4, 16, 2048, 70), (1, 48, 300, 64), (1, 100, 300, 130), (1, 64, 420, 130)]
 
 
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
@@ -67,18 +67,20 @@ def test_sdpa_pipelined_rising_scores(dev, d):
     _check(ops.sdpa(q, k, v, 1.0), q, k, v, 1.0, "bf16")
 
 
-@pytest.mark.parametrize("lk", [192, 193, 223, 224, 225, 256, 287, 300])
+# one to a few workgroups, which pipeline from 224 keys on, and more than 256, from 400 on
+@pytest.mark.parametrize("h,lq,lk", [(3, lk, lk) for lk in (192, 193, 223, 224, 225, 256, 287, 300, 320, 351)]
+                         + [(160, 130, lk) for lk in (399, 400, 416, 447)])
 @pytest.mark.parametrize("rotate", [False, True])
-def test_sdpa_f32_pipelined(dev, lk, rotate):
+def test_sdpa_f32_pipelined(dev, h, lq, lk, rotate):
     """The pipelined f32 kernel (D 64) over odd and even numbers of 32-key blocks and their remainders, against 64
     bits: |error| <= (d + lk) 2^-22 max|v|, an f32 sum's last place per product in scores and output, and 1.2e-6 of the
     result's 2-norm: f32 arithmetic stays near 5e-7 over these sizes, while q, k, p or v without their third term, or
     a product without that of the second terms, give 2.0e-6 and more."""
     from lux3d_fused import ops
-    print(f"\n[case] sdpa f32 pipelined lk={lk} rotate={rotate}", flush=True)
-    b, h, d, lq = 1, 3, 64, lk
+    print(f"\n[case] sdpa f32 pipelined h={h} lq={lq} lk={lk} rotate={rotate}", flush=True)
+    b, d = 1, 64
     g = torch.Generator(device="cpu").manual_seed(lk)
-    q, k, v = (torch.randn((b, lk, h, d), generator=g).to(dev).transpose(1, 2) for _ in range(3))
+    q, k, v = (torch.randn((b, n, h, d), generator=g).to(dev).transpose(1, 2) for n in (lq, lk, lk))
     out = torch.full((b, h, lq, d), float("nan"), device=dev)
     qd = q.double()
     if rotate:
