@@ -33,14 +33,20 @@ constexpr int64_t kFewRowsMaxM = 65535 * 64;
 // With 128 x 256 tiles alone a product of 1029 rows left most CUs idle or took
 // a second round for a few tiles: 1029 x 4096 -> 1024 154 -> 76 us, 1029 x 1536
 // -> 1536 76 -> 34, 512 x 8192 -> 2048 268 -> 91, 2049 x 1024 -> 4096 109 -> 91,
-// 256 x 1024 -> 4096 36.7 -> 16.1.
+// 256 x 1024 -> 4096 36.7 -> 16.1. The share of `one` that the 64 x 128 tiles
+// past a full round of 512 cost is fitted where it matters first, just past the
+// round (model against measured: 516 tiles 85 / 87 us, 552 62 / 62, 1032 90 /
+// 93, 1104 180 / 179); towards the next round it is up to a quarter too long
+// (752 tiles 144 / 116), so that some sizes keep the 128 x 256 tile where this
+// one is shorter (2500 x 1024 -> 4096: 111 us against 96), and none takes a
+// longer one than before.
 inline Q8Tile q8_tile_f32(int64_t m, int64_t n, int64_t k) {
   if (m <= 16) return {16, 16, 1};
   const double steps = (double)(k / 32), mid = q8_tiles(m, n, 64, 128);
   const double few = m > kFewRowsMaxM ? INFINITY : q8_rounds(q8_tiles(m, n, 64, 16)) * (262 * steps + 2000);
   const double k3 = q8_rounds(q8_tiles(m, n, 32, 128)) * (345 * steps + 3500);
   const double k2 = q8_rounds(mid) * (570 * steps + 4500);
-  // two a CU; the tiles past the last full round run as on half-empty CUs
+  // two a CU; the tiles past the last full round of them (see above)
   const double pair = 1050 * steps + 4000, one = 760 * steps + 4000, full = std::floor(mid / 512);
   const double k1 = mid <= 256 ? one
                     : mid <= 512 ? pair

@@ -598,10 +598,10 @@ class SparseConv3d:
             return out
         nbr = coords_or_nbr if coords_or_nbr.shape[-1] == 27 else sparse_neighbors(coords_or_nbr)
         n, cin = nbr.shape[0], self.in_channels
-        # the order of one call's rows costs 21-60 us: output-stationary tiles
-        # are faster where the convolution itself is short (us, with the order:
-        # 3k x 128 140 against 121, 20k x 64 110 / 74; 4k x 256 215 / 248, 20k
-        # x 128 154 / 175, 150k x 64 249 / 271)
+        # the order of one call's rows costs 25-70 us: output-stationary tiles
+        # are faster where the convolution itself is short (us, with the order,
+        # against those tiles: 4k x 128 156 / 129, 20k x 64 130 / 87; 2k x 256
+        # 231 / 247, 20k x 128 180 / 194, 150k x 64 270 / 308)
         long = cin >= 256 or (cin >= 128 and n >= 8192) or n >= 98304
         if (long and nbr.dim() == 2 and nbr.dtype == torch.int32 and nbr.is_contiguous()
                 and self._ordered(feats, n)):
@@ -633,8 +633,12 @@ class SparseConv3d:
 
 def _order_passes(n: int, cin: int) -> int:
     """Passes of the ordered convolution: 9 (of 3 taps) where a tile's rows would otherwise share too few masks of 9
-    taps and a pass over the output is cheap beside its products (5k x 1024: 1094 against 1272 us, 12k x 1024: 2239 /
-    2419); else 3 (2k x 1024: 672 against 735 us, 40k x 512: 1791 / 1913, 150k x 256: 990 / 1299)."""
+    taps and a pass over the output is cheap beside its products, else 3. Us, 3 / 9 passes, on a closed surface: 4k x
+    1024 1077 / 1009, 16k x 1024 3656 / 3077, 24k x 1024 4464 / 4298, 4k x 768 730 / 656, 24k x 768 2677 / 2653; 2k x
+    512 357 / 410, 24k x 512 1278 / 1327, 150k x 256 1847 / 2267, 20k x 128 150 / 221. Nine are shorter beyond 24576
+    voxels too (28k x 1024 5162 / 4886, 40k x 1024 6982 / 6889; half-filled shells gain up to 15%), but there a
+    rulebook of every wide set would hold the second table (144 bytes a voxel), and sets of that size are convolved
+    with 512 channels or fewer."""
     return 9 if cin >= 768 and 4096 <= n < 24576 else 3
 
 
@@ -642,7 +646,13 @@ class SparseRulebook:
     """Per-tap (dst, src) pair lists of a coordinate set (lux3d_sparse_rulebook)
     and its rows ordered by the taps they have (lux3d_sparse_order; one table
     per pass count that a convolution on it may take), built once and reused
-    by every convolution on it."""
+    by every convolution on it: from 64 input channels on they read a table,
+    narrower ones the pairs. 216 bytes a voxel and 18-30 us for the pairs, 120
+    bytes and 28-72 us for the table of 3 passes, and from 4096 to 24575
+    voxels 144 bytes and 25-29 us for that of 9. A convolution on it with a
+    table is shorter than with the pairs at every width and size timed (us:
+    24k x 1024 4298 against 5372, 24k x 512 1278 / 1723, 2k x 512 357 / 1001,
+    150k x 256 1847 / 3411, 4k x 64 92 / 155)."""
 
     def __init__(self, nbr: torch.Tensor):
         n = nbr.shape[0]

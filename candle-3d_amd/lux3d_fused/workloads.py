@@ -480,7 +480,7 @@ def cfg4_dinov3_rope(dev) -> Workload:
 
 
 # The configs[1..4] ops of the headline benchmark (the >=70%-of-peak targets), then extras.
-def _q8_linear(dev, cfg, m, k, n, what, xdt=torch.bfloat16) -> Workload:
+def _q8_linear(dev, cfg, m, k, n, what, xdt=torch.bfloat16, name="") -> Workload:
     """Q8_0 quantized linear y = x @ dequant(W)^T + bias at a model's shape.
     The weight is repacked once (load time, outside the timed launch); x
     rotates over sets that exceed the Infinity Cache, the weight stays one
@@ -493,7 +493,7 @@ def _q8_linear(dev, cfg, m, k, n, what, xdt=torch.bfloat16) -> Workload:
     qs, scales = ops.q8_0_repack(blocks, n, k)
     bias = _normal(s + 2, (n,), dev, torch.float32, 0.0, 0.5)
     nbytes = m * k * xe + n * k + n * (k // 32) * 4 + n * 4 + m * n * 2
-    n_sets = _n_sets(m * k * xe + m * n * 2)
+    n_sets = min(_n_sets(m * k * xe + m * n * 2), 64)
     xs = [_fill_like(x0, j) for j in range(n_sets)]
     ys = [torch.empty((m, n), dtype=torch.bfloat16, device=dev) for _ in range(n_sets)]
     dx = [ops.desc(v) for v in xs]
@@ -512,7 +512,8 @@ def _q8_linear(dev, cfg, m, k, n, what, xdt=torch.bfloat16) -> Workload:
                       f"x[{m},{k}] f32 @ W[{n},{k}]^T ({what})", launch, n_sets, flops=2 * m * k * n,
                       peak_tflops=2500.0 / 3)
     else:
-        wl = Workload("q8_0_linear", cfg, "q8_0_gemm_ring_kernel<BF16,...>", "bf16 x int8(Q8_0) -> f32 acc", nbytes,
+        kern = "q8_0_few_rows_kernel<BF16>" if m <= 16 else "q8_0_gemm_ring_kernel<BF16,...>"
+        wl = Workload(name or "q8_0_linear", cfg, kern, "bf16 x int8(Q8_0) -> f32 acc", nbytes,
                       f"x[{m},{k}] @ W[{n},{k}]^T ({what})", launch, n_sets, flops=2 * m * k * n)
     wl._keep = (xs, ys, qs, scales, bias, blocks, dx, dy, dq, dsc, db)
     return wl
@@ -526,6 +527,11 @@ def cfg4_q8_0_linear(dev) -> Workload:
 def cfg2_q8_0_linear(dev) -> Workload:
     # TripoSG width 2048 -> 4x feed-forward, both CFG halves (2 x 2048 tokens)
     return _q8_linear(dev, 2, 4096, 2048, 8192, "TripoSG FF up-projection")
+
+
+def cfg3_q8_0_linear_adaln(dev) -> Workload:
+    # TRELLIS.2's modulation vectors, one per batch element: the few-rows kernel
+    return _q8_linear(dev, 3, 2, 1536, 9216, "TRELLIS.2 AdaLN modulation, batch 2", name="q8_0_linear_adaln")
 
 
 def cfg2_q8_0_linear_f32(dev) -> Workload:
@@ -813,9 +819,12 @@ def _shell_coords(n, res, seed):
     return c[rng.permutation(len(c))[:n]]
 
 
-def _sparse_conv(dev, name, n, ch, res, reps, rulebook=True):
+def _sparse_conv(dev, name, n, ch, res, reps, route="ordered"):
     """SparseConv3d (trellis2_sparse.rs:197-243) on shell voxels: x f32
-    [N, C] -> [N, C], the ConvNeXt block conv of a decoder stage."""
+    [N, C] -> [N, C], the ConvNeXt block conv of a decoder stage, from a built
+    coordinate set. route "ordered" is what ops.SparseConv3d takes at these
+    sizes; "pairs" is lux3d_sparse_conv3d_rulebook, "output_stationary" is
+    lux3d_sparse_conv3d."""
     from . import _lib
     coords = torch.from_numpy(_shell_coords(n, res, 11)).to(dev)
     n = coords.shape[0]
@@ -831,26 +840,29 @@ def _sparse_conv(dev, name, n, ch, res, reps, rulebook=True):
 
     rb = ops.SparseRulebook(nbr)
     dp, dc = ops.desc(rb.pairs), ops.desc(rb.counts)
+    passes = ops._order_passes(n, ch)
+    planes = torch.empty(27 * ((ch + 31) // 32 * 32) * ch * 3, dtype=torch.bfloat16, device=dev)
+    dt, dpl = ops.desc(rb.tables[passes]), ops.desc(planes)
 
     def launch(i):
-        if rulebook:
+        if route == "ordered":
+            _lib.call("lux3d_sparse_conv3d_ordered", dx[i % 2], dt, dw, dpl, db, do[i % 2], _cur())
+        elif route == "pairs":
             _lib.call("lux3d_sparse_conv3d_rulebook", dx[i % 2], dp, dc, dw, db, do[i % 2], _cur())
         else:
             _lib.call("lux3d_sparse_conv3d", dx[i % 2], dn, dw, db, do[i % 2], _cur())
     nbytes = n * ch * 4 * 2 + n * 27 * 4 + 27 * ch * ch * 4
     # f32 arithmetic on the bf16 matrix cores: six bf16 MFMAs per f32 step,
     # so the ceiling is the bf16 peak / 6
-    if rulebook:
-        tile = 128 if ch >= 512 else 64
-        kern, arith, peak = (f"sparse_tap_x3_kernel<{tile},{tile}> x 27 taps",
-                             "f32 (bf16 matrix cores, three-term splits)", 2500.0 / 6)
-    else:
-        kern, arith, peak = ("sparse_conv_x3_kernel<64,64>", "f32 (bf16 matrix cores, three-term splits)",
-                             2500.0 / 6)
+    arith, peak = "f32 (bf16 matrix cores, three-term splits)", 2500.0 / 6
+    tile = 128 if ch >= 512 else 64
+    kern = {"ordered": f"sparse_ordered_x3_kernel x {passes} passes + split_weights_kernel",
+            "pairs": f"sparse_tap_x3_kernel<{tile},{tile}> x 27 taps",
+            "output_stationary": "sparse_conv_x3_kernel<64,64>"}[route]
     wl = Workload(name, 3, kern, arith, nbytes,
                   f"{n} shell voxels in {res}^3, C {ch} -> {ch}, {used / n:.1f} active taps per voxel", launch, 2,
                   flops=2 * used * ch * ch, reps=reps, peak_tflops=peak)
-    wl._keep = (coords, nbr, xs, w27, bias, outs, dx, do, dn, dw, db, rb, dp, dc)
+    wl._keep = (coords, nbr, xs, w27, bias, outs, dx, do, dn, dw, db, rb, dp, dc, planes, dt, dpl)
     return wl
 
 
@@ -864,9 +876,38 @@ def cfg3_sparse_conv_c256(dev) -> Workload:
     return _sparse_conv(dev, "sparse_conv_c256", 150000, 256, 256, 10)
 
 
+def cfg3_sparse_conv_c1024_pairs(dev) -> Workload:
+    # the C entry over pair lists on the same sets, for comparison
+    return _sparse_conv(dev, "sparse_conv_c1024_pairs", 24000, 1024, 64, 5, route="pairs")
+
+
+def cfg3_sparse_conv_c256_pairs(dev) -> Workload:
+    return _sparse_conv(dev, "sparse_conv_c256_pairs", 150000, 256, 256, 10, route="pairs")
+
+
 def cfg3_sparse_conv_c256_output_stationary(dev) -> Workload:
     # the one-kernel output-stationary path on the same set, for comparison
-    return _sparse_conv(dev, "sparse_conv_c256_output_stationary", 150000, 256, 256, 10, rulebook=False)
+    return _sparse_conv(dev, "sparse_conv_c256_output_stationary", 150000, 256, 256, 10, route="output_stationary")
+
+
+def cfg3_sparse_order(dev) -> Workload:
+    """The rows of a coordinate set ordered by their taps (lux3d_sparse_order,
+    3 passes), built once per set beside the pair lists. Algorithmic bytes:
+    the neighbour table read, the order table written."""
+    from . import _lib
+    coords = torch.from_numpy(_shell_coords(150000, 256, 11)).to(dev)
+    n = coords.shape[0]
+    nbr = ops.sparse_neighbors(coords)
+    tables = [torch.empty((3, n, 10), dtype=torch.int32, device=dev) for _ in range(2)]
+    ws = torch.empty(3 << 9, dtype=torch.int32, device=dev)
+    dn, dws, dt = ops.desc(nbr), ops.desc(ws), [ops.desc(v) for v in tables]
+
+    def launch(i):
+        _lib.call("lux3d_sparse_order", dn, dt[i % 2], dws, _cur())
+    wl = Workload("sparse_order", 3, "order_clear/rows/starts_kernel", "int32", n * 27 * 4 + n * 30 * 4,
+                  f"{n} shell voxels in 256^3, 3 passes", launch, 2, reps=20)
+    wl._keep = (coords, nbr, tables, ws, dn, dws, dt)
+    return wl
 
 
 def cfg3_sparse_rulebook(dev) -> Workload:
@@ -952,6 +993,7 @@ EXTRAS: List[Callable] = [
     cfg4_q8_0_linear_int8,
     cfg2_q8_0_linear_int8,
     cfg2_q8_0_linear_f32,
+    cfg3_q8_0_linear_adaln,
     cfg1_sdpa_frame,
     cfg1_sdpa_frame_qln,
     cfg1_sdpa_frame_f32,
@@ -970,7 +1012,10 @@ EXTRAS: List[Callable] = [
     cfg4_sdpa_dinov3_rope_bf16,
     cfg3_sparse_conv_c1024,
     cfg3_sparse_conv_c256,
+    cfg3_sparse_conv_c1024_pairs,
+    cfg3_sparse_conv_c256_pairs,
     cfg3_sparse_conv_c256_output_stationary,
+    cfg3_sparse_order,
     cfg3_sparse_rulebook,
     cfg3_c2s,
 ]
