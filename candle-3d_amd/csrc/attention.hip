@@ -760,7 +760,7 @@ __global__ __launch_bounds__(256, MINW) void attn_mfma_kernel(AttnParams p, int6
 // K and V arrive by direct global -> LDS loads in two stages of 64 keys; stage
 // g holds V's blocks 2 g, 2 g + 1 and K's blocks 2 g + 3, 2 g + 4, as steps 2
 // g and 2 g + 1 read them (what lies past Lk reads as zeros). One barrier per
-// stage; its successor's loads are issued behind it.
+// stage; its successor's loads are issued behind it. Lk must be above 64.
 template <typename T, int D, int QT, int MINW, int QP>
 __global__ __launch_bounds__(256, MINW) void attn_pipe_kernel(AttnParams p, int64_t nqb, int64_t nwg) {
   using M = Mma<T>;
@@ -877,7 +877,7 @@ __global__ __launch_bounds__(256, MINW) void attn_pipe_kernel(AttnParams p, int6
   auto sum_pair = [&](int qt) { l[qt] = __builtin_fmaf(l[qt], alpha[qt], ls[qt]); };
 
   // prologue: K's blocks 0, 1 and 2, 3 into the slot of stage 1, stage 0; the
-  // scores of the first pair and its maximum
+  // scores of the first pair, which is whole, and its maximum
   load_k(0, lds0 + STAGE + 2 * KB);
   load_k(2 * kblock, lds0 + STAGE);
   load_stage(0);
@@ -898,10 +898,6 @@ __global__ __launch_bounds__(256, MINW) void attn_pipe_kernel(AttnParams p, int6
   scores(sb);
 #pragma unroll
   for (int c = 0; c < NC; ++c) kf[c] = kfrag(STAGE - 2 * KB, c);
-  if (nkv <= 2) {
-    mask(0, sa);
-    mask(1, sb);
-  }
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
 #pragma unroll
@@ -1858,14 +1854,22 @@ hipError_t launch_t(const AttnParams &p, hipStream_t s) {
     if (p.mfma) {
       const bool dma = dma_fits(p, 2);
       if (p.D == 64) {
-        const int ks = key_groups(p, dma);
+        // One pair of 32-key blocks leaves nothing to overlap, and up to three
+        // whole pairs attn_mfma_kernel, which takes 64 keys at a time, does no
+        // more work (us, against pipelined: 800 heads x 64 queries x 64 keys
+        // 9.1 / 10.4, 400 x 128 x 128 8.2 / 8.8, x 192 10.0 / 10.8, 512 x 256 x
+        // 192 19.4 / 20.3; x 256 21.5 / 22.5, but 128 x 1374 x 256 27.7 / 28.0,
+        // 64 x 1024 x 256 12.0 / 12.0; 800 x 64 x 96 12.5 / 11.3, x 160 15.4 /
+        // 14.6)
+        const bool pipe = dma && p.Lk > 64 && (p.Lk > 192 || p.Lk % 64);
+        const int ks = key_groups(p, pipe);
         if (ks == 4) return launch_mfma<T, 64, 1, 128, 2, true, true, false, false, false, 4>(p, s);
         if (ks == 2) return launch_mfma<T, 64, 1, 64, 3, true, true, false, false, false, 2>(p, s);
         if (use_256_query(p)) {
-          if (dma) return launch_pipe<T, 64, 2, 2>(p, s);
+          if (pipe) return launch_pipe<T, 64, 2, 2>(p, s);
           return launch_mfma<T, 64, 2, 64, 2, true, true, true, false>(p, s);
         }
-        if (dma) return launch_pipe<T, 64, 1, 3>(p, s);
+        if (pipe) return launch_pipe<T, 64, 1, 3>(p, s);
         return launch_mfma<T, 64, 1, 64, 3, true, true, false, false>(p, s);
       }
       if (p.D == 128) {

@@ -28,10 +28,11 @@ def _check(got, q, k, v, scale, dt):
     assert bool((err <= bound).all()), float((err / bound).max())
 
 
-# (b, h, lq, lk): 1-9 key blocks of 32 and their remainders, 256 keys (the shortest D 128 takes), one row, query tiles
-# of 128 / 256 and one more, and grids on both sides of each rule of the dispatch
+# (b, h, lq, lk): 1-9 key blocks of 32 and their remainders (D 64 is pipelined from 65 keys on but for 128 and 192), 256
+# keys (the shortest D 128 takes), one row, query tiles of 128 / 256 and one more, and grids on both sides of each rule
+# of the dispatch
 SHAPES = [(1, 3, 130, 1), (2, 80, 130, 31), (2, 80, 130, 33), (2, 80, 129, 64), (2, 80, 128, 95), (2, 80, 127, 96),
-          (2, 80, 1, 128), (2, 80, 130, 129), (2, 80, 130, 160), (2, 80, 130, 191), (2, 80, 130, 224), (2, 80, 130, 255),
+          (2, 80, 1, 128), (2, 80, 130, 129), (2, 80, 130, 160), (2, 80, 130, 65), (2, 80, 130, 192), (2, 80, 130, 193), (2, 80, 130, 191), (2, 80, 130, 224), (2, 80, 130, 255),
           (2, 80, 130, 256), (2, 80, 257, 257), (2, 80, 130, 289), (1, 16, 1024, 300), (1, 16, 1029, 300),
           (4, 16, 2048, 70), (1, 48, 300, 64), (1, 100, 300, 130), (1, 64, 420, 130)]
 
@@ -128,9 +129,9 @@ def _backwards(t):
 
 
 # grids on both sides of the 128- / 256-query rule and beyond the key groups of either kernel; D 128 from the 256 keys
-# where the pipelined kernel starts, D 64 from one key; 1-6 pairs of 32-key blocks, whole, cut and with an odd block
-STAGED = [(400, 128, lk, 64, "") for lk in (1, 32, 33, 64, 65, 96, 130, 192, 224, 333)] \
-    + [(512, 256, lk, 64, "") for lk in (1, 33, 64, 95, 129, 192, 300)] \
+# where the pipelined kernel starts, D 64 from one key (pipelined from 65, but for 128 and 192); 1-6 pairs of 32-key blocks, whole, cut and with an odd block
+STAGED = [(400, 128, lk, 64, "") for lk in (1, 32, 33, 64, 65, 96, 97, 127, 130, 160, 192, 193, 224, 256, 320, 333)] \
+    + [(512, 256, lk, 64, "") for lk in (1, 33, 64, 95, 129, 192, 256, 300)] \
     + [(2, 130, lk, 128, "") for lk in (256, 257, 288, 289, 320, 383, 20000)] \
     + [(h, lq, lk, d, pro) for h, lq, lk, d in ((400, 128, 130, 64), (512, 256, 95, 64), (2, 130, 289, 128))
        for pro in ("_layernorm_rope2d", "_rms_norm_heads", "_l2norm_rope3d")]
