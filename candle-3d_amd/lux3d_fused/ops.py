@@ -597,19 +597,25 @@ class SparseConv3d:
                           _d(self.weight27), _d(self.bias), _d(out), _stream(feats))
             return out
         nbr = coords_or_nbr if coords_or_nbr.shape[-1] == 27 else sparse_neighbors(coords_or_nbr)
-        n, cin = nbr.shape[0], self.in_channels
-        # the order of one call's rows costs 25-70 us: output-stationary tiles
-        # are faster where the convolution itself is short (us, with the order,
-        # against those tiles: 4k x 128 156 / 129, 20k x 64 130 / 87; 2k x 256
-        # 231 / 247, 20k x 128 180 / 194, 150k x 64 270 / 308)
-        long = cin >= 256 or (cin >= 128 and n >= 8192) or n >= 98304
-        if (long and nbr.dim() == 2 and nbr.dtype == torch.int32 and nbr.is_contiguous()
+        n = nbr.shape[0]
+        if (self._order_pays(n) and nbr.dim() == 2 and nbr.dtype == torch.int32 and nbr.is_contiguous()
                 and self._ordered(feats, n)):
-            self._forward_ordered(_sparse_order(nbr, _order_passes(n, cin)), feats, out)
+            self._forward_ordered(_sparse_order(nbr, _order_passes(n, self.in_channels)), feats, out)
         else:
             _lib.call("lux3d_sparse_conv3d", _d(feats), _d(nbr), _d(self.weight27), _d(self.bias), _d(out),
                       _stream(feats))
         return out
+
+    def _order_pays(self, n: int) -> bool:
+        """Whether a call that has the neighbour table alone orders its rows. Order and weight planes cost 25-90 us a
+        call; output-stationary tiles are faster where the convolution itself is short: few voxels (us, those tiles
+        against ordered, on a closed surface and on scattered voxels: 8 x 512 54 / 70, 52 / 51, 12 x 1024 a quarter
+        less ordered on both, 200 x 256 197 / 213 scattered, 300 x 256 equal), and few products (128 -> 64: 16k voxels
+        136 / 144, 26k 139 / 146 scattered, 40k 13% less ordered; 128 -> 128: 9k 132 / 143 scattered, 20k 14% less;
+        128 -> 256: 9k 9-15% less; 64 -> 64: 20k 87 / 130, 100k 210 / 182)."""
+        cin, products = self.in_channels, n * self.in_channels * self.out_channels
+        return ((cin >= 512 and n >= 16) or (cin >= 256 and n >= 256)
+                or (cin >= 128 and n >= 8192 and products >= 1 << 28) or n >= 98304)
 
     def _ordered(self, feats: torch.Tensor, n: int) -> bool:
         """Whether lux3d_sparse_conv3d_ordered takes this call on n voxels (its layout and size limits). Any other

@@ -114,10 +114,11 @@ def test_sparse_conv3d_ordered_under_capture(dev, ops):
     work between replays and new features in the captured buffer."""
     print("\n[case] ordered conv under capture", flush=True)
     coords = random_coords(9000, 64, 5, True)
-    n, cin, cout = len(coords), 128, 96
+    n, cin, cout = len(coords), 128, 256
     g = torch.Generator(device="cpu").manual_seed(n)
     x = torch.randn((n, cin), generator=g).to(dev)
     conv = ops.SparseConv3d((torch.randn((cout, 27, cin), generator=g) / (27 * cin) ** 0.5).to(dev), None, cin, cout)
+    assert conv._order_pays(n)
     nbr = ops.sparse_neighbors(torch.from_numpy(coords).to(dev))
     rb = ops.SparseRulebook(nbr)
     conv.forward(rb, x), conv.forward(nbr, x)
@@ -174,7 +175,7 @@ def test_sparse_conv3d_ordered_exact_sums(dev, ops, orc, passes):
 def test_sparse_conv3d_routes_agree(dev, ops, orc):
     """forward() from coordinates, from a neighbour table and from a rulebook built on it before the table's buffer
     is reused, on the sizes where the route or the pass count changes."""
-    for n0, cin, cout in ((8192, 128, 64), (4100, 768, 64), (4000, 256, 96), (8100, 128, 64)):
+    for n0, cin, cout in ((8192, 128, 64), (4100, 768, 64), (4000, 256, 96), (8100, 128, 64), (20000, 128, 256), (60, 512, 96)):
         coords = random_coords(n0, 64, n0, True)
         n = len(coords)
         g = torch.Generator(device="cpu").manual_seed(n)

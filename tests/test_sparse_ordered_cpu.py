@@ -30,3 +30,15 @@ def test_sparse_ordered_argument_errors():
 def test_pass_counts():
     assert [ops._order_passes(n, 1024) for n in (4095, 4096, 24575, 24576)] == [3, 9, 9, 3]
     assert ops._order_passes(8000, 512) == 3
+
+
+def test_calls_that_order_their_rows():
+    """Both sides of each line of the rule for a call on a neighbour table."""
+    def pays(n, cin, cout):
+        conv = ops.SparseConv3d.__new__(ops.SparseConv3d)
+        conv.in_channels, conv.out_channels = cin, cout
+        return conv._order_pays(n)
+    for cin, cout, line in ((1024, 1024, 16), (512, 8, 16), (256, 32, 256), (496, 1024, 256), (128, 64, 32768),
+                            (128, 128, 16384), (128, 256, 8192), (192, 192, 8192), (240, 16, 69906), (128, 8, 98304),
+                            (64, 64, 98304)):
+        assert [pays(n, cin, cout) for n in (line - 1, line)] == [False, True], (cin, cout)
