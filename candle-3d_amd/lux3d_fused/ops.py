@@ -590,8 +590,9 @@ class SparseConv3d:
         out = torch.empty((feats.shape[0], self.out_channels), dtype=torch.float32, device=feats.device)
         if isinstance(coords_or_nbr, SparseRulebook):
             rb = coords_or_nbr
-            if self._ordered(feats, rb.nbr.shape[0]):
-                self._forward_ordered(rb.tables[_order_passes(feats.shape[0], self.in_channels)], feats, out)
+            tables = getattr(rb, "tables", None)  # a rulebook pickled before they existed has the pairs alone
+            if tables and self._ordered(feats, rb.nbr.shape[0]):
+                self._forward_ordered(tables[_order_passes(feats.shape[0], self.in_channels)], feats, out)
             else:
                 _lib.call("lux3d_sparse_conv3d_rulebook", _d(feats), _d(rb.pairs), _d(rb.counts),
                           _d(self.weight27), _d(self.bias), _d(out), _stream(feats))

@@ -173,8 +173,8 @@ def test_sparse_conv3d_ordered_exact_sums(dev, ops, orc, passes):
 
 
 def test_sparse_conv3d_routes_agree(dev, ops, orc):
-    """forward() from coordinates, from a neighbour table and from a rulebook built on it before the table's buffer
-    is reused, on the sizes where the route or the pass count changes."""
+    """forward() from coordinates, from a neighbour table, from a rulebook built on it before the table's buffer is
+    reused and from one without row orders, on the sizes where the route or the pass count changes."""
     for n0, cin, cout in ((8192, 128, 64), (4100, 768, 64), (4000, 256, 96), (8100, 128, 64), (20000, 128, 256), (60, 512, 96)):
         coords = random_coords(n0, 64, n0, True)
         n = len(coords)
@@ -187,6 +187,8 @@ def test_sparse_conv3d_routes_agree(dev, ops, orc):
         want = conv.forward(nbr, x)
         got = [conv.forward(c, x)]
         nbr.fill_(-1)
+        got.append(conv.forward(rb, x))
+        del rb.tables
         got.append(conv.forward(rb, x))
         for y in got:
             # f32 sums of up to 27 Cin terms in another order
