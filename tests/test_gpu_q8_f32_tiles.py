@@ -12,7 +12,8 @@ TILES = [(tile, m, n, k) for tile, m, n in (("32x128 / 3", 129, 1500), ("32x128 
                                             ("64x128 / 2", 700, 1500), ("64x128", 1100, 2060),
                                             ("64x128, aligned", 1088, 2176), ("128x256", 1100, 4100))
          for k in ((64,) if (tile, m) == ("64x128", 700) else
-                   (128 if tile == "64x128 / 2" else 64, 960, 1024, 1088))]
+                   (128 if tile == "64x128 / 2" else 64, 960, 1024, 1088))] \
+    + [("32x128 / 3", 16, 32000, 512), ("32x128 / 3", 7, 30001, 576)]
 
 
 @pytest.mark.parametrize("ydt", ["f32", "bf16", "f16"])

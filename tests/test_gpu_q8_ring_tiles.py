@@ -9,7 +9,8 @@ TDT = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}
 TILES = [(tile, m, n, k) for k in (960, 1024) for tile, m, n in (
          ("32x128", 129, 1500), ("32x128", 160, 1537), ("64x128", 700, 1500), ("64x128", 704, 1601),
          ("128x128", 1400, 1500), ("128x128, two a CU", 7100, 1100), ("160x128", 1400, 3100), ("128x256", 1100, 7000),
-         ("256x256", 1500, 6000))]
+         ("256x256", 1500, 6000))] \
+    + [("32x128", 16, 32000, 256), ("32x128", 5, 32700, 512), ("32x128", 257, 4096, 64), ("128x128", 2049, 1024, 128)]
 
 
 @pytest.mark.parametrize("ydt", ["bf16", "f32", "f16"])

@@ -53,11 +53,12 @@ def test_every_tile_is_named():
 
 
 def test_few_rows_sizes(choice):
-    """Up to 16 rows always; the few-rows tests' longer ones take its four row tiles wherever the costs say so, which
-    is for each k at 17 and more rows of a narrow weight."""
+    """Up to 16 rows of all but wide weights; the few-rows tests' longer ones take its four row tiles wherever the costs
+    say so, which is for each k at 17 and more rows of a narrow weight."""
     for dtype in ("f32", "bf16"):
         assert all(choice(dtype, m, n, k) == (16, 16, 1) for m in (1, 16) for n in (1, 9216) for k in (64, 8192))
         for k in test_gpu_q8_few_rows.KS:
+            assert all(choice(dtype, m, n, k) == (16, 16, 1) for m, n in test_gpu_q8_few_rows.SIZES if m <= 16)
             taken = {(m, n): choice(dtype, m, n, k) for m, n in test_gpu_q8_few_rows.SIZES if m > 16}
             assert all(t == (64, 16, 1) for t in taken.values()), (dtype, k, taken)
     # the row tiles are the launch's y: beyond 65535 of them another kernel takes the call
