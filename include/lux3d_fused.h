@@ -337,6 +337,9 @@ int lux3d_dequant_q8_0(const lux3d_tensor_t *blocks, const lux3d_tensor_t *y,
  * block's d: the f32 arithmetic up to the order of the sums (a non-finite d
  * makes the output non-finite as in the reference, though it can be +-inf
  * where the reference's per-weight 0 * inf gives NaN).
+ * The order of the f32 sums depends on the shape, the number of rows among
+ * it: a row's last bits may differ between calls of different row counts,
+ * and are the same in every call of one shape.
  * This is the dequantize-then-matmul path of candle's GPU backends; candle's
  * CPU path instead quantizes x to Q8_0 blocks and takes integer dot
  * products.                                                                 */
